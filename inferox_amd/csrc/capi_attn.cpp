@@ -2,14 +2,16 @@
 // operators of include/inferox.h (ifx_ops_attention_*, ifx_ops_qkv,
 // ifx_ops_gemv_residual): the same launchers the captured step enqueues, on
 // buffers the caller owns, so that each can be compared with the reference
-// loops it replaces.  Each call allocates its small device state (the
-// positions the kernels read, the chunk records or the split K/V), runs on the
-// given stream and returns when the work is complete.
+// loops it replaces.  Each call takes its device state (the positions the
+// kernels read, the chunk records or the split K/V) from a workspace that is
+// its own until it returns (host_workspace.h), runs on the given stream and
+// returns when the work is complete.
 #include <math.h>
 
 #include <algorithm>
 #include <vector>
 
+#include "host_workspace.h"
 #include "ifx_common.h"
 #include "kernels.h"
 
@@ -23,32 +25,43 @@ void rope_table_host(float base, uint64_t rope_dim, uint64_t n_pos, std::vector<
 
 namespace {
 
-// Device allocations of one call, freed after the stream has drained.
+// The device buffers of one call, each from its own workspace, given back
+// after the stream has drained.
 struct CallScratch {
+  static constexpr int kMost = 4;
   hipStream_t st = nullptr;
-  std::vector<void*> ptrs;
+  bool drained = false;
+  WorkspaceLease ws[kMost];
+  int n = 0;
   explicit CallScratch(hipStream_t s) : st(s) {}
   int alloc(void** p, size_t bytes) {
-    if (hipMalloc(p, std::max<size_t>(bytes, 16)) != hipSuccess)
+    if (n == kMost) return set_error(IFX_E_OOM, "workspaces of one call");
+    if (ws[n].take(std::max<size_t>(bytes, 16)) != hipSuccess)
       return set_error(IFX_E_OOM, "hipMalloc(%zu) failed", bytes);
-    ptrs.push_back(*p);
+    *p = ws[n++].ptr();
+    return IFX_OK;
+  }
+  // the end of a call whose launches all went out
+  int finish() {
+    IFX_HIP(hipStreamSynchronize(st));
+    drained = true;
     return IFX_OK;
   }
   ~CallScratch() {
-    if (!ptrs.empty()) (void)hipStreamSynchronize(st);
-    for (void* p : ptrs) (void)hipFree(p);
+    if (n && !drained) (void)hipStreamSynchronize(st);
   }
 };
 
 // The positions a step's kernels read: the token's cache row `len` (the
-// attention covers rows [0, len]) and its RoPE position.
+// attention covers rows [0, len]) and its RoPE position.  Written by a launch
+// on the call's stream (a blocking copy of these few bytes took ~15 us).
 int put_state(CallScratch& cs, uint32_t len, uint32_t rope_pos, DevState** out) {
   IFX_TRY(cs.alloc((void**)out, sizeof(DevState)));
   DevState d{};
   d.len = len;
   d.rope_pos = rope_pos;
   d.top_p = 1.0f;
-  IFX_HIP(hipMemcpy(*out, &d, sizeof d, hipMemcpyHostToDevice));
+  IFX_HIP(launch_put_state(*out, d, cs.st));
   return IFX_OK;
 }
 
@@ -119,8 +132,7 @@ int ifx_ops_attention_decode(const float* q, const void* k_cache, const void* v_
   a.out = out;
   IFX_TRY(alloc_records(cs, &a));
   IFX_HIP(launch_attn_decode(a, st));
-  IFX_HIP(hipStreamSynchronize(st));
-  return IFX_OK;
+  return cs.finish();
 }
 
 int ifx_ops_attention_decode_o(const float* q, const void* k_cache, const void* v_cache, int kv_type,
@@ -155,8 +167,7 @@ int ifx_ops_attention_decode_o(const float* q, const void* k_cache, const void* 
     IFX_HIP(launch_attn_decode(a, st));
     IFX_HIP(gemv_residual(go, h, st));
   }
-  IFX_HIP(hipStreamSynchronize(st));
-  return IFX_OK;
+  return cs.finish();
 }
 
 int ifx_ops_attention_prefill(const float* q, const void* k_cache, const void* v_cache, int kv_type,
@@ -181,8 +192,7 @@ int ifx_ops_attention_prefill(const float* q, const void* k_cache, const void* v
                            (uint32_t)n_kv_heads, (uint32_t)head_dim, (uint32_t)max_seq, causal != 0, ws,
                            kv_type == IFX_KV_F16};
   IFX_HIP(launch_attn_prefill(aa, st));
-  IFX_HIP(hipStreamSynchronize(st));
-  return IFX_OK;
+  return cs.finish();
 }
 
 int ifx_ops_gemv_residual(const ifx_tensor* w, const float* x, float* h, int mode, int* path_out, void* stream) {
@@ -255,8 +265,7 @@ int ifx_ops_qkv(const ifx_tensor* wq, const ifx_tensor* wk, const ifx_tensor* wv
     IFX_HIP(gemv_qkv(g, e, st));
   }
   if (path_out) *path_out = split ? 1 : 0;
-  IFX_HIP(hipStreamSynchronize(st));
-  return IFX_OK;
+  return cs.finish();
 }
 
 }  // extern "C"

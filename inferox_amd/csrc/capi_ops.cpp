@@ -3,10 +3,12 @@
 #include <string.h>
 
 #include <algorithm>
+#include <atomic>
 #include <mutex>
 #include <thread>
 #include <vector>
 
+#include "host_workspace.h"
 #include "ifx_common.h"
 #include "kernels.h"
 
@@ -18,6 +20,7 @@ static std::once_flag g_init_once;
 static int g_init_status = IFX_OK;
 static hipStream_t g_stream = nullptr;
 static hipEvent_t g_ev0 = nullptr, g_ev1 = nullptr;
+static std::atomic<long> g_tensors{0};  // uploaded matrices that live
 
 // The library targets gfx950 only: refuse any other device loudly.
 int device_init() {
@@ -168,6 +171,7 @@ int upload_matrix(uint32_t type, const uint8_t* src, uint64_t nbytes, uint64_t r
     delete t;
     return set_error(IFX_E_HIP, "upload failed: %s", hipGetErrorString(e));
   }
+  g_tensors++;
   *out = t;
   return IFX_OK;
 }
@@ -288,6 +292,7 @@ void ifx_tensor_free(ifx_tensor* t) {
   if (!t) return;
   if (t->alloc) (void)hipFree(t->alloc);
   delete t;
+  if (--g_tensors == 0) workspace_trim(g_stream);
 }
 
 int ifx_tensor_bytes(const ifx_tensor* t, uint64_t* dev, uint64_t* gguf) {
@@ -324,20 +329,31 @@ int ifx_matmul_qt(const float* a, uint64_t m, const ifx_tensor* w, float* c, voi
   if (m >= 2 && m <= 0xffffffffull && w->L.cols <= 0xffffffffull && gemm_type(w->L.type) && gemm_layout_ok(w->L)) {
     hipStream_t st = stream_of(stream);
     const uint64_t k = w->L.cols;
-    const uint64_t part_bytes = 64ull << 20;  // split-K partial tiles of short inputs
-    // one allocation: hi, lo planes, group sums, row exponents, partial tiles
+    const GemmW gw = gemm_w(w->L);
+    // one workspace: hi, lo planes, group sums, row exponents, split-K partial
+    // tiles of short inputs
+    const uint64_t part_limit = 64ull << 20;
     const uint64_t bh = (m * k * 2 + 255) & ~255ull, bg = (m * (k / 256 + 1) * 32 + 255) & ~255ull,
                    br = (m * 4 + 255) & ~255ull;
-    uint8_t* buf = nullptr;
-    IFX_HIP(hipMallocAsync((void**)&buf, 2 * bh + bg + br + part_bytes, st));
-    const GemmIn in{(const uint16_t*)buf, (const uint16_t*)(buf + bh), (const uint16_t*)(buf + 2 * bh),
-                    (const int*)(buf + 2 * bh + bg), (uint32_t)m, (uint32_t)k, (float*)(buf + 2 * bh + bg + br),
-                    part_bytes};
-    hipError_t e = launch_prep_rows(a, (uint32_t)m, (uint32_t)k, (uint32_t)k, nullptr, 0.f, in, st);
-    if (e == hipSuccess) {
-      const GemmW gw = gemm_w(w->L);
-      e = gemm_store(in, gw, c, (uint32_t)w->L.rows, st);
+    const uint64_t bytes = 2 * bh + bg + br + gemm_store_part_bytes((uint32_t)m, gw, part_limit);
+    auto enqueue = [&](uint8_t* buf) {
+      const GemmIn in{(const uint16_t*)buf, (const uint16_t*)(buf + bh), (const uint16_t*)(buf + 2 * bh),
+                      (const int*)(buf + 2 * bh + bg), (uint32_t)m, (uint32_t)k, (float*)(buf + 2 * bh + bg + br),
+                      part_limit};
+      const hipError_t e = launch_prep_rows(a, (uint32_t)m, (uint32_t)k, (uint32_t)k, nullptr, 0.f, in, st);
+      return e == hipSuccess ? gemm_store(in, gw, c, (uint32_t)w->L.rows, st) : e;
+    };
+    if (st == g_stream) {
+      StreamWorkspace ws(st);
+      IFX_HIP(ws.take(bytes));
+      IFX_HIP(enqueue((uint8_t*)ws.ptr()));
+      return IFX_OK;
     }
+    // a caller's stream (which may be under capture, or gone before the next
+    // call): allocated and freed in its order
+    uint8_t* buf = nullptr;
+    IFX_HIP(hipMallocAsync((void**)&buf, bytes, st));
+    const hipError_t e = enqueue(buf);
     const hipError_t ef = hipFreeAsync(buf, st);
     IFX_HIP(e);
     IFX_HIP(ef);

@@ -913,6 +913,16 @@ __global__ void __launch_bounds__(256) k_prep_rows_reg(const float* x, uint32_t 
 
 bool gemm_type(uint32_t t) { return t == T_Q4K || t == T_Q6K || t == T_Q8_0 || t == T_Q4_0; }
 
+uint64_t gemm_store_part_bytes(uint32_t m, const GemmW& w, uint64_t limit) {
+  GemmIn in{};
+  in.m = m;
+  in.part = (float*)1;  // a workspace of `limit` bytes; only its size is looked at
+  in.part_bytes = limit;
+  if (m == 0 || w.rows == 0) return 0;
+  const GemmArgs a = args_of(in, w, false);
+  return a.ksplit > 1 ? (uint64_t)a.ksplit * a.m * a.n * 4 : 0;
+}
+
 hipError_t gemm_store(const GemmIn& in, const GemmW& w, float* y, uint32_t ldy, hipStream_t st) {
   return dispatch(args_of(in, w, false), EpStore{y, ldy}, st);
 }

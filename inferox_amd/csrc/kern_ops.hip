@@ -231,6 +231,8 @@ __global__ void k_state(DevState* s, StateOp op) {
   }
 }
 
+__global__ void k_put_state(DevState* s, DevState value) { *s = value; }
+
 __global__ void k_fill_u32(uint32_t* p, uint32_t v, uint64_t n) {
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (uint64_t)gridDim.x * blockDim.x)
@@ -293,6 +295,11 @@ hipError_t launch_finalize(DevState* state, hipStream_t st) {
 
 hipError_t launch_state(DevState* state, const StateOp& op, hipStream_t st) {
   hipLaunchKernelGGL(k_state, dim3(1), dim3(1), 0, st, state, op);
+  return hipGetLastError();
+}
+
+hipError_t launch_put_state(DevState* state, const DevState& value, hipStream_t st) {
+  hipLaunchKernelGGL(k_put_state, dim3(1), dim3(1), 0, st, state, value);
   return hipGetLastError();
 }
 

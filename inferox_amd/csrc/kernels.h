@@ -179,6 +179,8 @@ struct GemmIn {
   uint64_t part_bytes = 0;
 };
 bool gemm_type(uint32_t type);
+// bytes of GemmIn::part that gemm_store of m rows uses when in.part_bytes is `limit`
+uint64_t gemm_store_part_bytes(uint32_t m, const GemmW& w, uint64_t limit);
 // y[t * ldy + n] = (A W^T)[t][n]
 hipError_t gemm_store(const GemmIn& in, const GemmW& w, float* y, uint32_t ldy, hipStream_t st);
 // x[t * ldx + n] += (A W^T)[t][n]
@@ -269,6 +271,8 @@ struct StateOp {
   unsigned long long seed = 0;
 };
 hipError_t launch_state(DevState* state, const StateOp& op, hipStream_t st);
+// *state = value, on the stream
+hipError_t launch_put_state(DevState* state, const DevState& value, hipStream_t st);
 hipError_t launch_fill_u32(uint32_t* p, uint32_t v, uint64_t n, hipStream_t st);
 
 // ---- attention (kern_attn.hip) ----
