@@ -8,43 +8,52 @@
 // matrices go to the int8-MFMA kernel of kern_gemv_mfma.hip.
 //
 // Work decomposition
-//   * Persistent workgroups of 8 wave64, two per CU (16 waves per CU, at most
-//     128 VGPRs each).  Each wave issues the loads of its first unit, then the
-//     workgroup stages x in LDS, optionally applying RMSNorm (ops::rms_norm,
-//     src/ops.rs:155-168) so the norm costs no launch, and precomputes
-//     16-element partial sums of x (the min/offset terms of the K-quants factor
-//     out as scale * sum(x)).
-//   * A wave owns tiles of R = 4 rows.  A "unit" is one 32-element group of
-//     each of the R rows per lane (lane l takes group l + 64 i), so each lane
-//     reads contiguous 16-byte pieces of the packed blocks and one x group read
-//     from LDS serves R rows.  The loads of the next unit are issued as soon as
-//     the current one is decoded; the other waves of the CU cover the latency.
-//     Tile and row bookkeeping is wave-uniform (scalar registers).
-//   * Row sums are reduced across the wave; the epilogue fuses RoPE + KV
-//     append (QKV), SwiGLU (gate/up), the residual add (O, down) or the logits
-//     store + greedy argmax (output head).
+//   * A row's 16-byte pieces lie one after another; lane l of the L lanes that
+//     share a row takes pieces l, l + L, ... (K of them), so every weight load
+//     of a wave covers contiguous memory.  The lane's x values (K pieces of
+//     them) stay in registers for all the rows the wave runs: no LDS, and no
+//     barrier between the kernel's start and its first dot product.  A launch
+//     on a small matrix is that start (the x loads, a few hundred cycles of
+//     arithmetic, the row reduction), not the stream: with x staged through
+//     LDS, 9 of 64 lanes at work on rows of 288 and 9 workgroups for 288 rows,
+//     a turn of the tiny model (24 steps) took 5534 us, now 4398.  A large
+//     matrix streams: 14336 x 4096 Q8_0 takes 12.2 us (5.1 TB/s; 16.6 before,
+//     with one unit of loads in flight).
+//   * Rows of at most 64 pieces (K = 1): L = 16, 32 or 64 lanes per row, so a
+//     wave runs 64 / L units at once.  Longer rows: a wave per unit up to
+//     4096 columns; past that S waves of a workgroup share each row (their
+//     sums meet in LDS, one barrier per unit).
+//   * A unit is two rows (2u, 2u + 1: a RoPE pair), or row u of gate and up.
+//     Each wave keeps the loads of two units in flight (one where a row takes
+//     32 registers or more) and refills a row's registers as soon as it is
+//     summed.
+//   * RMSNorm (ops::rms_norm, src/ops.rs:155-168) costs no launch: x * w is
+//     formed in registers, every group of lanes sums x . x over its own
+//     pieces (the whole row), and the scale, one scalar per vector, is applied
+//     to the row sums.
+//   * The epilogue fuses RoPE + KV append (QKV), SwiGLU (gate/up), the
+//     residual add (O, down) or the logits store + greedy argmax (head).
 // Compiled with -ffp-contract=off: only the explicit fmaf below are fused.
 #include <algorithm>
 
+#include "dev_lanes.h"
 #include "gemv_epi.h"
 
 namespace ifx {
 
 namespace {
 
-constexpr int kWaves = 8;
-constexpr int kBlocksPerCu = 2;  // 16 waves per CU
-constexpr int kWavesPerSimd = kBlocksPerCu * kWaves / 4;  // 4: at most 128 VGPRs per lane
-constexpr int kThreads = kWaves * 64;
-constexpr int kR = 4;
+constexpr int kWavesNarrow = 4;  // waves per workgroup, a wave per unit
+constexpr int kWavesWide = 8;    // S = 2, 4 or 8 of them per row
 
 struct KArgs {
   GemvSeg seg[3];
-  uint32_t ntiles[3];  // tiles per logical segment (paired: one logical segment)
-  uint32_t rot[3];     // first-wave rotation per segment (balances small segments)
-  uint32_t split;      // waves per row tile (1, 2, 4 or 8): they share its units
+  uint32_t nunits[3];  // per logical segment (paired: one logical segment)
+  uint32_t total;      // their sum
   int nseg;            // logical segments
-  uint32_t cols, groups;
+  uint32_t cols, pieces;
+  uint32_t lg_lanes;   // log2 of the lanes per row (6 unless K = 1)
+  uint32_t split;      // waves per row
   const float* x;
   const float* norm_w;
   float eps;
@@ -61,462 +70,398 @@ __device__ __forceinline__ uint32_t opaque(uint32_t v) {
 // byte b of v as a signed int8, to f32 (v_bfe_i32 + v_cvt_f32_i32)
 __device__ __forceinline__ float sbyte(int v, int b) { return (float)((v << (24 - 8 * b)) >> 24); }
 
-// x lives in LDS with each 32-element group padded to 36 floats, so lanes
-// reading consecutive groups (a 144-byte stride) spread over the banks.
-constexpr int kGroupStride = 36;
-__device__ __forceinline__ uint32_t xpad(uint32_t i) { return (i >> 5) * kGroupStride + (i & 31); }
-
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
-}
-
-template <class T>
-__device__ __forceinline__ T ldg(const void* p) { return *(const T*)p; }
-
-// Selects acc[r] for lane r (r < kR) with a chain of selects; the asm
-// barriers keep the compiler from folding it back into a dynamic index of a
-// register array (which it would place in scratch memory).
-__device__ __forceinline__ float lane_acc(const float* acc, int lane) {
-  float v = acc[0];
-#pragma unroll
-  for (int r = 1; r < kR; r++) {
-    v = lane == r ? acc[r] : v;
-    asm("" : "+v"(v));
-  }
-  return v;
-}
-
-// Row r of tile `tile` of logical segment s, wave-uniform.  Paired launches
-// (gate/up) put rows 2t, 2t+1 of segment 0 in r = 0, 1 and the same rows of
-// segment 1 in r = 2, 3.
-struct RowRef {
-  const uint8_t* body;
-  const uint8_t* scal;
-  uint64_t row;
-  bool ok;  // false for padding rows past the end of the segment
-};
-
-template <bool PAIRED>
-__device__ __forceinline__ RowRef row_of(const KArgs& a, int s, uint32_t tile, int r) {
-  // padding rows read the last real row (loads stay unconditional) and are
-  // skipped by the decode and the epilogue
-  if (PAIRED) {
-    const GemvSeg& sg = a.seg[r < kR / 2 ? 0 : 1];
-    const uint32_t row = tile * (kR / 2) + (r % (kR / 2));
-    return RowRef{sg.body, sg.scal, row < sg.rows ? row : sg.rows - 1, row < sg.rows};
-  }
-  const GemvSeg& sg = a.seg[s];
-  const uint32_t row = tile * kR + r;
-  return RowRef{sg.body, sg.scal, row < sg.rows ? row : sg.rows - 1, row < sg.rows};
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ uint4 ldw(const uint8_t* p) {
+  return *(const uint4*)p;
 }
 
 // ---------------------------------------------------------------------------
-// Per-type fragments: the raw bytes of one unit (group g of the kR rows of a
-// tile) held in registers, and the decode + dot of that group with x.
-//   load_row(a, s, tile, g, r): issue the loads of row r, group g (always a
-//     real group of a real row: padding rows and lanes are clamped).
-//   dot_row(a, s, tile, g, valid, xv, xsa, xsb, acc, r): acc[r] += row r . x
-//     over group g; xv holds the group's 32 x values, xsa/xsb its two
-//     16-element sums.  Lanes with !valid and padding rows add nothing.
-// The main loop is free of branches so that the compiler can wait for exactly
-// the loads a row needs (a join in the control flow makes it wait for all).
+// Per-type pieces: 16 bytes of a row's quants (and the scale they need) in
+// registers, and their dot product with the piece's kE x values.  P: pieces
+// per row.  sx: the sum of those x values.
 // ---------------------------------------------------------------------------
 
 // Q8_0 (device layout qs[32] | d): y = f32(i8 q) * delta (src/gguf/dequant.rs:101-109).
-struct FragQ80 {
-  uint4 qa[kR], qb[kR];
-  uint32_t d[kR];
-  template <bool P>
-  __device__ void load_row(const KArgs& a, int s, uint32_t tile, uint32_t g, int r) {
-    const RowRef rr = row_of<P>(a, s, tile, r);
-    const uint8_t* row = rr.body + rr.row * (a.groups * 32);
-    qa[r] = ldg<uint4>(row + g * 32);
-    qb[r] = ldg<uint4>(row + g * 32 + 16);
-    d[r] = ldg<uint16_t>(rr.scal + rr.row * (a.groups * 2) + g * 2);
+struct PieceQ80 {
+  static constexpr int kE = 16;
+  uint4 q;
+  uint32_t d;
+  __device__ __forceinline__ void load(const uint8_t* body, const uint8_t* scal, uint32_t row, uint32_t P, uint32_t p) {
+    const uint64_t i = (uint64_t)row * P + p;
+    q = ldw(body + i * 16);
+    d = ((const uint16_t*)scal)[i >> 1];
   }
   // q x = (u - 128) x with u = q ^ 0x80 unsigned: one convert per byte, the
-  // -128 sum(x) term from the staged group sums
-  template <bool P>
-  __device__ void dot_row(const KArgs& a, int s, uint32_t tile, uint32_t, bool valid, const float4* xv, float xsa,
-                          float xsb, float* acc, int r) const {
-    const uint32_t qw[8] = {qa[r].x, qa[r].y, qa[r].z, qa[r].w, qb[r].x, qb[r].y, qb[r].z, qb[r].w};
+  // -128 sum(x) term from sx
+  __device__ __forceinline__ float dot(const float* x, float sx) const {
+    const uint32_t qw[4] = {q.x, q.y, q.z, q.w};
     float s0 = 0.f, s1 = 0.f;
 #pragma unroll
-    for (int w = 0; w < 8; w++) {
-      const float4 xa = xv[w];
+    for (int w = 0; w < 4; w++) {
       const uint32_t u = opaque(qw[w] ^ 0x80808080u);
-      s0 = fmaf(cvtb(u, 0), xa.x, s0);
-      s1 = fmaf(cvtb(u, 1), xa.y, s1);
-      s0 = fmaf(cvtb(u, 2), xa.z, s0);
-      s1 = fmaf(cvtb(u, 3), xa.w, s1);
+      s0 = fmaf(cvtb(u, 0), x[4 * w], s0);
+      s1 = fmaf(cvtb(u, 1), x[4 * w + 1], s1);
+      s0 = fmaf(cvtb(u, 2), x[4 * w + 2], s0);
+      s1 = fmaf(cvtb(u, 3), x[4 * w + 3], s1);
     }
-    const float v = h2f(d[r]) * fmaf(-128.f, xsa + xsb, s0 + s1);
-    acc[r] += (valid && row_of<P>(a, s, tile, r).ok) ? v : 0.f;
+    return h2f(d) * fmaf(-128.f, sx, s0 + s1);
   }
 };
 
 // Q4_0 (device layout qs[16] | d): low nibble -> element j, high -> j+16, value q-8.
-struct FragQ40 {
-  uint4 q[kR];
-  uint32_t d[kR];
-  template <bool P>
-  __device__ void load_row(const KArgs& a, int s, uint32_t tile, uint32_t g, int r) {
-    const RowRef rr = row_of<P>(a, s, tile, r);
-    q[r] = ldg<uint4>(rr.body + rr.row * (a.groups * 16) + g * 16);
-    d[r] = ldg<uint16_t>(rr.scal + rr.row * (a.groups * 2) + g * 2);
+struct PieceQ40 {
+  static constexpr int kE = 32;
+  uint4 q;
+  uint32_t d;
+  __device__ __forceinline__ void load(const uint8_t* body, const uint8_t* scal, uint32_t row, uint32_t P, uint32_t p) {
+    const uint64_t i = (uint64_t)row * P + p;
+    q = ldw(body + i * 16);
+    d = ((const uint16_t*)scal)[i];
   }
-  template <bool P>
-  __device__ void dot_row(const KArgs& a, int s, uint32_t tile, uint32_t, bool valid, const float4* xv, float xsa,
-                          float xsb, float* acc, int r) const {
-    const uint32_t qw[4] = {q[r].x, q[r].y, q[r].z, q[r].w};
+  __device__ __forceinline__ float dot(const float* x, float sx) const {
+    const uint32_t qw[4] = {q.x, q.y, q.z, q.w};
     float s0 = 0.f, s1 = 0.f;
 #pragma unroll
     for (int w = 0; w < 4; w++) {
       const uint32_t lo = opaque(qw[w] & 0x0F0F0F0Fu), hi = opaque(qw[w] & 0xF0F0F0F0u);  // hi: 16 q
-      const float4 xa = xv[w], xb = xv[4 + w];
-      s0 = fmaf(cvtb(lo, 0), xa.x, s0);
-      s0 = fmaf(cvtb(lo, 1), xa.y, s0);
-      s0 = fmaf(cvtb(lo, 2), xa.z, s0);
-      s0 = fmaf(cvtb(lo, 3), xa.w, s0);
-      s1 = fmaf(cvtb(hi, 0), xb.x, s1);
-      s1 = fmaf(cvtb(hi, 1), xb.y, s1);
-      s1 = fmaf(cvtb(hi, 2), xb.z, s1);
-      s1 = fmaf(cvtb(hi, 3), xb.w, s1);
+#pragma unroll
+      for (int b = 0; b < 4; b++) {
+        s0 = fmaf(cvtb(lo, b), x[4 * w + b], s0);
+        s1 = fmaf(cvtb(hi, b), x[16 + 4 * w + b], s1);
+      }
     }
-    const float v = h2f(d[r]) * fmaf(-8.f, xsa + xsb, fmaf(s1, 0.0625f, s0));
-    acc[r] += (valid && row_of<P>(a, s, tile, r).ok) ? v : 0.f;
+    return h2f(d) * fmaf(-8.f, sx, fmaf(s1, 0.0625f, s0));
   }
 };
 
 // Q8_K (device layout sc[32] | qs[256]; {d, dmin}): y = ((d*sc)*q) - dmin.
-struct FragQ8K {
-  uint4 qa[kR], qb[kR];
-  uint32_t sc[kR], dd[kR];
-  template <bool P>
-  __device__ void load_row(const KArgs& a, int s, uint32_t tile, uint32_t g, int r) {
-    const RowRef rr = row_of<P>(a, s, tile, r);
-    const uint32_t nb = a.groups / 8, sub = g & 7;
-    const uint8_t* blk = rr.body + rr.row * (nb * 288) + (g / 8) * 288;
-    sc[r] = ldg<uint32_t>(blk + 4 * sub);
-    qa[r] = ldg<uint4>(blk + 32 + 32 * sub);
-    qb[r] = ldg<uint4>(blk + 48 + 32 * sub);
-    dd[r] = ldg<uint32_t>(rr.scal + rr.row * (nb * 4) + (g / 8) * 4);
+struct PieceQ8K {
+  static constexpr int kE = 16;
+  uint4 q;
+  uint32_t sc, dd;
+  __device__ __forceinline__ void load(const uint8_t* body, const uint8_t* scal, uint32_t row, uint32_t P, uint32_t p) {
+    const uint64_t b = (uint64_t)row * (P >> 4) + (p >> 4);
+    const uint8_t* blk = body + b * 288;
+    q = ldw(blk + 32 + 16 * (p & 15));
+    sc = *(const uint16_t*)(blk + 2 * (p & 15));
+    dd = ((const uint32_t*)scal)[b];
   }
-  template <bool P>
-  __device__ void dot_row(const KArgs& a, int s, uint32_t tile, uint32_t, bool valid, const float4* xv, float xsa,
-                          float xsb, float* acc, int r) const {
-    const uint32_t qw[8] = {qa[r].x, qa[r].y, qa[r].z, qa[r].w, qb[r].x, qb[r].y, qb[r].z, qb[r].w};
-    const float d = h2f(dd[r]), dmin = h2f(dd[r] >> 16);
+  __device__ __forceinline__ float dot(const float* x, float sx) const {
+    const uint32_t qw[4] = {q.x, q.y, q.z, q.w};
+    const float d = h2f(dd), dmin = h2f(dd >> 16);
     float tot = 0.f;
 #pragma unroll
-    for (int k = 0; k < 4; k++) {  // sub-blocks of 8 elements share one scale byte
-      float acc8 = 0.f;
+    for (int k = 0; k < 2; k++) {  // sub-blocks of 8 elements share one scale byte
+      float a8 = 0.f;
 #pragma unroll
-      for (int w = 0; w < 2; w++) {
-        const int v = (int)qw[2 * k + w];
-        const float4 x4 = xv[2 * k + w];
-        acc8 = fmaf(sbyte(v, 0), x4.x, acc8);
-        acc8 = fmaf(sbyte(v, 1), x4.y, acc8);
-        acc8 = fmaf(sbyte(v, 2), x4.z, acc8);
-        acc8 = fmaf(sbyte(v, 3), x4.w, acc8);
-      }
-      tot = fmaf(d * cvtb(sc[r], k), acc8, tot);
+      for (int e = 0; e < 8; e++) a8 = fmaf(sbyte((int)qw[2 * k + e / 4], e % 4), x[8 * k + e], a8);
+      tot = fmaf(d * cvtb(sc, k), a8, tot);
     }
-    const float v = fmaf(-dmin, xsa + xsb, tot);
-    acc[r] += (valid && row_of<P>(a, s, tile, r).ok) ? v : 0.f;
+    return fmaf(-dmin, sx, tot);
   }
 };
 
-// F32 / F16 rows of whole groups: read at use, no prefetch (toy models, tests).
-struct FragF32 {
-  template <bool P>
-  __device__ void load_row(const KArgs&, int, uint32_t, uint32_t, int) {}
-  template <bool P>
-  __device__ void dot_row(const KArgs& a, int s, uint32_t tile, uint32_t g, bool valid, const float4* xv, float,
-                          float, float* acc, int r) const {
-    const RowRef rr = row_of<P>(a, s, tile, r);
-    const float4* w4 = (const float4*)rr.body + (rr.row * (uint64_t)a.groups + g) * 8;
+struct PieceF32 {
+  static constexpr int kE = 4;
+  uint4 q;
+  __device__ __forceinline__ void load(const uint8_t* body, const uint8_t*, uint32_t row, uint32_t P, uint32_t p) {
+    q = ldw(body + ((uint64_t)row * P + p) * 16);
+  }
+  __device__ __forceinline__ float dot(const float* x, float) const {
+    float s = __uint_as_float(q.x) * x[0];
+    s = fmaf(__uint_as_float(q.y), x[1], s);
+    s = fmaf(__uint_as_float(q.z), x[2], s);
+    return fmaf(__uint_as_float(q.w), x[3], s);
+  }
+};
+
+struct PieceF16 {
+  static constexpr int kE = 8;
+  uint4 q;
+  __device__ __forceinline__ void load(const uint8_t* body, const uint8_t*, uint32_t row, uint32_t P, uint32_t p) {
+    q = ldw(body + ((uint64_t)row * P + p) * 16);
+  }
+  __device__ __forceinline__ float dot(const float* x, float) const {
+    const uint32_t qw[4] = {q.x, q.y, q.z, q.w};
     float s0 = 0.f, s1 = 0.f;
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
-      const float4 w = w4[i], x = xv[i];
-      s0 = fmaf(w.x, x.x, s0);
-      s1 = fmaf(w.y, x.y, s1);
-      s0 = fmaf(w.z, x.z, s0);
-      s1 = fmaf(w.w, x.w, s1);
+    for (int w = 0; w < 4; w++) {
+      s0 = fmaf(h2f(qw[w]), x[2 * w], s0);
+      s1 = fmaf(h2f(qw[w] >> 16), x[2 * w + 1], s1);
     }
-    acc[r] += (valid && rr.ok) ? s0 + s1 : 0.f;
+    return s0 + s1;
   }
 };
 
-struct FragF16 {
-  template <bool P>
-  __device__ void load_row(const KArgs&, int, uint32_t, uint32_t, int) {}
-  template <bool P>
-  __device__ void dot_row(const KArgs& a, int s, uint32_t tile, uint32_t g, bool valid, const float4* xv, float,
-                          float, float* acc, int r) const {
-    const RowRef rr = row_of<P>(a, s, tile, r);
-    const uint4* w4 = (const uint4*)rr.body + (rr.row * (uint64_t)a.groups + g) * 4;
-    float s0 = 0.f, s1 = 0.f;
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const uint4 w = w4[i];
-      const uint32_t ww[4] = {w.x, w.y, w.z, w.w};
-#pragma unroll
-      for (int k = 0; k < 2; k++) {
-        const float4 x = xv[2 * i + k];
-        s0 = fmaf(h2f(ww[2 * k]), x.x, s0);
-        s1 = fmaf(h2f(ww[2 * k] >> 16), x.y, s1);
-        s0 = fmaf(h2f(ww[2 * k + 1]), x.z, s0);
-        s1 = fmaf(h2f(ww[2 * k + 1] >> 16), x.w, s1);
-      }
-    }
-    acc[r] += (valid && rr.ok) ? s0 + s1 : 0.f;
-  }
-};
-
-// Hands the reduced sums of a finished tile to the row epilogue (gemv_epi.h):
-// lane r < kR owns row r (paired: lanes 0, 1 own the gate rows, whose up rows
-// sit at r + 2).
+// Where the rows of the logical segments lie.  Held in registers behind an
+// asm barrier: a segment chosen per unit from the kernel's arguments would be
+// indexed through scratch memory.
 template <class Epi>
-__device__ __forceinline__ void emit(const Epi& epi, typename Epi::Wave& ws, const KArgs& a, int s, uint32_t tile,
-                                     const float* acc, int lane) {
-  constexpr bool P = Epi::kPaired;
-  if (lane < (P ? kR / 2 : kR)) {
-    const RowRef rr = row_of<P>(a, s, tile, lane);
-    if (rr.ok) {
-      const float v = lane_acc(acc, lane);
-      const float partner = P ? lane_acc(acc, lane + kR / 2) : (Epi::kNeighbor ? lane_acc(acc, lane ^ 1) : 0.f);
-      const int es = P ? 0 : s;
-      epi.row(ws, es, (uint32_t)rr.row, v, partner, epi.pre(ws, es, (uint32_t)rr.row));
+struct Segs {
+  static constexpr int kN = Epi::kPaired ? 2 : Epi::kNeighbor ? 3 : 1;  // gate/up; q/k/v; one matrix
+  const uint8_t* body[kN];
+  const uint8_t* scal[kN];
+  uint32_t rows[kN];
+  __device__ __forceinline__ explicit Segs(const KArgs& a) {
+#pragma unroll
+    for (int i = 0; i < kN; i++) {
+      body[i] = a.seg[i].body;
+      scal[i] = a.seg[i].scal;
+      rows[i] = a.seg[i].rows;
+      asm("" : "+s"(body[i]), "+s"(scal[i]), "+s"(rows[i]));
     }
   }
-}
+};
 
-// The row tiles of one logical segment owned by this wave's tile group
-// (a.split waves of one workgroup): tiles first, first+TG, ..., `iters` of them
-// (the same count for every wave of the workgroup, so that the LDS reduction
-// of a split tile can use workgroup barriers).  Wave j of the group takes the
-// units j, j+split, ... of each tile.  `f` arrives holding the loads of the
-// first unit.  As soon as row r of the current unit is decoded, the loads of
-// row r of the next unit are issued into the same registers, so the wave keeps
-// loads in flight while it computes (a second register buffer would cost
-// occupancy).  Past the wave's last unit the loads repeat a real unit.
-template <class Frag, class Epi>
-__device__ __forceinline__ void run_segment(const KArgs& a, const Epi& epi, typename Epi::Wave& ws, int s,
-                                            uint32_t first, uint32_t TG, uint32_t iters, uint32_t j, Frag& f,
-                                            const float* xl, const float* xs, float* part, int lane, int wave) {
-  constexpr bool P = Epi::kPaired;
-  const uint32_t NG = (a.groups + 63) / 64, S = a.split;
-  for (uint32_t k = 0; k < iters; k++) {
-    const uint32_t tile = first + k * TG;
-    const bool live = tile < a.ntiles[s];  // uniform over the wave
-    float acc[kR];
-#pragma unroll
-    for (int r = 0; r < kR; r++) acc[r] = 0.f;
-    if (live) {
-      for (uint32_t it = j; it < NG; it += S) {
-        const uint32_t g = lane + 64 * it, gc = min(g, a.groups - 1);
-        uint32_t nt = tile, ni = it + S;
-        if (ni >= NG) {
-          ni = j;
-          nt += TG;
-        }
-        if (nt >= a.ntiles[s]) nt = tile;  // uniform select: no branch around the loads
-        const uint32_t ng = min(lane + 64 * ni, a.groups - 1);
-        const float4* xv4 = (const float4*)(xl + kGroupStride * gc);
-        float4 xv[8];
-#pragma unroll
-        for (int i = 0; i < 8; i++) xv[i] = xv4[i];
-        const float xsa = xs[2 * gc], xsb = xs[2 * gc + 1];
-#pragma unroll
-        for (int r = 0; r < kR; r++) {
-          f.template dot_row<P>(a, s, tile, gc, g < a.groups, xv, xsa, xsb, acc, r);
-          f.template load_row<P>(a, s, nt, ng, r);
-        }
-      }
-    }
-#pragma unroll
-    for (int r = 0; r < kR; r++) acc[r] = wave_sum(acc[r]);
-    if (S > 1) {
-      // partial sums of the group's waves through LDS (double-buffered: one barrier per tile)
-      float* pb = part + (k & 1) * kWaves * kR;
-      if (lane < kR) pb[wave * kR + lane] = lane_acc(acc, lane);
-      __syncthreads();
-      if (j == 0 && live) {
-#pragma unroll
-        for (int r = 0; r < kR; r++) {
-          float v = 0.f;
-          for (uint32_t i = 0; i < S; i++) v += pb[(wave + i) * kR + r];
-          acc[r] = v;
-        }
-        emit(epi, ws, a, s, tile, acc, lane);
-      }
-    } else if (live) {
-      emit(epi, ws, a, s, tile, acc, lane);
-    }
-  }
-}
-
-// rms_norm (src/ops.rs:162-167): scale = 1/sqrt(mean(x^2) + eps); x = (x*scale)*w.
-// Reduces the per-thread sums of squares over the workgroup.
-__device__ __forceinline__ float norm_scale(const KArgs& a, float ss, float* red, int lane, int wave) {
-  ss = wave_sum(ss);
-  if (lane == 0) red[wave] = ss;
-  __syncthreads();
-  float tot = 0.f;
-#pragma unroll
-  for (int w = 0; w < kWaves; w++) tot += red[w];
-  return 1.0f / sqrtf(tot / (float)a.cols + a.eps);
-}
-
-// Workgroup prologue (cols % 32 == 0): x, optionally RMS-normalised, into LDS
-// and the 16-element sums of x.  Every thread issues all its float4 loads of
-// x (and of the norm weights, staged in wl) before the first wait, so the
-// prologue costs one memory round trip.
-constexpr int kStage = 8;  // float4 loads per thread per batch
-template <bool NORM>
-__device__ __forceinline__ float stage_load(const KArgs& a, float* xl, float* wl, int tid) {
-  const uint32_t n4 = a.cols / 4;
-  const float4* x4 = (const float4*)a.x;
-  const float4* w4 = (const float4*)a.norm_w;
-  float ss = 0.f;
-  for (uint32_t b = tid; b < n4; b += kThreads * kStage) {
-    float4 v[kStage], w[kStage];
-#pragma unroll
-    for (int k = 0; k < kStage; k++) {
-      const uint32_t i = min(b + k * kThreads, n4 - 1);  // clamped: loads stay unconditional
-      v[k] = x4[i];
-      if (NORM) w[k] = w4[i];
-    }
-#pragma unroll
-    for (int k = 0; k < kStage; k++) {
-      const uint32_t i = b + k * kThreads;
-      if (i < n4) {
-        *(float4*)(xl + xpad(4 * i)) = v[k];  // 4 | 32: a float4 never straddles a group
-        if (NORM) {
-          *(float4*)(wl + 4 * i) = w[k];
-          ss = fmaf(v[k].x, v[k].x, ss);
-          ss = fmaf(v[k].y, v[k].y, ss);
-          ss = fmaf(v[k].z, v[k].z, ss);
-          ss = fmaf(v[k].w, v[k].w, ss);
-        }
-      }
-    }
-  }
-  return ss;
-}
-
-__device__ __forceinline__ void stage_x(const KArgs& a, float* xl, float* xs, float* wl, float* red, int tid,
-                                        int lane, int wave) {
-  const uint32_t n4 = a.cols / 4;
-  if (a.norm_w) {
-    const float ss = stage_load<true>(a, xl, wl, tid);
-    const float scale = norm_scale(a, ss, red, lane, wave);
-    for (uint32_t i = tid; i < n4; i += kThreads) {
-      float4 v = *(float4*)(xl + xpad(4 * i));
-      const float4 w = *(const float4*)(wl + 4 * i);
-      v.x = (v.x * scale) * w.x;
-      v.y = (v.y * scale) * w.y;
-      v.z = (v.z * scale) * w.z;
-      v.w = (v.w * scale) * w.w;
-      *(float4*)(xl + xpad(4 * i)) = v;
-    }
+// Unit u of the launch: the rows of its two sums.  Units past the end read
+// unit 0 (in bounds, unused); the row past an odd segment's end reads the last.
+struct Unit {
+  int s;
+  uint32_t r0, r1;
+  bool ok1;
+};
+template <class Epi>
+__device__ __forceinline__ Unit unit_of(const KArgs& a, const Segs<Epi>& g, uint32_t u) {
+  Unit n;
+  u = u < a.total ? u : 0u;
+  n.s = 0;
+  if constexpr (Epi::kPaired) {
+    n.r0 = n.r1 = u;
+    n.ok1 = true;
   } else {
-    stage_load<false>(a, xl, wl, tid);
+    uint32_t rows = g.rows[0];
+    if constexpr (Segs<Epi>::kN == 3) {
+      const uint32_t n1 = a.nunits[0], n2 = n1 + a.nunits[1];
+      n.s = u >= n2 ? 2 : u >= n1 ? 1 : 0;
+      rows = n.s == 2 ? g.rows[2] : n.s == 1 ? g.rows[1] : rows;
+      u -= n.s == 2 ? n2 : n.s == 1 ? n1 : 0u;
+    }
+    n.r0 = 2 * u;
+    n.ok1 = n.r0 + 1 < rows;
+    n.r1 = n.ok1 ? n.r0 + 1 : n.r0;
   }
-  __syncthreads();
-  for (uint32_t j = tid; j < a.cols / 16; j += kThreads) {
-    const float4* p = (const float4*)(xl + (j >> 1) * kGroupStride + 16 * (j & 1));
-    const float4 u0 = p[0], u1 = p[1], u2 = p[2], u3 = p[3];
-    xs[j] = ((u0.x + u0.y) + (u0.z + u0.w)) + ((u1.x + u1.y) + (u1.z + u1.w)) +
-            (((u2.x + u2.y) + (u2.z + u2.w)) + ((u3.x + u3.y) + (u3.z + u3.w)));
-  }
-  __syncthreads();
+  return n;
 }
 
-// Prologue of the generic kernel (any cols): x, optionally RMS-normalised, into LDS.
-__device__ __forceinline__ void stage_x_generic(const KArgs& a, float* xl, float* red, int tid, int lane,
-                                                int wave) {
+template <class Epi, class Q, int K>
+struct Buf {
+  Q q[2][K];
+  // row t of unit u
+  template <int t>
+  __device__ __forceinline__ void load(const KArgs& a, const Segs<Epi>& g, uint32_t u, const uint32_t (&pc)[K]) {
+    const Unit n = unit_of<Epi>(a, g, u);
+    const uint8_t *b = g.body[0], *sc = g.scal[0];
+    if constexpr (Epi::kPaired) {
+      b = g.body[t];
+      sc = g.scal[t];
+    } else if constexpr (Segs<Epi>::kN == 3) {
+      b = n.s == 2 ? g.body[2] : n.s == 1 ? g.body[1] : b;
+      sc = n.s == 2 ? g.scal[2] : n.s == 1 ? g.scal[1] : sc;
+    }
+#pragma unroll
+    for (int i = 0; i < K; i++) q[t][i].load(b, sc, t ? n.r1 : n.r0, a.pieces, pc[i]);
+    __builtin_amdgcn_sched_barrier(0);  // rows in order: the loop's waits assume it
+  }
+  __device__ __forceinline__ float dot(int t, const float (&x)[K][Q::kE], const float (&sx)[K], const bool (&valid)[K]) const {
+    float v = 0.f;
+#pragma unroll
+    for (int i = 0; i < K; i++) {
+      const float p = q[t][i].dot(x[i], sx[i]);
+      v += valid[i] ? p : 0.f;
+    }
+    return v;
+  }
+};
+
+// the sum of v over the lanes that share a row, in each of them
+template <int K>
+__device__ __forceinline__ float lanes_sum(float v, uint32_t lg) {
+  v = bfly<1, false>(v);
+  v = bfly<2, false>(v);
+  v = bfly<4, false>(v);
+  v = bfly<8, false>(v);
+  if (K > 1 || lg > 4) v = bfly<16, false>(v);
+  if (K > 1 || lg > 5) v = bfly<32, false>(v);
+  return v;
+}
+
+constexpr int kMinWaves = 2;  // per SIMD
+
+// K pieces of a row per lane; WIDE: a.split waves of the workgroup per row.
+template <class Epi, class Q, int K, bool WIDE>
+__global__ void __launch_bounds__(64 * (WIDE ? kWavesWide : kWavesNarrow), kMinWaves) k_gemv(KArgs a, Epi epi) {
+  constexpr int kW = WIDE ? kWavesWide : kWavesNarrow, kE = Q::kE;
+  constexpr bool P2 = Epi::kPaired;
+  // units in flight; 0: a row's loads go out when its turn comes (F32: 64
+  // registers a row; the other waves of the CU cover them)
+  constexpr int kDepth = sizeof(Q) * K > 128 ? 0 : sizeof(Q) * K > 100 ? 1 : 2;
+  constexpr int kSlots = kDepth ? kDepth : 1;
+  __shared__ float part[2][kW][2];
+  __shared__ float red[kW];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const uint32_t lg = K > 1 ? 6u : a.lg_lanes, ll = (uint32_t)lane & ((1u << lg) - 1u), G = 64u >> lg;
+  const uint32_t S = WIDE ? a.split : 1u, j = WIDE ? (uint32_t)wave % S : 0u;
+  // groups of G units: this wave takes g0, g0 + TW, ...; `iters` covers the
+  // workgroup's first wave, which has the most
+  const uint32_t NG = (a.total + G - 1) >> (6 - lg);
+  const uint32_t GPB = kW / S, TW = gridDim.x * GPB, gb = blockIdx.x * GPB, g0 = gb + (uint32_t)wave / S;
+  const uint32_t iters = gb < NG ? (NG - 1 - gb) / TW + 1 : 0u;
+  const uint32_t u0 = (g0 << (6 - lg)) + (K > 1 ? 0u : (uint32_t)lane >> lg), ustep = TW << (6 - lg);
+
+  const Segs<Epi> sg(a);
+  typename Epi::Wave ws;
+  epi.begin(ws);
+  uint32_t pc[K];
+  bool valid[K];
+#pragma unroll
+  for (int i = 0; i < K; i++) {
+    const uint32_t p = K > 1 || WIDE ? (uint32_t)lane + 64u * (j + S * i) : ll;
+    valid[i] = p < a.pieces;
+    pc[i] = min(p, a.pieces - 1);
+  }
+  float x[K][kE], sx[K];
+#pragma unroll
+  for (int i = 0; i < K; i++)
+#pragma unroll
+    for (int e = 0; e < kE; e += 4) {
+      const float4 v = *(const float4*)(a.x + (uint64_t)pc[i] * kE + e);
+      x[i][e] = v.x; x[i][e + 1] = v.y; x[i][e + 2] = v.z; x[i][e + 3] = v.w;
+    }
+  float nscale = 1.f, ss = 0.f;
+  if (a.norm_w) {
+#pragma unroll
+    for (int i = 0; i < K; i++)
+#pragma unroll
+      for (int e = 0; e < kE; e += 4) {
+        const float4 v = *(const float4*)(a.norm_w + (uint64_t)pc[i] * kE + e);
+        const float w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+          const float t = x[i][e + c];
+          ss = valid[i] ? fmaf(t, t, ss) : ss;
+          x[i][e + c] = t * w[c];
+        }
+      }
+  }
+  Buf<Epi, Q, K> buf[kSlots];
+#pragma unroll
+  for (int d = 0; d < kDepth; d++) {
+    buf[d].template load<0>(a, sg, u0 + d * ustep, pc);
+    buf[d].template load<1>(a, sg, u0 + d * ustep, pc);
+  }
+  if (a.norm_w) {  // rms_norm (src/ops.rs:162-167): scale = 1/sqrt(mean(x^2) + eps)
+    ss = lanes_sum<K>(ss, lg);
+    if (WIDE) {
+      if (lane == 0) red[wave] = ss;
+      __syncthreads();
+      ss = 0.f;
+      for (uint32_t q = 0; q < S; q++) ss += red[(wave - j) + q];
+    }
+    nscale = 1.0f / sqrtf(ss / (float)a.cols + a.eps);
+  }
+#pragma unroll
+  for (int i = 0; i < K; i++) {
+    sx[i] = 0.f;
+#pragma unroll
+    for (int e = 0; e < kE; e += 4) sx[i] += (x[i][e] + x[i][e + 1]) + (x[i][e + 2] + x[i][e + 3]);
+  }
+
+  for (uint32_t it0 = 0; it0 < iters; it0 += kSlots) {
+#pragma unroll
+    for (int d = 0; d < kSlots; d++) {
+      const uint32_t it = it0 + d, u = u0 + it * ustep;
+      // lane ll < 2 (paired: 0) of the first wave emits row ll of its unit
+      const bool live = it < iters && u < a.total && (!WIDE || j == 0) && ll < (P2 ? 1u : 2u);
+      const Unit n = unit_of<Epi>(a, sg, u);
+      const bool mine = live && (ll == 0 || n.ok1);
+      const uint32_t r = ll == 0 ? n.r0 : n.r1;
+      typename Epi::Pre pre{};
+      if (mine) pre = epi.pre(ws, Segs<Epi>::kN == 3 ? n.s : 0, r);
+      if constexpr (kDepth == 0) buf[d].template load<0>(a, sg, u, pc);
+      float v0 = buf[d].dot(0, x, sx, valid);
+      if constexpr (kDepth > 0) buf[d].template load<0>(a, sg, u + kDepth * ustep, pc);
+      else buf[d].template load<1>(a, sg, u, pc);
+      float v1 = buf[d].dot(1, x, sx, valid);
+      if constexpr (kDepth > 0) buf[d].template load<1>(a, sg, u + kDepth * ustep, pc);
+      v0 = lanes_sum<K>(v0, lg);
+      v1 = lanes_sum<K>(v1, lg);
+      if (WIDE) {
+        if (lane == 0) {
+          part[it & 1][wave][0] = v0;
+          part[it & 1][wave][1] = v1;
+        }
+        __syncthreads();
+        v0 = v1 = 0.f;
+        for (uint32_t q = 0; q < S; q++) {
+          v0 += part[it & 1][(wave - j) + q][0];
+          v1 += part[it & 1][(wave - j) + q][1];
+        }
+      }
+      v0 *= nscale;
+      v1 *= nscale;
+      if (mine) epi.row(ws, Segs<Epi>::kN == 3 ? n.s : 0, r, ll == 0 ? v0 : v1, ll == 0 ? v1 : v0, pre);
+    }
+  }
+  epi.finish(ws, lane);
+}
+
+// ---------------------------------------------------------------------------
+// F32 / F16 rows that are not whole 32-element groups: x in LDS (optionally
+// RMS-normalised), lanes stride over the elements of each row, a wave per tile
+// of kR rows.
+// ---------------------------------------------------------------------------
+constexpr int kGWaves = 8, kGThreads = kGWaves * 64, kR = 4;
+constexpr int kGroupStride = 36;
+__device__ __forceinline__ uint32_t xpad(uint32_t i) { return (i >> 5) * kGroupStride + (i & 31); }
+
+struct GArgs {
+  GemvSeg seg[3];
+  uint32_t ntiles[3];
+  uint32_t rot[3];  // first-wave rotation per segment (balances small segments)
+  int nseg;
+  uint32_t cols;
+  const float* x;
+  const float* norm_w;
+  float eps;
+};
+
+// Row r of tile `tile` of logical segment s.  Paired launches (gate/up) put
+// rows 2t, 2t + 1 of segment 0 in r = 0, 1 and those of segment 1 in r = 2, 3.
+struct RowRef {
+  const uint8_t* body;
+  uint64_t row;
+  bool ok, f32;
+};
+template <bool PAIRED>
+__device__ __forceinline__ RowRef row_of(const GArgs& a, int s, uint32_t tile, int r) {
+  const GemvSeg& sg = a.seg[PAIRED ? (r < kR / 2 ? 0 : 1) : s];
+  const uint32_t row = PAIRED ? tile * (kR / 2) + (r % (kR / 2)) : tile * kR + r;
+  return RowRef{sg.body, row < sg.rows ? row : sg.rows - 1, row < sg.rows, sg.type == T_F32};
+}
+
+template <class Epi>
+__global__ void __launch_bounds__(kGThreads) k_gemv_generic(GArgs a, Epi epi) {
+  constexpr bool P = Epi::kPaired;
+  extern __shared__ float xl[];
+  __shared__ float red[kGWaves];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   float ss = 0.f;
-  for (uint32_t i = tid; i < a.cols; i += kThreads) {
+  for (uint32_t i = tid; i < a.cols; i += kGThreads) {
     const float v = a.x[i];
     xl[xpad(i)] = v;
     ss = fmaf(v, v, ss);
   }
   if (a.norm_w) {
-    const float scale = norm_scale(a, ss, red, lane, wave);
-    for (uint32_t i = tid; i < a.cols; i += kThreads) xl[xpad(i)] = (xl[xpad(i)] * scale) * a.norm_w[i];
+    ss = wave_sum(ss);
+    if (lane == 0) red[wave] = ss;
+    __syncthreads();
+    float tot = 0.f;
+    for (int w = 0; w < kGWaves; w++) tot += red[w];
+    const float scale = 1.0f / sqrtf(tot / (float)a.cols + a.eps);
+    for (uint32_t i = tid; i < a.cols; i += kGThreads) xl[xpad(i)] = (xl[xpad(i)] * scale) * a.norm_w[i];
   }
   __syncthreads();
-}
-
-// Main kernel: every segment decodes with Frag.
-template <class Epi, class Frag>
-__global__ void __launch_bounds__(kThreads, kWavesPerSimd) k_gemv(KArgs a, Epi epi) {
-  extern __shared__ float lds[];
-  float* xl = lds;                                    // [groups][36]
-  float* xs = lds + (size_t)a.groups * kGroupStride;  // [cols/16]
-  float* wl = xs + ((a.cols / 16 + 3) & ~3u);         // [cols] norm weights (norm launches), 16-B aligned
-  __shared__ float red[kWaves];
-  __shared__ float part[2 * kWaves * kR];
-  // the wave index is uniform: tile and row bookkeeping stays in scalar registers
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  // tile groups of a.split waves; TG groups in the grid
-  const uint32_t S = a.split, GPB = kWaves / S, TG = gridDim.x * GPB;
-  const uint32_t tg = blockIdx.x * GPB + wave / S, j = wave % S;
-  typename Epi::Wave ws;
-  epi.begin(ws);
-  // tiles per group of this workgroup for segment s: the count of its busiest group
-  auto block_iters = [&](int s) -> uint32_t {
-    uint32_t n = 0;
-    for (uint32_t q = 0; q < GPB; q++) {
-      const uint32_t f0 = (blockIdx.x * GPB + q + TG - a.rot[s]) % TG;
-      if (f0 < a.ntiles[s]) n = max(n, (a.ntiles[s] - 1 - f0) / TG + 1);
-    }
-    return n;
-  };
-  const uint32_t NG = (a.groups + 63) / 64;
-  const uint32_t g0 = min(lane + 64 * min(j, NG - 1), a.groups - 1);
-
-  // first unit of segment 0 in flight while x is staged
-  constexpr bool P = Epi::kPaired;
-  {
-    const uint32_t first = (tg + TG - a.rot[0]) % TG;
-    Frag f;
-    // lanes past the last group load a real group (unconditional loads keep
-    // the fragments' live ranges short); their values are never used
-    if (first < a.ntiles[0]) {
-#pragma unroll
-      for (int r = 0; r < kR; r++) f.template load_row<P>(a, 0, first, g0, r);
-    }
-    stage_x(a, xl, xs, wl, red, tid, lane, wave);
-    run_segment<Frag, Epi>(a, epi, ws, 0, first, TG, block_iters(0), j, f, xl, xs, part, lane, wave);
-  }
-  for (int s = 1; s < a.nseg; s++) {
-    const uint32_t first = (tg + TG - a.rot[s]) % TG;
-    const uint32_t iters = block_iters(s);
-    if (iters == 0) continue;
-    const uint32_t t0 = first < a.ntiles[s] ? first : 0;
-    Frag f;
-#pragma unroll
-    for (int r = 0; r < kR; r++) f.template load_row<P>(a, s, t0, g0, r);
-    run_segment<Frag, Epi>(a, epi, ws, s, first, TG, iters, j, f, xl, xs, part, lane, wave);
-  }
-  epi.finish(ws, lane);
-}
-
-// Rows that are not whole 32-element groups (F32/F16 only): lanes stride over
-// the elements of each row.
-template <class Epi>
-__global__ void __launch_bounds__(kThreads) k_gemv_generic(KArgs a, Epi epi) {
-  extern __shared__ float lds[];
-  __shared__ float red[kWaves];
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  stage_x_generic(a, lds, red, tid, lane, wave);
-  const uint32_t W = gridDim.x * kWaves, wid = blockIdx.x * kWaves + wave;
+  const uint32_t W = gridDim.x * kGWaves, wid = blockIdx.x * kGWaves + wave;
   typename Epi::Wave ws;
   epi.begin(ws);
   for (int s = 0; s < a.nseg; s++) {
@@ -524,20 +469,25 @@ __global__ void __launch_bounds__(kThreads) k_gemv_generic(KArgs a, Epi epi) {
       float acc[kR] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int r = 0; r < kR; r++) {
-        const RowRef rr = row_of<Epi::kPaired>(a, s, t, r);
-        if (!rr.ok) continue;
-        const bool f32 = a.seg[Epi::kPaired ? (r < kR / 2 ? 0 : 1) : s].type == T_F32;
+        const RowRef rr = row_of<P>(a, s, t, r);
         const uint64_t base = rr.row * a.cols;
         float v = 0.f;
         for (uint32_t l = lane; l < a.cols; l += 64) {
-          const float w = f32 ? ((const float*)rr.body)[base + l] : h2f(((const uint16_t*)rr.body)[base + l]);
-          v = fmaf(w, lds[xpad(l)], v);
+          const float w = rr.f32 ? ((const float*)rr.body)[base + l] : h2f(((const uint16_t*)rr.body)[base + l]);
+          v = fmaf(w, xl[xpad(l)], v);
         }
-        acc[r] = v;
+        acc[r] = wave_sum(v);
       }
-#pragma unroll
-      for (int r = 0; r < kR; r++) acc[r] = wave_sum(acc[r]);
-      emit(epi, ws, a, s, t, acc, lane);
+      // lane r < kR owns row r (paired: lanes 0, 1 the gate rows)
+      if (lane < (P ? kR / 2 : kR)) {
+        const RowRef rr = row_of<P>(a, s, t, lane);
+        const int o = P ? lane + kR / 2 : lane ^ 1;
+        const float v = lane == 0 ? acc[0] : lane == 1 ? acc[1] : lane == 2 ? acc[2] : acc[3];
+        const float partner = o == 0 ? acc[0] : o == 1 ? acc[1] : o == 2 ? acc[2] : acc[3];
+        const int es = P ? 0 : s;
+        if (rr.ok) epi.row(ws, es, (uint32_t)rr.row, v, P || Epi::kNeighbor ? partner : 0.f,
+                           epi.pre(ws, es, (uint32_t)rr.row));
+      }
     }
   }
   epi.finish(ws, lane);
@@ -555,23 +505,74 @@ int device_cu_count() {
   return n;
 }
 
-// Rows of >16K columns need more than 64 KiB of LDS: each kernel instance
-// opts in once, through a block-scope static of a function instantiated per
-// kernel (initialised the first time a launch gets there, once even when
-// sessions run on several threads).
+// Rows of >14K columns need more than 64 KiB of LDS in the generic kernel:
+// each instance opts in once, through a block-scope static of a function
+// instantiated per kernel (initialised the first time a launch gets there,
+// once even when sessions run on several threads).
 template <class K>
 hipError_t allow_lds(K kernel) {
   return hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024);
 }
 
-template <class Epi, class F>
-hipError_t dispatch(const KArgs& a, const Epi& epi, uint32_t blocks, size_t lds, hipStream_t st) {
+template <class Epi>
+hipError_t launch_generic(const GemvLaunch& L, const Epi& epi, size_t lds, hipStream_t st) {
+  GArgs a{};
+  a.cols = L.cols;
+  a.x = L.x;
+  a.norm_w = L.norm_w;
+  a.eps = L.eps;
+  a.nseg = Epi::kPaired ? 1 : L.nseg;
+  for (int s = 0; s < L.nseg; s++) a.seg[s] = L.seg[s];
+  uint32_t total = 0;
+  for (int s = 0; s < a.nseg; s++) {
+    const uint32_t per = Epi::kPaired ? kR / 2 : kR;
+    a.ntiles[s] = (L.seg[s].rows + per - 1) / per;
+    total += a.ntiles[s];
+  }
+  if (total == 0) return hipSuccess;
+  const uint32_t per_cu = (uint32_t)std::max<size_t>(1, std::min<size_t>(2, (160 * 1024) / lds));
+  const uint32_t blocks = std::min<uint32_t>((total + kGWaves - 1) / kGWaves, per_cu * device_cu_count());
+  uint32_t acc = 0;
+  for (int s = 0; s < a.nseg; s++) {
+    a.rot[s] = acc % (blocks * kGWaves);
+    acc += a.ntiles[s];
+  }
   if (lds > 64 * 1024) {
-    static const hipError_t opted = allow_lds(k_gemv<Epi, F>);
+    static const hipError_t opted = allow_lds(k_gemv_generic<Epi>);
     if (opted != hipSuccess) return opted;
   }
-  hipLaunchKernelGGL((k_gemv<Epi, F>), dim3(blocks), dim3(kThreads), lds, st, a, epi);
+  hipLaunchKernelGGL(k_gemv_generic<Epi>, dim3(blocks), dim3(kGThreads), lds, st, a, epi);
   return hipGetLastError();
+}
+
+template <class Epi, class Q, int K, bool WIDE>
+hipError_t go(const KArgs& a, const Epi& epi, hipStream_t st) {
+  constexpr uint32_t kW = WIDE ? kWavesWide : kWavesNarrow;
+  const uint32_t G = 64u >> a.lg_lanes, groups = (a.total + G - 1) / G, per = kW / a.split;
+  // persistent: as many workgroups as run at once (kMinWaves waves per SIMD)
+  const uint32_t most = (uint32_t)device_cu_count() * (4 * kMinWaves / kW);
+  const uint32_t blocks = std::min((groups + per - 1) / per, most);
+  hipLaunchKernelGGL((k_gemv<Epi, Q, K, WIDE>), dim3(blocks), dim3(64 * kW), 0, st, a, epi);
+  return hipGetLastError();
+}
+
+// K: the smallest of the type's piece counts that covers a row with one wave
+// (x then takes at most 64 registers); longer rows: KM pieces and S waves.
+template <class Epi, class Q, int K2, int K4, int KM>
+hipError_t dispatch(KArgs a, const Epi& epi, hipStream_t st) {
+  a.pieces = a.cols / Q::kE;
+  a.lg_lanes = 6;
+  a.split = 1;
+  if (a.pieces <= 64) {
+    a.lg_lanes = a.pieces <= 16 ? 4 : a.pieces <= 32 ? 5 : 6;
+    return go<Epi, Q, 1, false>(a, epi, st);
+  }
+  if (K2 < K4 && a.pieces <= 64 * K2) return go<Epi, Q, K2, false>(a, epi, st);
+  if (K4 < KM && a.pieces <= 64 * K4) return go<Epi, Q, K4, false>(a, epi, st);
+  if (a.pieces <= 64 * KM) return go<Epi, Q, KM, false>(a, epi, st);
+  a.split = a.pieces <= 128 * KM ? 2 : a.pieces <= 256 * KM ? 4 : 8;
+  if (a.pieces > 64 * KM * a.split) return hipErrorInvalidValue;
+  return go<Epi, Q, KM, true>(a, epi, st);
 }
 
 template <class Epi>
@@ -582,69 +583,45 @@ hipError_t launch(const GemvLaunch& L, const Epi& epi, hipStream_t st) {
   for (int s = 0; s < L.nseg; s++) n_mfma += mfma_type(L.seg[s].type) ? 1 : 0;
   if (n_mfma == L.nseg) return launch_mfma(L, epi, st);
   if (n_mfma != 0) return hipErrorInvalidValue;
-  KArgs a{};
-  a.cols = L.cols;
-  a.groups = (L.cols + 31) / 32;
-  a.x = L.x;
-  a.norm_w = L.norm_w;
-  a.eps = L.eps;
   const bool generic = L.cols % 32 != 0;
   for (int s = 0; s < L.nseg; s++) {
-    a.seg[s] = L.seg[s];
     const uint32_t t = L.seg[s].type;
     if (t == T_Q8K && L.cols % 256) return hipErrorInvalidValue;
     if (generic && t != T_F32 && t != T_F16) return hipErrorInvalidValue;
   }
-  if (Epi::kPaired) {
-    if (L.nseg != 2 || L.seg[0].rows != L.seg[1].rows || L.seg[0].type != L.seg[1].type) return hipErrorInvalidValue;
-    a.nseg = 1;
-    a.ntiles[0] = (L.seg[0].rows + kR / 2 - 1) / (kR / 2);
-  } else {
-    a.nseg = L.nseg;
-    for (int s = 0; s < L.nseg; s++) a.ntiles[s] = (L.seg[s].rows + kR - 1) / kR;
-  }
-  const size_t lds = (size_t)a.groups * kGroupStride * 4 + (size_t)((a.cols / 16 + 3) & ~3u) * 4 +
-                     (L.norm_w && !generic ? (size_t)a.cols * 4 : 0);
+  if (Epi::kPaired &&
+      (L.nseg != 2 || L.seg[0].rows != L.seg[1].rows || L.seg[0].type != L.seg[1].type))
+    return hipErrorInvalidValue;
+  // The longest rows taken: what 150 KiB hold of x, its 16-element sums and
+  // the norm weights (32336 columns, 17552 with a norm), so that both kernels
+  // accept the same matrices.
+  const size_t lds = (size_t)((L.cols + 31) / 32) * kGroupStride * 4 + (size_t)((L.cols / 16 + 3) & ~3u) * 4 +
+                     (L.norm_w && !generic ? (size_t)L.cols * 4 : 0);
   if (lds > 150 * 1024) return hipErrorInvalidValue;
-  uint32_t total = 0;
-  for (int s = 0; s < a.nseg; s++) total += a.ntiles[s];
-  if (total == 0) return hipSuccess;
-  // persistent grid: as many workgroups as fit per CU (LDS-bound for long
-  // rows).  Long rows (at least 4 units) with fewer row tiles than resident
-  // waves share each tile's units among `split` waves (the 8B down projection:
-  // 1024 tiles of 7 units).
-  const uint32_t per_cu = (uint32_t)std::max<size_t>(1, std::min<size_t>(kBlocksPerCu, (160 * 1024) / lds));
-  const uint32_t resident = per_cu * device_cu_count() * kWaves;
-  const uint32_t NG = (a.groups + 63) / 64;
-  uint32_t split = 1;
-  if (!generic && NG >= 4)
-    while (split < (uint32_t)kWaves && split < NG && total * split < resident) split *= 2;
-  a.split = split;
-  const uint32_t blocks = std::min<uint32_t>((total * split + kWaves - 1) / kWaves, per_cu * device_cu_count());
-  const uint32_t TG = blocks * (kWaves / split);
-  uint32_t acc = 0;
+  if (generic) return launch_generic(L, epi, lds, st);
+  if (!Epi::kPaired && L.nseg > Segs<Epi>::kN) return hipErrorInvalidValue;
+  KArgs a{};
+  a.cols = L.cols;
+  a.x = L.x;
+  a.norm_w = L.norm_w;
+  a.eps = L.eps;
+  a.nseg = Epi::kPaired ? 1 : L.nseg;
+  for (int s = 0; s < L.nseg; s++) a.seg[s] = L.seg[s];
   for (int s = 0; s < a.nseg; s++) {
-    a.rot[s] = acc % TG;
-    acc += a.ntiles[s];
+    a.nunits[s] = Epi::kPaired ? L.seg[s].rows : (L.seg[s].rows + 1) / 2;
+    a.total += a.nunits[s];
   }
-  if (generic) {
-    if (lds > 64 * 1024) {
-      static const hipError_t opted = allow_lds(k_gemv_generic<Epi>);
-      if (opted != hipSuccess) return opted;
-    }
-    hipLaunchKernelGGL(k_gemv_generic<Epi>, dim3(blocks), dim3(kThreads), lds, st, a, epi);
-    return hipGetLastError();
-  }
+  if (a.total == 0) return hipSuccess;
   // one type per launch on this path (the mixed Q4_K / Q6_K layers take the MFMA kernel)
   const uint32_t ta = L.seg[0].type;
   for (int s = 1; s < a.nseg; s++)
     if (L.seg[s].type != ta) return hipErrorInvalidValue;
   switch (ta) {
-    case T_Q8_0: return dispatch<Epi, FragQ80>(a, epi, blocks, lds, st);
-    case T_Q4_0: return dispatch<Epi, FragQ40>(a, epi, blocks, lds, st);
-    case T_Q8K: return dispatch<Epi, FragQ8K>(a, epi, blocks, lds, st);
-    case T_F32: return dispatch<Epi, FragF32>(a, epi, blocks, lds, st);
-    case T_F16: return dispatch<Epi, FragF16>(a, epi, blocks, lds, st);
+    case T_Q8_0: return dispatch<Epi, PieceQ80, 2, 4, 4>(a, epi, st);
+    case T_Q4_0: return dispatch<Epi, PieceQ40, 2, 2, 2>(a, epi, st);
+    case T_Q8K: return dispatch<Epi, PieceQ8K, 4, 4, 4>(a, epi, st);
+    case T_F32: return dispatch<Epi, PieceF32, 4, 16, 16>(a, epi, st);
+    case T_F16: return dispatch<Epi, PieceF16, 2, 4, 8>(a, epi, st);
     default: return hipErrorInvalidValue;
   }
 }
