@@ -130,7 +130,8 @@ int ifx_ops_attention_decode(const float* q, const void* k_cache, const void* v_
   IFX_TRY(put_state(cs, (uint32_t)(n_rows - 1), 0, &state));
   a.state = state;
   a.out = out;
-  IFX_TRY(alloc_records(cs, &a));
+  a.one_chunk = n_rows <= a.chunk;
+  if (!a.one_chunk) IFX_TRY(alloc_records(cs, &a));
   IFX_HIP(launch_attn_decode(a, st));
   return cs.finish();
 }
@@ -164,6 +165,7 @@ int ifx_ops_attention_decode_o(const float* q, const void* k_cache, const void* 
     IFX_HIP(launch_attn_partials(a, st));
     IFX_HIP(launch_mfma_residual_merge(go, a, h, st, merge_bound));
   } else {
+    a.one_chunk = n_rows <= a.chunk;
     IFX_HIP(launch_attn_decode(a, st));
     IFX_HIP(gemv_residual(go, h, st));
   }

@@ -69,8 +69,8 @@ struct ifx_session {
   // captured steps: [sampling][merge bound / 8] (the greedy step, the step
   // with the sampler before finalize; each with the attention merge in its own
   // launch (bound 0) or in the O projection's prologue, which loads the first
-  // `merge_bound` chunk records up front)
-  static constexpr int kMergeGraphs = 7;
+  // `merge_bound` chunk records up front; the last: one chunk, no merge)
+  static constexpr int kMergeGraphs = 8, kOneChunkGraph = 7;
   hipGraphExec_t exec[2][kMergeGraphs] = {};
   bool graph_tried[2][kMergeGraphs] = {};
   bool sampling = false;                 // set for the duration of ifx_generate_sampled
@@ -78,6 +78,7 @@ struct ifx_session {
   // through the tiled launches, the attention merge in its own launch
   bool deterministic = false;
   uint32_t merge_bound = 0;              // of the step being enqueued: 0, or a multiple of 8 up to 48
+  bool one_chunk = false;                // of the step being enqueued: it attends at most attn_chunk rows
   float* probs = nullptr;                // sampler weights [vocab]
   void* sample_ws = nullptr;             // sampler histogram, sums and candidates (sample_ws_bytes)
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -365,6 +366,7 @@ int enqueue_class(ifx_session* s, int k, size_t l) {
       AttnArgs a{qkv_split(s) ? layer_q(s, l) : s->q, kc, vc, s->attn, s->partial, s->state, (uint32_t)c.n_heads,
                  (uint32_t)c.n_kv_heads, (uint32_t)c.head_dim, s->max_chunks, s->attn_chunk,
                  (uint32_t)s->max_seq, kv16};
+      a.one_chunk = s->one_chunk;
       const GemvLaunch go = o_launch(s, L);
       // the merge of the chunk records moves into the O launch's prologue
       const bool fused = s->merge_bound && merge_o_supported(go, a);
@@ -414,17 +416,17 @@ uint64_t tensor_stream_bytes(const ifx_tensor* t) { return t->L.body_bytes + t->
 // step's chunk count rounded up to a multiple of merge_o_bound_step() as the
 // records its prologue loads.  `rows` bounds the rows the step attends (the
 // cache rows before it + 1).  IFX_MERGE_O=0 / 1 takes the separate / the
-// fused merge at any length.
+// fused merge at any length.  Rows of one chunk need no merge (AttnArgs::
+// one_chunk; the same bits as the separate merge gives).
 void choose_merge(ifx_session* s, uint64_t rows) {
-  if (s->deterministic) {
-    s->merge_bound = 0;
-    return;
-  }
   const uint64_t nch = (rows + s->attn_chunk - 1) / s->attn_chunk, step = merge_o_bound_step();
   const uint32_t most = merge_o_first_chunks();
   const uint32_t bound = (uint32_t)std::max<uint64_t>(step, (nch + step - 1) / step * step);
   const char* f = getenv("IFX_MERGE_O");
-  if (f && (f[0] == '0' || f[0] == '1') && f[1] == 0) s->merge_bound = f[0] == '1' ? std::min(bound, most) : 0;
+  const bool forced = !s->deterministic && f && (f[0] == '0' || f[0] == '1') && f[1] == 0;
+  s->one_chunk = nch <= 1 && !forced;
+  if (s->deterministic || s->one_chunk) s->merge_bound = 0;
+  else if (forced) s->merge_bound = f[0] == '1' ? std::min(bound, most) : 0;
   else s->merge_bound = nch <= most ? bound : 0;
 }
 
@@ -432,7 +434,7 @@ void choose_merge(ifx_session* s, uint64_t rows) {
 // runtime refuses capture.
 int run_step(ifx_session* s, uint64_t rows) {
   choose_merge(s, rows);
-  const int gi = (int)(s->merge_bound / merge_o_bound_step());
+  const int gi = s->one_chunk ? ifx_session::kOneChunkGraph : (int)(s->merge_bound / merge_o_bound_step());
   if (gi >= ifx_session::kMergeGraphs) return set_error(IFX_E_INVALID_ARG, "merge bound %u", s->merge_bound);
   hipGraphExec_t& exec = s->exec[s->sampling][gi];
   bool& tried = s->graph_tried[s->sampling][gi];

@@ -396,8 +396,16 @@ __global__ void __launch_bounds__(kThreads, GT == 8 ? 3 : 1) k_attn_decode(AttnA
       acc.x += wo[w][g][cp].x;
       acc.y += wo[w][g][cp].y;
     }
-    *(float2*)(part + g * HD + 2 * cp) = acc;
+    if (a.one_chunk) {  // the softmax is over this chunk alone: what its merge would write
+      float L = wst[0][1][g];
+#pragma unroll
+      for (int w = 1; w < kThreads / 64; w++) L += wst[w][1][g];
+      *(float2*)(a.out + ((uint64_t)hk * G + g) * HD + 2 * cp) = make_float2(acc.x / L, acc.y / L);
+    } else {
+      *(float2*)(part + g * HD + 2 * cp) = acc;
+    }
   }
+  if (a.one_chunk) return;
   if (tid < (int)G) {
     float L = wst[0][1][tid];
 #pragma unroll
@@ -547,6 +555,15 @@ void launch_typed(const AttnArgs& a0, hipStream_t st, bool merge) {
   const char* hf = getenv("IFX_ATTN_HKF");
   const bool forced = hf && (hf[0] == '0' || hf[0] == '1') && hf[1] == 0;
   a.hk_fast = forced ? hf[0] == '1' : (uint64_t)a.max_chunks * a.n_kv_heads <= 2ull * (uint64_t)attn_cu_count();
+  if (a.one_chunk) {
+    // One launch instead of two, and no workgroups for the cache's other
+    // chunks: a step of at most 64 rows pays one kernel latency less per layer
+    // (tiny model, 24 steps of 6 layers: 4394 -> 3823 us; the operator over 16
+    // rows 27.9 -> 24.0 us).
+    a.max_chunks = 1;
+    a.hk_fast = 1;
+    merge = false;
+  }
   const dim3 grid = a.hk_fast ? dim3(a.n_kv_heads, a.max_chunks) : dim3(a.max_chunks, a.n_kv_heads);
   const uint32_t G = a.n_heads / a.n_kv_heads;
 #define IFX_ATTN(HD_, G_)                                                                          \

@@ -286,6 +286,9 @@ struct AttnArgs {
   uint32_t n_heads, n_kv_heads, head_dim, max_chunks, chunk, max_seq;
   uint32_t kv_f16;
   uint32_t hk_fast = 0;  // chunk grid ordered kv head fastest (set by the launcher)
+  // the attended rows fit one chunk (the host's bound on them is at most
+  // `chunk`): the chunk's workgroup writes the attention output itself
+  uint32_t one_chunk = 0;
 };
 hipError_t launch_attn_decode(const AttnArgs& a, hipStream_t st);
 // the chunk records only (their merge is left to launch_mfma_residual_merge)
