@@ -39,17 +39,10 @@ def test_steps_across_the_line(tiny_path, monkeypatch):
     g = GpuModel(tiny_path)
     ids = synth.token_ids(70, g.vocab, seed=5)
 
-    def steps(prefill):
+    def steps():
         s = g.session(96)
         s.set_deterministic(True)
-        s.set_prefill_batch(0)
-        if prefill:
-            assert s.prefill(ids[:prefill], want_logits=False)[0] == 0
-        out = []
-        for t in ids[prefill:]:
-            rc, lg = s.decode_step(int(t))
-            assert rc == 0
-            out.append(lg)
+        out = [s.decode_step(int(t))[1] for t in ids]
         s.close()
         return np.array(out)
 
@@ -61,7 +54,6 @@ def test_steps_across_the_line(tiny_path, monkeypatch):
         monkeypatch.delenv("IFX_MERGE_O")
         return np.array(out)
 
-    one = steps(0)
-    assert np.array_equal(one, separate(monkeypatch))  # Q8_0 launches have one summation order
-    assert np.array_equal(steps(60)[3:], steps(63))
+    # Q8_0 launches have one summation order, deterministic session or not
+    assert np.array_equal(steps(), separate(monkeypatch))
     g.close()
