@@ -109,7 +109,7 @@ int upload_matrix(uint32_t type, const uint8_t* src, uint64_t nbytes, uint64_t r
                      (unsigned long long)cols);
   ifx_tensor* t = new ifx_tensor();
   const uint64_t body_al = (body + 255) / 256 * 256;
-  if (hipMalloc(&t->alloc, body_al + scal + 16) != hipSuccess) {
+  if (hipMalloc(&t->alloc, body_al + scal + kTensorPad) != hipSuccess) {
     delete t;
     return set_error(IFX_E_OOM, "hipMalloc of %llu bytes failed", (unsigned long long)(body_al + scal));
   }
@@ -321,6 +321,30 @@ int ifx_gemv(const ifx_tensor* w, const float* x, float* y, void* stream) {
   return IFX_OK;
 }
 
+}  // extern "C"
+
+// Runs enqueue(workspace of `bytes`) on st: the kept one on the library's
+// stream; on a caller's stream (which may be under capture, or gone before the
+// next call) one allocated and freed in its order.
+template <class F>
+static int with_workspace(hipStream_t st, uint64_t bytes, F enqueue) {
+  if (st == g_stream) {
+    StreamWorkspace ws(st);
+    IFX_HIP(ws.take(bytes));
+    IFX_HIP(enqueue((uint8_t*)ws.ptr()));
+    return IFX_OK;
+  }
+  uint8_t* buf = nullptr;
+  IFX_HIP(hipMallocAsync((void**)&buf, bytes, st));
+  const hipError_t e = enqueue(buf);
+  const hipError_t ef = hipFreeAsync(buf, st);
+  IFX_HIP(e);
+  IFX_HIP(ef);
+  return IFX_OK;
+}
+
+extern "C" {
+
 int ifx_matmul_qt(const float* a, uint64_t m, const ifx_tensor* w, float* c, void* stream) {
   IFX_TRY(device_init());
   if (!w || (m && (!a || !c))) return set_error(IFX_E_INVALID_ARG, "null argument");
@@ -330,6 +354,14 @@ int ifx_matmul_qt(const float* a, uint64_t m, const ifx_tensor* w, float* c, voi
     hipStream_t st = stream_of(stream);
     const uint64_t k = w->L.cols;
     const GemmW gw = gemm_w(w->L);
+    if (gemm_skinny_ok(a, m, gw, c)) {  // a few tokens: one launch from the f32 rows
+      const uint64_t part = gemm_skinny_ws_bytes((uint32_t)m, gw);
+      if (part == 0) {
+        IFX_HIP(gemm_skinny(a, (uint32_t)m, gw, c, nullptr, st));
+        return IFX_OK;
+      }
+      return with_workspace(st, part, [&](uint8_t* ws) { return gemm_skinny(a, (uint32_t)m, gw, c, (float*)ws, st); });
+    }
     // one workspace: hi, lo planes, group sums, row exponents, split-K partial
     // tiles of short inputs
     const uint64_t part_limit = 64ull << 20;
@@ -343,21 +375,7 @@ int ifx_matmul_qt(const float* a, uint64_t m, const ifx_tensor* w, float* c, voi
       const hipError_t e = launch_prep_rows(a, (uint32_t)m, (uint32_t)k, (uint32_t)k, nullptr, 0.f, in, st);
       return e == hipSuccess ? gemm_store(in, gw, c, (uint32_t)w->L.rows, st) : e;
     };
-    if (st == g_stream) {
-      StreamWorkspace ws(st);
-      IFX_HIP(ws.take(bytes));
-      IFX_HIP(enqueue((uint8_t*)ws.ptr()));
-      return IFX_OK;
-    }
-    // a caller's stream (which may be under capture, or gone before the next
-    // call): allocated and freed in its order
-    uint8_t* buf = nullptr;
-    IFX_HIP(hipMallocAsync((void**)&buf, bytes, st));
-    const hipError_t e = enqueue(buf);
-    const hipError_t ef = hipFreeAsync(buf, st);
-    IFX_HIP(e);
-    IFX_HIP(ef);
-    return IFX_OK;
+    return with_workspace(st, bytes, enqueue);
   }
   for (uint64_t i = 0; i < m; i++) {
     GemvLaunch L;

@@ -91,6 +91,11 @@ __host__ __device__ inline void tile_strides(uint32_t type, uint64_t rows, uint6
   *bstride = row_tiles(rows) * unit;
 }
 
+// bytes of an uploaded matrix's allocation past its arrays: kernels that read
+// rows of 32-blocks eight blocks at a time may read (and not use) up to seven
+// blocks past the last row
+constexpr uint64_t kTensorPad = 256;
+
 struct DevLayout {
   uint32_t type = 0;
   uint64_t rows = 0, cols = 0;

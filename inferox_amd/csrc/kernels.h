@@ -199,6 +199,17 @@ hipError_t gemm_rows(const GemmIn& in, const GemmW& w, void* y, uint32_t ldy, ui
 // mid[t * ld + n] = swiglu(gate row n . A[t], up row n . A[t])
 hipError_t gemm_swiglu(const GemmIn& in, const GemmW& gate, const GemmW& up, float* mid, uint32_t ld,
                        hipStream_t st);
+// y[m][rows] = x[m][cols] W^T for m <= kSkinnyRows tokens, straight from the
+// f32 rows in one launch (kern_gemm_skinny.hip); ws: gemm_skinny_ws_bytes bytes
+constexpr uint32_t kSkinnyRows = 64;
+// y may not overlap x: workgroups still read x while others write y (the other
+// GEMM reads its own copy of x)
+inline bool gemm_skinny_ok(const float* x, uint64_t m, const GemmW& w, const float* y) {
+  const uintptr_t x0 = (uintptr_t)x, y0 = (uintptr_t)y;
+  return m <= kSkinnyRows && (x0 + m * w.cols * 4 <= y0 || y0 + m * w.rows * 4 <= x0);
+}
+uint64_t gemm_skinny_ws_bytes(uint32_t m, const GemmW& w);
+hipError_t gemm_skinny(const float* x, uint32_t m, const GemmW& w, float* y, float* ws, hipStream_t st);
 // rows x cols of x (row stride ld), rms_norm'ed with norm_w when non-null
 // (src/ops.rs:155-180), into the GEMM operand `out` (out.k == cols, rows <= out.m)
 hipError_t launch_prep_rows(const float* x, uint32_t rows, uint32_t ld, uint32_t cols, const float* norm_w,

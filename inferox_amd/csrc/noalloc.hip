@@ -81,6 +81,11 @@ int ifx_matmul_qt_noalloc(const float* a, uint64_t m, const ifx_tensor* w, float
                        (unsigned long long)kMaxElems);
     uint8_t* s = nullptr;
     IFX_TRY(scratch_on_device(&s));
+    // a few tokens: the launch ifx_matmul_qt takes, its partial sums in the array
+    if (gemm_skinny_ok(a, m, gemm_w(w->L), c) && gemm_skinny_ws_bytes((uint32_t)m, gemm_w(w->L)) <= kScratchBytes) {
+      IFX_HIP(gemm_skinny(a, (uint32_t)m, gemm_w(w->L), c, (float*)s, st));
+      return IFX_OK;
+    }
     // the same carving as ifx_matmul_qt's allocation, inside the array
     const uint64_t bh = al256(m * k * 2), bg = al256(m * (k / 256 + 1) * 32), br = al256(m * 4);
     const uint64_t used = 2 * bh + bg + br;
