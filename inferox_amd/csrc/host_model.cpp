@@ -66,13 +66,16 @@ struct ifx_session {
   DevState* state = nullptr;
   uint32_t *out_tokens = nullptr, *feed_ids = nullptr;
   uint32_t attn_chunk = 64, max_chunks = 0;
-  // captured steps: [sampling][merge bound / 8] (the greedy step, the step
-  // with the sampler before finalize; each with the attention merge in its own
+  // captured steps: [kind][merge bound / 8] (the greedy step, the step with the
+  // sampler before finalize, the step of a prompt token whose logits nobody
+  // reads: no output head; each with the attention merge in its own
   // launch (bound 0) or in the O projection's prologue, which loads the first
   // `merge_bound` chunk records up front; the last: one chunk, no merge)
   static constexpr int kMergeGraphs = 8, kOneChunkGraph = 7;
-  hipGraphExec_t exec[2][kMergeGraphs] = {};
-  bool graph_tried[2][kMergeGraphs] = {};
+  static constexpr int kKinds = 3, kFeedKind = 2;
+  hipGraphExec_t exec[kKinds][kMergeGraphs] = {};
+  bool graph_tried[kKinds][kMergeGraphs] = {};
+  bool feed_only = false;                // of the step being enqueued: no output head
   bool sampling = false;                 // set for the duration of ifx_generate_sampled
   // fixed summation order (ifx_session_set_deterministic): q/k/v, O and down
   // through the tiled launches, the attention merge in its own launch
@@ -337,7 +340,7 @@ int enqueue_class(ifx_session* s, int k, size_t l) {
       return IFX_OK;
     }
     case 7:
-      if (s->sampling)
+      if (s->sampling && !s->feed_only)
         IFX_HIP(launch_sample(s->logits, s->probs, sample_ws(s->sample_ws), (uint32_t)c.vocab_size, s->state, st));
       IFX_HIP(launch_finalize(s->state, st));
       return IFX_OK;
@@ -403,7 +406,7 @@ int enqueue_step(ifx_session* s) {
   IFX_TRY(enqueue_class(s, 0, 0));
   for (size_t l = 0; l < s->m->layers.size(); l++)
     for (int k = 1; k <= 5; k++) IFX_TRY(enqueue_class(s, k, l));
-  IFX_TRY(enqueue_class(s, 6, 0));
+  if (!s->feed_only) IFX_TRY(enqueue_class(s, 6, 0));
   IFX_TRY(enqueue_class(s, 7, 0));
   return IFX_OK;
 }
@@ -432,12 +435,21 @@ void choose_merge(ifx_session* s, uint64_t rows) {
 
 // Replay the captured step (capturing it on first use); direct launches if the
 // runtime refuses capture.
-int run_step(ifx_session* s, uint64_t rows) {
+// head = false: a prompt token before the last whose logits are not asked for;
+// only its K and V rows matter (a 32000 x 288 Q8_0 head is a tenth of the tiny
+// model's step, the 8B head 5%).
+int run_step(ifx_session* s, uint64_t rows, bool head = true) {
   choose_merge(s, rows);
+  s->feed_only = !head;
+  struct Reset {
+    ifx_session* s;
+    ~Reset() { s->feed_only = false; }
+  } reset{s};
+  const int kind = head ? (s->sampling ? 1 : 0) : ifx_session::kFeedKind;
   const int gi = s->one_chunk ? ifx_session::kOneChunkGraph : (int)(s->merge_bound / merge_o_bound_step());
   if (gi >= ifx_session::kMergeGraphs) return set_error(IFX_E_INVALID_ARG, "merge bound %u", s->merge_bound);
-  hipGraphExec_t& exec = s->exec[s->sampling][gi];
-  bool& tried = s->graph_tried[s->sampling][gi];
+  hipGraphExec_t& exec = s->exec[kind][gi];
+  bool& tried = s->graph_tried[kind][gi];
   if (!tried) {
     tried = true;
     // IFX_NO_GRAPH=1: launch the step's kernels directly (used under profilers
@@ -816,7 +828,7 @@ int ifx_session_set_deterministic(ifx_session* s, int on) {
   if (s->deterministic == (on == 1)) return IFX_OK;
   // the captured steps hold the other launches: capture again on next use
   IFX_HIP(hipStreamSynchronize(s->stream));
-  for (int i = 0; i < 2; i++)
+  for (int i = 0; i < ifx_session::kKinds; i++)
     for (int j = 0; j < ifx_session::kMergeGraphs; j++) {
       if (s->exec[i][j]) IFX_HIP(hipGraphExecDestroy(s->exec[i][j]));
       s->exec[i][j] = nullptr;
@@ -877,7 +889,7 @@ int ifx_prefill(ifx_session* s, const uint32_t* ids, uint64_t n, float* logits_o
   IFX_HIP(hipEventRecord(s->ev0, s->stream));
   const size_t V = m->cfg.vocab_size;
   for (uint64_t t = 0; t < n; t++) {
-    IFX_TRY(run_step(s, s->len + t + 1));
+    IFX_TRY(run_step(s, s->len + t + 1, logits_out != nullptr || t + 1 == n));
     if (logits_out)
       IFX_HIP(hipMemcpyAsync(logits_out + t * V, s->logits, V * 4, hipMemcpyDeviceToHost, s->stream));
   }
