@@ -1,5 +1,7 @@
 // kern_ops.hip — f32 operators (src/ops.rs) on device buffers, greedy argmax
 // and the per-step state kernels.  Compiled with -ffp-contract=off.
+#include <algorithm>
+
 #include "kernels.h"
 
 namespace ifx {
@@ -44,7 +46,7 @@ __global__ void __launch_bounds__(256) k_matmul_t(const float* __restrict__ a, c
   if (lane == 0) c[out] = s;
 }
 
-// ops::rms_norm_rows (src/ops.rs:155-180).
+// ops::rms_norm_rows (src/ops.rs:155-180): a workgroup per row.
 __global__ void __launch_bounds__(256) k_rms_norm(float* __restrict__ x, const float* __restrict__ w,
                                                   uint64_t n, float eps) {
   __shared__ float red[4];
@@ -56,22 +58,74 @@ __global__ void __launch_bounds__(256) k_rms_norm(float* __restrict__ x, const f
   for (uint64_t i = threadIdx.x; i < n; i += blockDim.x) row[i] = (row[i] * scale) * w[i];
 }
 
+// The same for rows of whole quads up to 4096 K columns, which stay in
+// registers between the sum and the scaling: one round trip to memory instead
+// of 2 n / 256 (100 rows of 4096: 11.6 us by the loop above).
+template <int K>
+__global__ void __launch_bounds__(1024) k_rms_norm_reg(float* __restrict__ x, const float* __restrict__ w,
+                                                       uint32_t n4, float n, float eps) {
+  __shared__ float red[16];
+  float4* row = (float4*)x + (uint64_t)blockIdx.x * n4;
+  float4 v[K], g[K];
+  float ss = 0.f;
+#pragma unroll
+  for (int k = 0; k < K; k++) {
+    const uint32_t i = threadIdx.x + blockDim.x * k;
+    const bool ok = i < n4;
+    v[k] = ok ? row[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+    g[k] = ok ? ((const float4*)w)[i] : v[k];
+  }
+#pragma unroll
+  for (int k = 0; k < K; k++) {
+    ss = fmaf(v[k].x, v[k].x, ss);
+    ss = fmaf(v[k].y, v[k].y, ss);
+    ss = fmaf(v[k].z, v[k].z, ss);
+    ss = fmaf(v[k].w, v[k].w, ss);
+  }
+  ss = block_reduce<false>(ss, red);
+  const float scale = 1.0f / sqrtf(ss / n + eps);
+#pragma unroll
+  for (int k = 0; k < K; k++) {
+    const uint32_t i = threadIdx.x + blockDim.x * k;
+    if (i < n4)
+      row[i] = make_float4((v[k].x * scale) * g[k].x, (v[k].y * scale) * g[k].y, (v[k].z * scale) * g[k].z,
+                           (v[k].w * scale) * g[k].w);
+  }
+}
+
 __device__ __forceinline__ float silu_ref(float g) {
   float c = fminf(fmaxf(g, -80.f), 80.f);
   if (g != g) c = g;
   return g * (1.0f / (1.0f + expf(-c)));
 }
 
-__global__ void k_swiglu(const float* g, const float* u, float* o, uint64_t n) {
-  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (uint64_t)gridDim.x * blockDim.x)
-    o[i] = silu_ref(g[i]) * u[i];
+// Elementwise kernels, four elements per thread where every pointer is
+// 16-byte aligned (QUADS; the last n % 4 elements singly).
+template <bool QUADS, class F>
+__device__ __forceinline__ void each(float* o, const float* a, const float* b, uint64_t n, F f) {
+  const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x, step = (uint64_t)gridDim.x * blockDim.x;
+  if (QUADS) {
+    for (uint64_t i = t; i < n / 4; i += step) {
+      const float4 x = ((const float4*)a)[i], y = ((const float4*)b)[i];
+      ((float4*)o)[i] = make_float4(f(x.x, y.x), f(x.y, y.y), f(x.z, y.z), f(x.w, y.w));
+    }
+    if (t < n % 4) {
+      const uint64_t i = n / 4 * 4 + t;
+      o[i] = f(a[i], b[i]);
+    }
+  } else {
+    for (uint64_t i = t; i < n; i += step) o[i] = f(a[i], b[i]);
+  }
 }
 
+template <bool QUADS>
+__global__ void k_swiglu(const float* g, const float* u, float* o, uint64_t n) {
+  each<QUADS>(o, g, u, n, [](float a, float b) { return silu_ref(a) * b; });
+}
+
+template <bool QUADS>
 __global__ void k_add(float* o, const float* b, uint64_t n) {
-  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (uint64_t)gridDim.x * blockDim.x)
-    o[i] = o[i] + b[i];
+  each<QUADS>(o, o, b, n, [](float x, float y) { return x + y; });
 }
 
 // ops::softmax_rows (src/ops.rs:223-239): max (NaN-skipping, like f32::max),
@@ -256,17 +310,41 @@ hipError_t launch_matmul_t_f32(const float* a, const float* b, float* c, uint64_
 hipError_t launch_rms_norm_rows(float* x, const float* w, uint64_t n, uint64_t rows, float eps,
                                 hipStream_t st) {
   if (rows == 0 || n == 0) return hipSuccess;
+  const bool quads = n % 4 == 0 && ((uintptr_t)x | (uintptr_t)w) % 16 == 0;
+  if (quads && n <= 16384) {
+    const uint32_t n4 = (uint32_t)(n / 4), threads = std::min(1024u, (n4 + 63) / 64 * 64);
+    if (n4 <= 1024)
+      hipLaunchKernelGGL(k_rms_norm_reg<1>, dim3((unsigned)rows), dim3(threads), 0, st, x, w, n4, (float)n, eps);
+    else
+      hipLaunchKernelGGL(k_rms_norm_reg<4>, dim3((unsigned)rows), dim3(threads), 0, st, x, w, n4, (float)n, eps);
+    return hipGetLastError();
+  }
   hipLaunchKernelGGL(k_rms_norm, dim3((unsigned)rows), dim3(256), 0, st, x, w, n, eps);
   return hipGetLastError();
 }
 
+// (an output that starts inside an input is left to the one-element form: its
+// elements are read and written in the order they always were)
+static bool quads_ok(const float* o, const float* a, const float* b, uint64_t n) {
+  auto clear = [&](const float* p) {
+    return p == o || (uintptr_t)p + n * 4 <= (uintptr_t)o || (uintptr_t)o + n * 4 <= (uintptr_t)p;
+  };
+  return ((uintptr_t)o | (uintptr_t)a | (uintptr_t)b) % 16 == 0 && clear(a) && clear(b);
+}
+
 hipError_t launch_swiglu(const float* g, const float* u, float* o, uint64_t n, hipStream_t st) {
-  hipLaunchKernelGGL(k_swiglu, dim3(blocks_for(n)), dim3(256), 0, st, g, u, o, n);
+  if (quads_ok(o, g, u, n))
+    hipLaunchKernelGGL(k_swiglu<true>, dim3(blocks_for((n + 3) / 4)), dim3(256), 0, st, g, u, o, n);
+  else
+    hipLaunchKernelGGL(k_swiglu<false>, dim3(blocks_for(n)), dim3(256), 0, st, g, u, o, n);
   return hipGetLastError();
 }
 
 hipError_t launch_add(float* o, const float* b, uint64_t n, hipStream_t st) {
-  hipLaunchKernelGGL(k_add, dim3(blocks_for(n)), dim3(256), 0, st, o, b, n);
+  if (quads_ok(o, o, b, n))
+    hipLaunchKernelGGL(k_add<true>, dim3(blocks_for((n + 3) / 4)), dim3(256), 0, st, o, b, n);
+  else
+    hipLaunchKernelGGL(k_add<false>, dim3(blocks_for(n)), dim3(256), 0, st, o, b, n);
   return hipGetLastError();
 }
 
