@@ -126,9 +126,7 @@ int ifx_ops_attention_decode(const float* q, const void* k_cache, const void* v_
   IFX_TRY(decode_args(q, k_cache, v_cache, kv_type, max_seq, n_rows, n_heads, n_kv_heads, head_dim, &a));
   hipStream_t st = ops_stream(stream);
   CallScratch cs(st);
-  DevState* state;
-  IFX_TRY(put_state(cs, (uint32_t)(n_rows - 1), 0, &state));
-  a.state = state;
+  a.rows = (uint32_t)n_rows;
   a.out = out;
   a.one_chunk = n_rows <= a.chunk;
   if (!a.one_chunk) IFX_TRY(alloc_records(cs, &a));
@@ -150,9 +148,6 @@ int ifx_ops_attention_decode_o(const float* q, const void* k_cache, const void* 
                      (unsigned long long)w_o->L.cols, (unsigned long long)(n_heads * head_dim));
   hipStream_t st = ops_stream(stream);
   CallScratch cs(st);
-  DevState* state;
-  IFX_TRY(put_state(cs, (uint32_t)(n_rows - 1), 0, &state));
-  a.state = state;
   IFX_TRY(alloc_records(cs, &a));
   float* attn = attn_out;
   if (!attn) IFX_TRY(cs.alloc((void**)&attn, n_heads * head_dim * 4));
@@ -162,9 +157,13 @@ int ifx_ops_attention_decode_o(const float* q, const void* k_cache, const void* 
     if (!merge_o_supported(go, a))
       return set_error(IFX_E_INVALID_ARG, "the merge in the O projection needs 8 kv heads, head dim 128, 4 or 8 "
                                           "query heads per kv head and a K-split Q4_K/Q6_K W_o");
+    DevState* state;
+    IFX_TRY(put_state(cs, (uint32_t)(n_rows - 1), 0, &state));
+    a.state = state;
     IFX_HIP(launch_attn_partials(a, st));
     IFX_HIP(launch_mfma_residual_merge(go, a, h, st, merge_bound));
   } else {
+    a.rows = (uint32_t)n_rows;
     a.one_chunk = n_rows <= a.chunk;
     IFX_HIP(launch_attn_decode(a, st));
     IFX_HIP(gemv_residual(go, h, st));

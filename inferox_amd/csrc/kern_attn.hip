@@ -173,7 +173,13 @@ constexpr int kRowsPerWave = kChunk / (kThreads / 64);  // 16
 // Cache rows [lo, hi) the current token attends to.  The three fields are read
 // unconditionally, so that they come in one memory round trip (a conditional
 // read of len would be a second one).
-__device__ __forceinline__ void attended_rows(const DevState* st, uint32_t& lo, uint32_t& hi) {
+__device__ __forceinline__ void attended_rows(const AttnArgs& a, uint32_t& lo, uint32_t& hi) {
+  if (a.rows) {  // uniform
+    lo = 0;
+    hi = a.rows;
+    return;
+  }
+  const DevState* st = a.state;
   const uint32_t len = st->len, attn_lo = st->attn_lo, attn_end = st->attn_end;
   lo = attn_lo;
   hi = attn_end ? attn_end : len + 1;
@@ -213,7 +219,7 @@ __global__ void __launch_bounds__(kThreads, GT == 8 ? 3 : 1) k_attn_decode(AttnA
   const uint32_t G = GT > 0 ? (uint32_t)GT : a.n_heads / a.n_kv_heads;
   const uint32_t HD = HDT > 0 ? (uint32_t)HDT : a.head_dim, nc4 = HD / 4, nck = HD / EPC;
   uint32_t lo, hi;
-  attended_rows(a.state, lo, hi);
+  attended_rows(a, lo, hi);
   const uint32_t nrows = hi > lo ? hi - lo : 0;
   const uint32_t nch = (nrows + kChunk - 1) / kChunk;
   if (c >= nch) return;
@@ -435,7 +441,7 @@ __global__ void __launch_bounds__(kThreads) k_attn_merge(AttnArgs a) {
   const uint32_t HD = HDT > 0 ? (uint32_t)HDT : a.head_dim, nc4 = HD / 4 / CS;  // float4 columns of the slice
   const uint32_t h = blockIdx.x / CS, hk = h / G, g = h % G, cb = (blockIdx.x % CS) * nc4;
   uint32_t lo, hi;
-  attended_rows(a.state, lo, hi);
+  attended_rows(a, lo, hi);
   const uint32_t nrows = hi > lo ? hi - lo : 0;
   const uint32_t nch = (nrows + kChunk - 1) / kChunk;
   if (nch == 0) return;

@@ -300,6 +300,10 @@ struct AttnArgs {
   // the attended rows fit one chunk (the host's bound on them is at most
   // `chunk`): the chunk's workgroup writes the attention output itself
   uint32_t one_chunk = 0;
+  // non-zero: the rows [0, rows) attended are known to the host and state is
+  // not read (a kernel of its own to write it, and its read before the K/V
+  // loads, cost an operator call ~3 us)
+  uint32_t rows = 0;
 };
 hipError_t launch_attn_decode(const AttnArgs& a, hipStream_t st);
 // the chunk records only (their merge is left to launch_mfma_residual_merge)
