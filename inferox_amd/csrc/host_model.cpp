@@ -478,6 +478,14 @@ int run_step(ifx_session* s, uint64_t rows, bool head = true) {
   return enqueue_step(s);
 }
 
+// A copy that has ended on return, on the session's stream.  hipMemcpy, hipMemset
+// and hipDeviceSynchronize fail while any thread captures a stream, and end that
+// capture: a session's calls must leave the first steps of others alone.
+hipError_t copy_now(ifx_session* s, void* dst, const void* src, size_t n, hipMemcpyKind kind) {
+  const hipError_t e = hipMemcpyAsync(dst, src, n, kind, s->stream);
+  return e == hipSuccess ? hipStreamSynchronize(s->stream) : e;
+}
+
 int state_op(ifx_session* s, uint32_t kind, uint32_t value, uint32_t len) {
   StateOp op{kind, value, len};
   IFX_HIP(launch_state(s->state, op, s->stream));
@@ -783,10 +791,12 @@ int ifx_session_create_kv(ifx_model* m, uint64_t max_seq_len, int kv_type, ifx_s
   init.out_tokens = s->out_tokens;
   init.out_cap = (uint32_t)max_seq_len;
   init.top_p = 1.0f;
-  if (hipMemcpy(s->rope_cs, cs.data(), cs.size() * 8, hipMemcpyHostToDevice) != hipSuccess ||
-      hipMemcpy(s->state, &init, sizeof init, hipMemcpyHostToDevice) != hipSuccess ||
-      hipMemset(s->kc, 0, kv_bytes) != hipSuccess || hipMemset(s->vc, 0, kv_bytes) != hipSuccess ||
-      hipMemset(s->sample_ws, 0, sample_ws_bytes()) != hipSuccess || hipDeviceSynchronize() != hipSuccess) {
+  if (copy_now(s, s->rope_cs, cs.data(), cs.size() * 8, hipMemcpyHostToDevice) != hipSuccess ||
+      copy_now(s, s->state, &init, sizeof init, hipMemcpyHostToDevice) != hipSuccess ||
+      hipMemsetAsync(s->kc, 0, kv_bytes, s->stream) != hipSuccess ||
+      hipMemsetAsync(s->vc, 0, kv_bytes, s->stream) != hipSuccess ||
+      hipMemsetAsync(s->sample_ws, 0, sample_ws_bytes(), s->stream) != hipSuccess ||
+      hipStreamSynchronize(s->stream) != hipSuccess) {
     session_free(s);
     return set_error(IFX_E_HIP, "session initialisation failed");
   }
@@ -917,7 +927,7 @@ int ifx_decode_greedy(ifx_session* s, uint32_t token, uint64_t n_steps, uint32_t
   (void)hipEventElapsedTime(&s->last_ms, s->ev0, s->ev1);
   s->len += n_steps;
   if (n_steps == 0) return IFX_OK;
-  IFX_HIP(hipMemcpy(out_tokens, s->out_tokens + first, n_steps * 4, hipMemcpyDeviceToHost));
+  IFX_HIP(copy_now(s, out_tokens, s->out_tokens + first, n_steps * 4, hipMemcpyDeviceToHost));
   int rc = IFX_OK;
   for (uint64_t i = 0; i < n_steps; i++) {
     if (out_tokens[i] & 0x80000000u) rc = IFX_E_NAN_LOGIT;
@@ -948,7 +958,7 @@ int ifx_generate(ifx_session* s, const uint32_t* prompt, uint64_t n, uint64_t ma
   (void)hipEventElapsedTime(&s->last_ms, s->ev0, s->ev1);
   s->len += max_tokens;
   if (max_tokens == 0) return IFX_OK;
-  IFX_HIP(hipMemcpy(out_tokens, s->out_tokens + (n - 1), max_tokens * 4, hipMemcpyDeviceToHost));
+  IFX_HIP(copy_now(s, out_tokens, s->out_tokens + (n - 1), max_tokens * 4, hipMemcpyDeviceToHost));
   int rc = IFX_OK;
   for (uint64_t i = 0; i < max_tokens; i++) {
     if (out_tokens[i] & 0x80000000u) rc = IFX_E_NAN_LOGIT;
@@ -1086,7 +1096,7 @@ int ifx_kv_import(ifx_session* s, const float* k, const float* v, uint64_t len) 
         const float* src = (which ? v : k) + host;
         for (uint64_t t = 0; t < len; t++)
           for (uint64_t d = 0; d < hd; d++) blk[t * hd + d] = f32_to_f16(src[t * kvd + d]);
-        IFX_HIP(hipMemcpy((which ? s->vc : s->kc) + dev, blk.data(), len * hd * 2, hipMemcpyHostToDevice));
+        IFX_HIP(copy_now(s, (which ? s->vc : s->kc) + dev, blk.data(), len * hd * 2, hipMemcpyHostToDevice));
       }
     }
   IFX_TRY(state_op(s, STATE_RESET, 0, (uint32_t)len));
@@ -1108,17 +1118,18 @@ int ifx_kv_export(ifx_session* s, float* k, float* v, uint64_t len) {
     for (uint64_t h = 0; h < c.n_kv_heads; h++) {
       const uint64_t dev = (l * c.n_kv_heads + h) * s->max_seq * hd * es, host = l * len * kvd + h * hd;
       if (es == 4) {
-        IFX_HIP(hipMemcpy2D(k + host, kvd * 4, s->kc + dev, hd * 4, hd * 4, len, hipMemcpyDeviceToHost));
-        IFX_HIP(hipMemcpy2D(v + host, kvd * 4, s->vc + dev, hd * 4, hd * 4, len, hipMemcpyDeviceToHost));
+        IFX_HIP(hipMemcpy2DAsync(k + host, kvd * 4, s->kc + dev, hd * 4, hd * 4, len, hipMemcpyDeviceToHost, s->stream));
+        IFX_HIP(hipMemcpy2DAsync(v + host, kvd * 4, s->vc + dev, hd * 4, hd * 4, len, hipMemcpyDeviceToHost, s->stream));
         continue;
       }
       for (int which = 0; which < 2; which++) {
-        IFX_HIP(hipMemcpy(blk.data(), (which ? s->vc : s->kc) + dev, len * hd * 2, hipMemcpyDeviceToHost));
+        IFX_HIP(copy_now(s, blk.data(), (which ? s->vc : s->kc) + dev, len * hd * 2, hipMemcpyDeviceToHost));
         float* dst = (which ? v : k) + host;
         for (uint64_t t = 0; t < len; t++)
           for (uint64_t d = 0; d < hd; d++) dst[t * kvd + d] = f16_to_f32(blk[t * hd + d]);
       }
     }
+  IFX_HIP(hipStreamSynchronize(s->stream));
   return IFX_OK;
 }
 
@@ -1229,8 +1240,7 @@ int ifx_session_profile_ordered(ifx_session* s, uint32_t token, uint64_t n_steps
 
 int ifx_session_last_token(ifx_session* s, uint32_t* token) {
   if (!s || !token) return set_error(IFX_E_INVALID_ARG, "null argument");
-  IFX_HIP(hipStreamSynchronize(s->stream));
-  IFX_HIP(hipMemcpy(token, &s->state->cur_token, 4, hipMemcpyDeviceToHost));
+  IFX_HIP(copy_now(s, token, &s->state->cur_token, 4, hipMemcpyDeviceToHost));
   return IFX_OK;
 }
 
