@@ -62,6 +62,8 @@ constexpr int kThreads = 512;
 constexpr int kAPlane = kBM * kLdk, kWPlane = kBN * kLdk;  // halves in one 128 (256) x 32 plane
 constexpr uint32_t kMagic = 0x64006400u;  // fp16 1024 in both halves: 0x6400 | u is 1024 + u (u < 1024)
 
+constexpr uint32_t kTargetWgs = 256;  // workgroups at once: one per CU
+
 struct GemmArgs {
   const uint16_t* ahi;   // [m][k] fp16, chunk order 0 4 1 5 2 6 3 7
   const uint16_t* alo;
@@ -70,9 +72,14 @@ struct GemmArgs {
   uint32_t m, k;         // k = cols of the weight matrix, a multiple of 32
   GemmW w0, w1;          // w1: the second matrix of a paired launch (gate/up)
   uint32_t n;            // output columns: rows of w0 (paired: of each)
-  uint32_t ksplit;       // K ranges over grid.z; > 1: partial tiles to `part`
+  uint32_t nx, tiles;    // column tiles; all tiles
+  uint32_t full;         // tiles [0, full) run whole, the others as ksplit K ranges (if any)
+  uint32_t rounds;       // both kinds in one launch: full / 256, else 0
+  bool half;             // tiles of at most 64 tokens run as half a tile
+  uint32_t ksplit;       // > 1: partial tiles to `part`
   uint32_t kps;          // 32-wide K steps per range (a multiple of the block's steps)
-  float* part;           // [ksplit][m][ncols], ncols = n (paired: 2n, up after gate)
+  uint32_t mbase, ncols; // first row of tile `full`; n (paired: 2n, up after gate)
+  float* part;           // [ksplit][m - mbase][ncols]
 };
 
 __device__ __forceinline__ h2 as_h2(uint32_t v) { return __builtin_bit_cast(h2, v); }
@@ -369,26 +376,40 @@ struct EpTraits<EpRope> {
   static constexpr bool kPaired = false, kNeighbor = true;
 };
 
-template <int T, class Ep>
-__global__ void __launch_bounds__(kThreads, 1) k_gemm(GemmArgs a, Ep ep) {
+// The LDS of a workgroup: arrays of their own rather than one struct's, so that
+// the writes of one can move past the reads of another.
+template <int T>
+struct GemmLds {
+  static constexpr int kNw = WQ<T>::kPLo ? 2 : 1;  // weight planes: p (hi), [p lo]
+  _Float16 (&la)[2][2][kAPlane];                   // [buffer][A hi, A lo]
+  _Float16 (&lw)[2][kNw][kWPlane];                 // [buffer][p hi, p lo]
+  typename WQ<T>::Side (&side)[2];
+  int (&rexp)[kBM];
+};
+
+// K steps [ks0, ks1) (whole scale blocks) of one tile of 32 MI tokens (from m0)
+// by 256 weight rows (from the tile's first output column n0): MI = 4, or 2 for
+// half a tile.  Through the epilogue, or (part) to the range's partial rows.
+template <int T, class Ep, int MI>
+__device__ __forceinline__ void gemm_tile(const GemmArgs& a, const Ep& ep, const GemmLds<T>& lds, uint32_t m0, uint32_t n0,
+                                          uint32_t ks0, uint32_t ks1, float* part) {
   using Q = WQ<T>;
   constexpr bool kPaired = EpTraits<Ep>::kPaired;
-  constexpr int kNw = Q::kPLo ? 2 : 1;  // weight planes: p (hi), [p lo]
-  __shared__ __attribute__((aligned(16))) _Float16 la[2][2][kAPlane];    // [buffer][A hi, A lo]
-  __shared__ __attribute__((aligned(16))) _Float16 lw[2][kNw][kWPlane];  // [buffer][p hi, p lo]
-  __shared__ __attribute__((aligned(16))) typename Q::Side side[2];
-  __shared__ int rexp[kBM];
+  constexpr int kNw = GemmLds<T>::kNw;
+  auto& la = lds.la;
+  auto& lw = lds.lw;
+  auto& side = lds.side;
+  auto& rexp = lds.rexp;
   // the wave index as a scalar: the wave's fragment rows and columns are
   // uniform over it and stay out of the vector registers
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 2, wn = wave & 3;
-  const uint32_t m0 = blockIdx.y * kBM;
-  // output columns of the tile (paired: gate rows n0.. in W rows 0..127, up in 128..255)
-  const uint32_t n0 = blockIdx.x * (kPaired ? kBN / 2 : kBN);
+  // (output columns of a paired tile: gate rows n0.. in W rows 0..127, up in 128..255)
 
   // staging roles: A row ar chunk ac (both planes), W row wr half h.
   // Rows past the operands read a clamped row: their outputs are never stored.
-  const int h = tid & 1, wr = tid >> 1, ar = tid >> 2, ac = tid & 3;
+  // (half a tile: the second half of the threads repeats the first's A loads)
+  const int h = tid & 1, wr = tid >> 1, ar = (tid >> 2) & (32 * MI - 1), ac = tid & 3;
   const uint32_t at = min(m0 + (uint32_t)ar, a.m - 1);
   const GemmW& ws = (kPaired && wr >= kBN / 2) ? a.w1 : a.w0;
   const uint32_t w_rows_avail = (T == T_Q4K || T == T_Q6K) ? (ws.rows + 15u) & ~15u : ws.rows;
@@ -424,9 +445,9 @@ __global__ void __launch_bounds__(kThreads, 1) k_gemm(GemmArgs a, Ep ep) {
     rw.stage(lw[buf][0], Q::kPLo ? lw[buf][kNw - 1] : nullptr, side[sbi], g, wr, h, sb0);
   };
 
-  f4 acc[4][4], cs[4][4];
+  f4 acc[MI][4], cs[MI][4];
 #pragma unroll
-  for (int i = 0; i < 4; i++)
+  for (int i = 0; i < MI; i++)
 #pragma unroll
     for (int j = 0; j < 4; j++) {
       acc[i][j] = f4{0.f, 0.f, 0.f, 0.f};
@@ -450,8 +471,8 @@ __global__ void __launch_bounds__(kThreads, 1) k_gemm(GemmArgs a, Ep ep) {
       if (Q::kPLo) bl[j] = *(const h8*)&lw[buf][kNw - 1][swz(wcol[j] + fi, fg)];
     }
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const int r = wm * 64 + 16 * i + fi;
+    for (int i = 0; i < MI; i++) {
+      const int r = wm * (16 * MI) + 16 * i + fi;
       const h8 ah = *(const h8*)&la[buf][0][swz(r, fg)];
       const h8 al = *(const h8*)&la[buf][1][swz(r, fg)];
 #pragma unroll
@@ -475,7 +496,7 @@ __global__ void __launch_bounds__(kThreads, 1) k_gemm(GemmArgs a, Ep ep) {
 #pragma unroll
     for (int j = 0; j < 4; j++) dj[j] = sd.d[wcol[j] + fi];
 #pragma unroll
-    for (int i = 0; i < 4; i++)
+    for (int i = 0; i < MI; i++)
 #pragma unroll
       for (int j = 0; j < 4; j++)
 #pragma unroll
@@ -487,10 +508,10 @@ __global__ void __launch_bounds__(kThreads, 1) k_gemm(GemmArgs a, Ep ep) {
       // against b1 b2 in each lane's 8 k slots: the same sum of products), at
       // the cost of one K = 16 one on gfx950.
       const h4 z = {0, 0, 0, 0};
-      h4 a1[4], a2[4], b1[4], b2[4];
+      h4 a1[MI], a2[MI], b1[4], b2[4];
 #pragma unroll
-      for (int i = 0; i < 4; i++) {
-        a1[i] = *(const h4*)&sd.sa[wm * 64 + 16 * i + fi][4 * fg];
+      for (int i = 0; i < MI; i++) {
+        a1[i] = *(const h4*)&sd.sa[wm * (16 * MI) + 16 * i + fi][4 * fg];
         a2[i] = fg < 2 ? a1[i] : z;
       }
 #pragma unroll
@@ -500,7 +521,7 @@ __global__ void __launch_bounds__(kThreads, 1) k_gemm(GemmArgs a, Ep ep) {
         b2[j] = fg < 2 ? lo : z;
       }
 #pragma unroll
-      for (int i = 0; i < 4; i++)
+      for (int i = 0; i < MI; i++)
 #pragma unroll
         for (int j = 0; j < 4; j++) {
           const h8 a = __builtin_shufflevector(a1[i], a2[i], 0, 1, 2, 3, 4, 5, 6, 7);
@@ -515,7 +536,6 @@ __global__ void __launch_bounds__(kThreads, 1) k_gemm(GemmArgs a, Ep ep) {
   // (its last readers finished before the previous barrier), then issues the
   // raw loads of step ks + 2: one barrier per step, and a whole block of
   // steps unrolled so that the MFMAs and the unpacking interleave.
-  const uint32_t ks0 = blockIdx.z * a.kps, ks1 = min(a.k / kBK, ks0 + a.kps);
   const uint32_t klast = ks1 - 1;  // loads past the range re-read its last step (unused)
   __syncthreads();  // rexp
   load_step(ks0, 0, true);
@@ -544,15 +564,14 @@ __global__ void __launch_bounds__(kThreads, 1) k_gemm(GemmArgs a, Ep ep) {
 
   // epilogue: C[4 fg + r][fi] of fragment (i, j)
 #pragma unroll
-  for (int i = 0; i < 4; i++) {
+  for (int i = 0; i < MI; i++) {
 #pragma unroll
     for (int r = 0; r < 4; r++) {
-      const int tl = wm * 64 + 16 * i + 4 * fg + r;
+      const int tl = wm * (16 * MI) + 16 * i + 4 * fg + r;
       const uint32_t t = m0 + (uint32_t)tl;
       const float inv = ldexpf(1.0f, rexp[tl] - 14);
-      if (a.ksplit > 1) {  // partial tile of this K range; the reduce applies the epilogue
-        const uint32_t ncols = kPaired ? 2 * a.n : a.n;
-        float* pr = a.part + ((uint64_t)blockIdx.z * a.m + t) * ncols;
+      if (part) {  // partial tile of this K range; the reduce applies the epilogue
+        float* pr = part + (uint64_t)(t - a.mbase) * a.ncols;
 #pragma unroll
         for (int j = 0; j < 4; j++) {
           uint32_t n, col;
@@ -587,17 +606,51 @@ __global__ void __launch_bounds__(kThreads, 1) k_gemm(GemmArgs a, Ep ep) {
   }
 }
 
+// Tiles in order, columns fastest.  Tiles [0, a.full) run whole; each later
+// one is a.ksplit workgroups, a K range each, whose partial tiles the reduce
+// adds.  A tile with at most 64 tokens in the chunk runs as half a tile (Q6_K
+// 4096 x 14336 of 129 tokens 105 -> 97 us, Q4_K 14336 x 4096 of 300 131 -> 126)
+// where it has 32 steps or more: below, the second body's instructions cost
+// more than its products (a 512-wide MLP of 433 tokens 76.0 -> 78.2).
+template <int T, class Ep>
+__global__ void __launch_bounds__(kThreads, 1) k_gemm(GemmArgs a, Ep ep) {
+  __shared__ __attribute__((aligned(16))) _Float16 la[2][2][kAPlane];
+  __shared__ __attribute__((aligned(16))) _Float16 lw[2][GemmLds<T>::kNw][kWPlane];
+  __shared__ __attribute__((aligned(16))) typename WQ<T>::Side side[2];
+  __shared__ int rexp[kBM];
+  const GemmLds<T> lds{la, lw, side, rexp};
+  uint32_t tx = blockIdx.x, ty = blockIdx.y, z = blockIdx.z;
+  bool whole = a.ksplit == 1;
+  if (a.rounds) {  // whole rounds, then ranges: 256 tiles per blockIdx.y
+    whole = ty < a.rounds;
+    z = whole ? 0u : ty - a.rounds;
+    const uint32_t tile = (whole ? ty * kTargetWgs : a.full) + tx;
+    if (tile >= a.tiles) return;
+    ty = tile / a.nx;
+    tx = tile - ty * a.nx;
+  }
+  const uint32_t m0 = ty * kBM, n0 = tx * (EpTraits<Ep>::kPaired ? kBN / 2 : kBN);
+  const uint32_t ks0 = whole ? 0u : z * a.kps, ks1 = whole ? a.k / kBK : min(a.k / kBK, ks0 + a.kps);
+  float* part = whole ? nullptr : a.part + (uint64_t)z * (a.m - a.mbase) * a.ncols;
+  if (!a.half || a.m - m0 > kBM / 2) gemm_tile<T, Ep, 4>(a, ep, lds, m0, n0, ks0, ks1, part);
+  else gemm_tile<T, Ep, 2>(a, ep, lds, m0, n0, ks0, ks1, part);
+}
+
 // Sum of the K-range partials of output (t, n) in range order, then the
 // epilogue: partner = column n ^ 1 (RoPE) or the up value of n (paired).
+// A row per blockIdx.y; outputs of the whole tiles are skipped.
 template <class Ep>
-__global__ void k_gemm_reduce(GemmArgs a, Ep ep) {
-  const uint64_t idx = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= (uint64_t)a.m * a.n) return;
-  const uint32_t t = (uint32_t)(idx / a.n), n = (uint32_t)(idx % a.n);
-  const uint32_t ncols = EpTraits<Ep>::kPaired ? 2 * a.n : a.n;
+__device__ __forceinline__ bool in_ranges(const GemmArgs& a, uint32_t t, uint32_t n) {
+  return t / kBM * a.nx + n / (EpTraits<Ep>::kPaired ? kBN / 2 : kBN) >= a.full;
+}
+template <class Ep>
+__global__ void __launch_bounds__(256) k_gemm_reduce(GemmArgs a, Ep ep) {
+  const uint32_t t = a.mbase + blockIdx.y, n = blockIdx.x * blockDim.x + threadIdx.x;
+  if (n >= a.n || !in_ranges<Ep>(a, t, n)) return;
+  const float* pr = a.part + (uint64_t)blockIdx.y * a.ncols;
+  const uint64_t range = (uint64_t)(a.m - a.mbase) * a.ncols;
   float v = 0.f, partner = 0.f;
-  for (uint32_t z = 0; z < a.ksplit; z++) {
-    const float* pr = a.part + ((uint64_t)z * a.m + t) * ncols;
+  for (uint32_t z = 0; z < a.ksplit; z++, pr += range) {
     v += pr[n];
     if (EpTraits<Ep>::kPaired) partner += pr[n + a.n];
     else if (EpTraits<Ep>::kNeighbor && (n ^ 1u) < a.n) partner += pr[n ^ 1u];
@@ -605,23 +658,22 @@ __global__ void k_gemm_reduce(GemmArgs a, Ep ep) {
   ep(t, n, v, partner);
 }
 
-// The same sums four outputs (t, 4i .. 4i + 3) per thread, as 16-byte loads
-// (n % 4 == 0): each output's partials are added in the same order, so the
+// The same sums four outputs (t, n .. n + 3) per thread, as 16-byte loads
+// (a.n % 4 == 0): each output's partials are added in the same order, so the
 // bits are those of k_gemm_reduce.  The RoPE partner n ^ 1 is in the same four.
 template <class Ep>
-__global__ void k_gemm_reduce4(GemmArgs a, Ep ep) {
-  const uint32_t n4 = a.n / 4;
-  const uint64_t idx = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= (uint64_t)a.m * n4) return;
-  const uint32_t t = (uint32_t)(idx / n4), n = 4 * (uint32_t)(idx % n4);
-  const uint32_t ncols = EpTraits<Ep>::kPaired ? 2 * a.n : a.n;
+__global__ void __launch_bounds__(256) k_gemm_reduce4(GemmArgs a, Ep ep) {
+  const uint32_t t = a.mbase + blockIdx.y, n = 4 * (blockIdx.x * blockDim.x + threadIdx.x);
+  if (n >= a.n || !in_ranges<Ep>(a, t, n)) return;
+  const float* pr = a.part + (uint64_t)blockIdx.y * a.ncols + n;
+  const uint64_t range = (uint64_t)(a.m - a.mbase) * a.ncols;
   float4 v = make_float4(0.f, 0.f, 0.f, 0.f), u = v;
-  for (uint32_t z = 0; z < a.ksplit; z++) {
-    const float* pr = a.part + ((uint64_t)z * a.m + t) * ncols;
-    const float4 x = *(const float4*)(pr + n);
+#pragma unroll 4
+  for (uint32_t z = 0; z < a.ksplit; z++, pr += range) {
+    const float4 x = *(const float4*)pr;
     v.x += x.x; v.y += x.y; v.z += x.z; v.w += x.w;
     if (EpTraits<Ep>::kPaired) {
-      const float4 y = *(const float4*)(pr + n + a.n);
+      const float4 y = *(const float4*)(pr + a.n);
       u.x += y.x; u.y += y.y; u.z += y.z; u.w += y.w;
     }
   }
@@ -634,17 +686,15 @@ __global__ void k_gemm_reduce4(GemmArgs a, Ep ep) {
 
 template <int T, class Ep>
 hipError_t go(const GemmArgs& a, const Ep& ep, hipStream_t st) {
-  const uint32_t bn = EpTraits<Ep>::kPaired ? kBN / 2 : kBN;
-  dim3 grid((a.n + bn - 1) / bn, (a.m + kBM - 1) / kBM, a.ksplit);
+  const dim3 grid = a.rounds ? dim3(kTargetWgs, a.rounds + a.ksplit) : dim3(a.nx, a.tiles / a.nx, a.ksplit);
   hipLaunchKernelGGL((k_gemm<T, Ep>), grid, dim3(kThreads), 0, st, a, ep);
   if (a.ksplit > 1) {
-    if (a.n % 4 == 0) {
-      const uint64_t total = (uint64_t)a.m * (a.n / 4);
-      hipLaunchKernelGGL((k_gemm_reduce4<Ep>), dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, a, ep);
-    } else {
-      const uint64_t total = (uint64_t)a.m * a.n;
-      hipLaunchKernelGGL((k_gemm_reduce<Ep>), dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, a, ep);
-    }
+    const bool by4 = a.n % 4 == 0;
+    // the fewest workgroups per row, of waves as even as they come
+    const uint32_t each = by4 ? a.n / 4 : a.n, nwg = (each + 255) / 256;
+    const dim3 rows(nwg, a.m - a.mbase), threads((each + 64 * nwg - 1) / (64 * nwg) * 64);
+    if (by4) hipLaunchKernelGGL((k_gemm_reduce4<Ep>), rows, threads, 0, st, a, ep);
+    else hipLaunchKernelGGL((k_gemm_reduce<Ep>), rows, threads, 0, st, a, ep);
   }
   return hipGetLastError();
 }
@@ -670,9 +720,18 @@ hipError_t dispatch(const GemmArgs& a, const Ep& ep, hipStream_t st) {
   }
 }
 
-// Tiles of fewer than one workgroup per CU split K over grid.z (at least 8
-// steps per range), as far as the partial buffer holds them.
-constexpr uint32_t kTargetWgs = 256, kMinStepsPerSplit = 8;
+// How a launch's tiles meet the CUs (one workgroup each).  Rounds of whole
+// tiles leave CUs idle in the last one, or in the only one; those tiles can be
+// cut into K ranges of at least 8 steps, as far as the partial buffer holds
+// them.  The plan with the least estimated time is taken, in K steps (~0.95
+// us): rounds of steps and ~8 steps' worth of prologue and epilogue, then for
+// ranges the reduce launch (~4 us, and the partial tiles written and read at
+// ~4.5 TB/s).  Against ranges only for fewer than 256 tiles, and as many of
+// them as pass 256 workgroups: Q4_K 14336 x 4096 of 129 tokens 93.1 -> 75.0 us
+// (112 tiles ran as 336 workgroups, two rounds), of 512 168.0 -> 147.8 and of
+// 2048 503 -> 485 (a last round of 192 tiles); Q8_0 of 100 tokens 78.4 -> 58.9;
+// Q6_K 4096 x 14336 of 300 tokens 191.5 -> 155.1.
+constexpr uint32_t kMinStepsPerSplit = 8, kMinHalfSteps = 32, kMaxReduceRows = 65535;  // rows of the reduce: its grid's y
 
 GemmArgs args_of(const GemmIn& in, const GemmW& w, bool paired) {
   GemmArgs a{};
@@ -688,15 +747,37 @@ GemmArgs args_of(const GemmIn& in, const GemmW& w, bool paired) {
   const uint32_t nk = a.k / kBK, bn = paired ? kBN / 2 : kBN;
   const uint32_t sb = (w.type == T_Q4K || w.type == T_Q6K) ? 8u : 1u;  // steps per scale block
   const uint64_t tiles = (uint64_t)((a.n + bn - 1) / bn) * ((a.m + kBM - 1) / kBM);
-  uint32_t split = 1;
-  if (in.part && tiles < kTargetWgs) {
-    split = (uint32_t)std::min<uint64_t>((kTargetWgs + tiles - 1) / tiles, std::max<uint32_t>(1, nk / kMinStepsPerSplit));
-    const uint64_t per = (uint64_t)a.m * a.n * (paired ? 2 : 1) * 4;
-    split = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>({split, in.part_bytes / per, 64}));
+  a.nx = (a.n + bn - 1) / bn;
+  a.tiles = a.full = (uint32_t)tiles;
+  a.ncols = a.n * (paired ? 2 : 1);
+  a.kps = (nk + sb - 1) / sb * sb;  // ranges of whole scale blocks
+  a.ksplit = 1;
+  a.mbase = 0;
+  a.half = a.kps >= kMinHalfSteps;
+  if (!in.part || !a.ncols || !a.m) return a;
+  auto rounds = [](uint64_t wgs) { return (double)((wgs + kTargetWgs - 1) / kTargetWgs); };
+  double best = rounds(tiles) * (nk + 8.0);
+  // all tiles in ranges, or those past the last whole round
+  const uint64_t whole = tiles / kTargetWgs * kTargetWgs;
+  for (uint64_t full = 0; full < tiles; full += whole) {
+    const uint64_t mbase = full / a.nx * kBM, per = (a.m - mbase) * a.ncols * 4, rest = tiles - full;
+    const uint64_t most = a.m - mbase > kMaxReduceRows ? 0 : std::min<uint64_t>({nk / kMinStepsPerSplit, in.part_bytes / per, 64});
+    for (uint32_t s = 2; s <= most; s++) {
+      const uint32_t kps = ((nk + s - 1) / s + sb - 1) / sb * sb, ranges = (nk + kps - 1) / kps;
+      const double bytes = 2.0 * ranges * (double)rest * (kBM * kBN * 4);
+      const double c = rounds(full) * (nk + 8.0) + rounds(rest * ranges) * (kps + 8.0) + 4.0 + bytes / 4.5e6;
+      if (ranges > 1 && c < best) {
+        best = c;
+        a.full = (uint32_t)full;
+        a.kps = kps;
+        a.ksplit = ranges;
+        a.mbase = (uint32_t)mbase;
+      }
+    }
+    if (whole == 0) break;
   }
-  a.kps = (nk + split - 1) / split;
-  a.kps = (a.kps + sb - 1) / sb * sb;  // ranges of whole scale blocks
-  a.ksplit = (nk + a.kps - 1) / a.kps;
+  a.rounds = a.full < a.tiles ? a.full / kTargetWgs : 0;
+  a.half = a.kps >= kMinHalfSteps;
   a.part = a.ksplit > 1 ? in.part : nullptr;
   return a;
 }
@@ -920,7 +1001,7 @@ uint64_t gemm_store_part_bytes(uint32_t m, const GemmW& w, uint64_t limit) {
   in.part_bytes = limit;
   if (m == 0 || w.rows == 0) return 0;
   const GemmArgs a = args_of(in, w, false);
-  return a.ksplit > 1 ? (uint64_t)a.ksplit * a.m * a.n * 4 : 0;
+  return a.ksplit > 1 ? (uint64_t)a.ksplit * (a.m - a.mbase) * a.ncols * 4 : 0;
 }
 
 hipError_t gemm_store(const GemmIn& in, const GemmW& w, float* y, uint32_t ldy, hipStream_t st) {
