@@ -7,7 +7,10 @@
 //
 // Arithmetic as in kern_gemm.hip: both products run on the fp16 matrix cores
 // with each operand an fp16 hi/lo pair (three MFMAs per step, f32
-// accumulation), within the rounding of the f32 reference.  The fp16 range is
+// accumulation), within the rounding of the f32 reference.  An element of a
+// binary16 cache times its power of two is one fp16 value: its lo part is zero
+// and neither stored nor read, and two MFMAs give the same bits (32 heads of
+// 128 over 2048 rows 147 -> 113 us, 300 rows 39.4 -> 32.8).  The fp16 range is
 // kept by power-of-2 scales: per query row and per key row for q . k (undone
 // per score), and one per 64-key V block.  The V block scales are folded into
 // the softmax weights against a running reference exponent (the weights of a
@@ -177,7 +180,7 @@ __global__ void __launch_bounds__(kPrepThreads) k_kv_prep(AttnPrefillArgs a, Pre
       }
       const int ch = qq * CPT + i;
       *(h8*)(w.kh + row + 8 * ch) = hi;
-      *(h8*)(w.kl + row + 8 * ch) = lo;
+      if (sizeof(E) == 4) *(h8*)(w.kl + row + 8 * ch) = lo;
     }
   }
 
@@ -214,21 +217,24 @@ __global__ void __launch_bounds__(kPrepThreads) k_kv_prep(AttnPrefillArgs a, Pre
     }
     const uint64_t off = (((uint64_t)hk * nkb + b) * HP + d) * kKB + 8 * c;
     *(h8*)(w.vh + off) = hi;
-    *(h8*)(w.vl + off) = lo;
+    if (sizeof(E) == 4) *(h8*)(w.vl + off) = lo;
   }
 }
 
 // ---------------------------------------------------------------------------
 // Attention: grid 1-D over (query block, head), heaviest query blocks first.
 // ---------------------------------------------------------------------------
-template <int HD>
+// LO: K and V have lo planes (an f32 cache).
+template <int HD, bool LO>
 __global__ void __launch_bounds__(kThreads, 1) k_attn_prefill(AttnPrefillArgs a, PrepWs w) {
   using D = Dims<HD>;
   constexpr int HP = D::HP, NCH = D::NCH, NKS = D::NKS, NT = D::NT;
-  constexpr int UK = kKB * NCH * 2 / kThreads;  // K chunks per thread (both planes)
-  constexpr int UV = HP * 8 * 2 / kThreads;     // V^T chunks per thread
-  __shared__ __attribute__((aligned(16))) _Float16 Kh[kKB * HP], Kl[kKB * HP];
-  __shared__ __attribute__((aligned(16))) _Float16 Vh[HP * kKB], Vl[HP * kKB];
+  constexpr int NP = LO ? 2 : 1;  // planes
+  constexpr int UK = (kKB * NCH * NP + kThreads - 1) / kThreads;  // K chunks per thread (every plane)
+  constexpr int UV = (HP * 8 * NP + kThreads - 1) / kThreads;     // V^T chunks per thread
+  constexpr bool kWhole = kKB * NCH * NP % kThreads == 0;         // every thread has UK of them (and UV: as many)
+  __shared__ __attribute__((aligned(16))) _Float16 Kh[kKB * HP], Kl[LO ? kKB * HP : 8];
+  __shared__ __attribute__((aligned(16))) _Float16 Vh[HP * kKB], Vl[LO ? HP * kKB : 8];
   __shared__ __attribute__((aligned(16))) float kfac_s[kKB];  // per key of the block: 2^(e_k - 14) log2(e) / sqrt(hd)
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -288,7 +294,7 @@ __global__ void __launch_bounds__(kThreads, 1) k_attn_prefill(AttnPrefillArgs a,
 #pragma unroll
     for (int u = 0; u < UK; u++) {
       const int c = tid + kThreads * u, pl = c / (kKB * NCH), rem = c % (kKB * NCH);
-      rk[u] = *(const u4*)((pl ? w.kl : w.kh) + kbase + (uint64_t)rem * 8);
+      if (kWhole || pl < NP) rk[u] = *(const u4*)((pl ? w.kl : w.kh) + kbase + (uint64_t)rem * 8);
     }
     if (tid < kKB) rke = w.kexp[(uint64_t)hk * npad + kb * kKB + tid];
   };
@@ -297,7 +303,7 @@ __global__ void __launch_bounds__(kThreads, 1) k_attn_prefill(AttnPrefillArgs a,
 #pragma unroll
     for (int u = 0; u < UV; u++) {
       const int c = tid + kThreads * u, pl = c / (HP * 8), rem = c % (HP * 8);
-      rv[u] = *(const u4*)((pl ? w.vl : w.vh) + vbase + (uint64_t)rem * 8);
+      if (kWhole || pl < NP) rv[u] = *(const u4*)((pl ? w.vl : w.vh) + vbase + (uint64_t)rem * 8);
     }
     rve = w.vexp[(uint64_t)hk * nkb_all + kb];
   };
@@ -305,12 +311,12 @@ __global__ void __launch_bounds__(kThreads, 1) k_attn_prefill(AttnPrefillArgs a,
 #pragma unroll
     for (int u = 0; u < UK; u++) {
       const int c = tid + kThreads * u, pl = c / (kKB * NCH), rem = c % (kKB * NCH);
-      *(u4*)((pl ? Kl : Kh) + swz<HP>(rem / NCH, rem % NCH)) = rk[u];
+      if (kWhole || pl < NP) *(u4*)((pl ? Kl : Kh) + swz<HP>(rem / NCH, rem % NCH)) = rk[u];
     }
 #pragma unroll
     for (int u = 0; u < UV; u++) {
       const int c = tid + kThreads * u, pl = c / (HP * 8), rem = c % (HP * 8);
-      *(u4*)((pl ? Vl : Vh) + swzv(rem >> 3, rem & 7)) = rv[u];
+      if (kWhole || pl < NP) *(u4*)((pl ? Vl : Vh) + swzv(rem >> 3, rem & 7)) = rv[u];
     }
     if (tid < kKB) kfac_s[tid] = ldexpf(kc, rke - 14);
   };
@@ -344,10 +350,12 @@ __global__ void __launch_bounds__(kThreads, 1) k_attn_prefill(AttnPrefillArgs a,
 #pragma unroll
       for (int j = 0; j < 4; j++) {
         const h8 kh8 = *(const h8*)&Kh[swz<HP>(16 * j + fi, 4 * ks + fg)];
-        const h8 kl8 = *(const h8*)&Kl[swz<HP>(16 * j + fi, 4 * ks + fg)];
         s[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh8, qh[ks], s[j], 0, 0, 0);
         s[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh8, ql[ks], s[j], 0, 0, 0);
-        s[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kl8, qh[ks], s[j], 0, 0, 0);
+        if constexpr (LO) {
+          const h8 kl8 = *(const h8*)&Kl[swz<HP>(16 * j + fi, 4 * ks + fg)];
+          s[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kl8, qh[ks], s[j], 0, 0, 0);
+        }
       }
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -425,13 +433,15 @@ __global__ void __launch_bounds__(kThreads, 1) k_attn_prefill(AttnPrefillArgs a,
         const int vr = 16 * t + fi;
         const h4 vha = *(const h4*)&Vh[swzv(vr, va >> 3) + (va & 7)];
         const h4 vhb = *(const h4*)&Vh[swzv(vr, vb >> 3) + (vb & 7)];
-        const h4 vla = *(const h4*)&Vl[swzv(vr, va >> 3) + (va & 7)];
-        const h4 vlb = *(const h4*)&Vl[swzv(vr, vb >> 3) + (vb & 7)];
         const h8 vh8 = __builtin_shufflevector(vha, vhb, 0, 1, 2, 3, 4, 5, 6, 7);
-        const h8 vl8 = __builtin_shufflevector(vla, vlb, 0, 1, 2, 3, 4, 5, 6, 7);
         o[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh8, p8h, o[t], 0, 0, 0);
         o[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh8, p8l, o[t], 0, 0, 0);
-        o[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vl8, p8h, o[t], 0, 0, 0);
+        if constexpr (LO) {
+          const h4 vla = *(const h4*)&Vl[swzv(vr, va >> 3) + (va & 7)];
+          const h4 vlb = *(const h4*)&Vl[swzv(vr, vb >> 3) + (vb & 7)];
+          const h8 vl8 = __builtin_shufflevector(vla, vlb, 0, 1, 2, 3, 4, 5, 6, 7);
+          o[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vl8, p8h, o[t], 0, 0, 0);
+        }
         if (t % 4 == 3) __builtin_amdgcn_sched_barrier(0);  // V fragments of four tiles live at once
       }
     }
@@ -456,7 +466,8 @@ hipError_t go(const AttnPrefillArgs& a, hipStream_t st) {
   if (a.kv_f16) hipLaunchKernelGGL((k_kv_prep<HD, _Float16>), dim3(nkb, a.n_kv_heads), dim3(kPrepThreads), 0, st, a, w);
   else hipLaunchKernelGGL((k_kv_prep<HD, float>), dim3(nkb, a.n_kv_heads), dim3(kPrepThreads), 0, st, a, w);
   const dim3 grid(((a.n + kQ - 1) / kQ) * a.n_heads);
-  hipLaunchKernelGGL(k_attn_prefill<HD>, grid, dim3(kThreads), 0, st, a, w);
+  if (a.kv_f16) hipLaunchKernelGGL((k_attn_prefill<HD, false>), grid, dim3(kThreads), 0, st, a, w);
+  else hipLaunchKernelGGL((k_attn_prefill<HD, true>), grid, dim3(kThreads), 0, st, a, w);
   return hipGetLastError();
 }
 
