@@ -20,9 +20,10 @@
 //
 // Two launches per layer:
 //   * k_kv_prep: one workgroup per (64-key block, kv head) splits the chunk's
-//     K rows (row scale) and its V block, transposed (block scale), into fp16
-//     hi/lo planes in the workspace, once for all the query heads and query
-//     blocks that read them.
+//     K rows (row scale), and another its V block, transposed (block scale),
+//     into fp16 hi/lo planes in the workspace, once for all the query heads and
+//     query blocks that read them.  Bound by latency: the V block's loads all go
+//     out together.
 //   * k_attn_prefill: a workgroup of 8 waves owns 128 query rows of one head,
 //     wave w rows 16w .. 16w + 15 with their q scale and fp16 pairs in
 //     registers.  Per 64-key block it copies K and V^T into LDS (the next
@@ -34,7 +35,11 @@
 //     already holds (V^T's columns read in that order), so the softmax
 //     weights never leave registers, and the row max and sum take two
 //     shuffles.  64 KB of LDS and one workgroup per CU (two waves per SIMD):
-//     each staged block serves 128 queries.
+//     each staged block serves 128 queries.  Per block of keys the LDS reads,
+//     the matrix products and the softmax take about 1.7, 1.3 and 0.8 us of the
+//     4.2 measured: they hardly overlap.  Copies straight to LDS in two buffers
+//     (159 us for 32 heads of 128 over 2048 rows, against 148), and workgroups
+//     of four waves with 32 queries each, two per CU (160), were slower.
 // MFMA lane layout (16x16x32): lane i + 16g holds A[i][8g..8g+7] and
 // B[8g..8g+7][i], and receives C[4g + r][i] in register r.
 #include "kernels.h"
@@ -48,7 +53,14 @@ typedef _Float16 h4 __attribute__((ext_vector_type(4)));
 typedef float f4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u4 __attribute__((ext_vector_type(4)));  // a native vector: stays in registers
 
-constexpr int kQ = 128, kKB = 64, kThreads = 512, kPrepThreads = 256;
+constexpr int kKB = 64, kThreads = 512, kPrepThreads = 256;
+// Workgroups of 128 queries that fill the chip.  Fewer leave CUs idle while
+// each walks its key blocks one after the other: twice as many workgroups of 64
+// queries, with half of a block per wave, shorten that walk (with the prep's
+// two halves, 32 heads of 128: 300 rows 40.0 -> 33.5 us, 512 rows 53.1 -> 41.7;
+// 6 heads of 48 over 2048 rows 87.6 -> 64.0).  From 256 on they would only
+// stage each block twice as often.
+constexpr uint32_t kFull = 256;
 
 __device__ __forceinline__ int exp_of(uint32_t bits) {
   const int e = (int)((bits >> 23) & 255u) - 127;
@@ -148,8 +160,8 @@ __global__ void __launch_bounds__(kPrepThreads) k_kv_prep(AttnPrefillArgs a, Pre
   const E* kbase = (const E*)a.k_cache + ((uint64_t)hk * a.max_seq + a.row0) * HD;
   const E* vbase = (const E*)a.v_cache + ((uint64_t)hk * a.max_seq + a.row0) * HD;
 
-  // K: row kr, chunks qq * CPT .. + CPT - 1; the row scale from the four threads' maxima
-  {
+  // blockIdx.z 0: K row kr, chunks qq * CPT .. + CPT - 1; the row scale from the four threads' maxima
+  if (blockIdx.z == 0) {
     const int kr = tid >> 2, qq = tid & 3;
     const uint32_t key = k0 + (uint32_t)kr;
     float v[CPT][8];
@@ -182,15 +194,25 @@ __global__ void __launch_bounds__(kPrepThreads) k_kv_prep(AttnPrefillArgs a, Pre
       *(h8*)(w.kh + row + 8 * ch) = hi;
       if (sizeof(E) == 4) *(h8*)(w.kl + row + 8 * ch) = lo;
     }
+    return;
   }
 
   // V block: into LDS, block maximum, then transposed rows d (64 keys each)
   float mx = 0.f;
-  for (int c = tid; c < kKB * (HD / 4); c += kPrepThreads) {
-    const int r = c / (HD / 4), col = 4 * (c % (HD / 4));
+  constexpr int kV = kKB * (HD / 4) / kPrepThreads;  // loads per thread, all in flight
+  static_assert(kKB * (HD / 4) % kPrepThreads == 0);
+  float4 xv[kV];
+#pragma unroll
+  for (int u = 0; u < kV; u++) {
+    const int c = tid + kPrepThreads * u, r = c / (HD / 4), col = 4 * (c % (HD / 4));
     const uint32_t key = k0 + (uint32_t)r;
-    float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (key < a.n) x = load4(vbase + (uint64_t)key * HD + col);
+    xv[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (key < a.n) xv[u] = load4(vbase + (uint64_t)key * HD + col);
+  }
+#pragma unroll
+  for (int u = 0; u < kV; u++) {
+    const int c = tid + kPrepThreads * u, r = c / (HD / 4), col = 4 * (c % (HD / 4));
+    const float4 x = xv[u];
     vblk[r][col] = x.x;
     vblk[r][col + 1] = x.y;
     vblk[r][col + 2] = x.z;
@@ -225,11 +247,16 @@ __global__ void __launch_bounds__(kPrepThreads) k_kv_prep(AttnPrefillArgs a, Pre
 // Attention: grid 1-D over (query block, head), heaviest query blocks first.
 // ---------------------------------------------------------------------------
 // LO: K and V have lo planes (an f32 cache).
-template <int HD, bool LO>
+// KS = 2: the workgroup has 64 queries, and its waves 4 to 7 take the second
+// half of each block's keys for the queries of waves 0 to 3; the two sets of
+// running sums meet in LDS at the end.
+template <int HD, bool LO, int KS>
 __global__ void __launch_bounds__(kThreads, 1) k_attn_prefill(AttnPrefillArgs a, PrepWs w) {
   using D = Dims<HD>;
   constexpr int HP = D::HP, NCH = D::NCH, NKS = D::NKS, NT = D::NT;
   constexpr int NP = LO ? 2 : 1;  // planes
+  constexpr int QW = 8 / KS, kQ = 16 * QW;  // waves over queries, queries of the workgroup
+  constexpr int NJ = 4 / KS, NC = 2 / KS;   // a wave's 16-key tiles and 32-key steps of a block
   constexpr int UK = (kKB * NCH * NP + kThreads - 1) / kThreads;  // K chunks per thread (every plane)
   constexpr int UV = (HP * 8 * NP + kThreads - 1) / kThreads;     // V^T chunks per thread
   constexpr bool kWhole = kKB * NCH * NP % kThreads == 0;         // every thread has UK of them (and UV: as many)
@@ -238,6 +265,7 @@ __global__ void __launch_bounds__(kThreads, 1) k_attn_prefill(AttnPrefillArgs a,
   __shared__ __attribute__((aligned(16))) float kfac_s[kKB];  // per key of the block: 2^(e_k - 14) log2(e) / sqrt(hd)
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int qw = wave % QW, kw = wave / QW;  // its queries and its share of each block's keys
   const int fi = lane & 15, fg = lane >> 4;
   const uint32_t nqb = (a.n + kQ - 1) / kQ;
   const uint32_t qb = nqb - 1 - blockIdx.x / a.n_heads, h = blockIdx.x % a.n_heads;
@@ -247,7 +275,7 @@ __global__ void __launch_bounds__(kThreads, 1) k_attn_prefill(AttnPrefillArgs a,
   const float kc = 1.44269504088896341f / sqrtf((float)HD);  // log2(e) / sqrt(hd)
 
   // ---- this lane's query (fi) as the B operand of S^T = K Q^T, in registers ----
-  const uint32_t qt = q0 + 16 * wave + fi;
+  const uint32_t qt = q0 + 16 * qw + fi;
   h8 qh[NKS], ql[NKS];
   float qinv;
   {
@@ -339,21 +367,22 @@ __global__ void __launch_bounds__(kThreads, 1) k_attn_prefill(AttnPrefillArgs a,
     const bool more = kb + 1 < nkb;
     if (more) load_k(kb + 1);
 
-    // ---- S^T: keys 16j + 4fg + r (rows) x this lane's query fi (column) ----
+    // ---- S^T: keys kq + 16j + 4fg + r (rows) x this lane's query fi (column) ----
     // (one head-dim step at a time: four independent accumulator chains, and
     // the fragments of one step live at once)
-    f4 s[4];
+    const int kq = 16 * NJ * kw;  // the wave's first key of the block
+    f4 s[NJ];
 #pragma unroll
-    for (int j = 0; j < 4; j++) s[j] = f4{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < NJ; j++) s[j] = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int ks = 0; ks < NKS; ks++) {
 #pragma unroll
-      for (int j = 0; j < 4; j++) {
-        const h8 kh8 = *(const h8*)&Kh[swz<HP>(16 * j + fi, 4 * ks + fg)];
+      for (int j = 0; j < NJ; j++) {
+        const h8 kh8 = *(const h8*)&Kh[swz<HP>(kq + 16 * j + fi, 4 * ks + fg)];
         s[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh8, qh[ks], s[j], 0, 0, 0);
         s[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh8, ql[ks], s[j], 0, 0, 0);
         if constexpr (LO) {
-          const h8 kl8 = *(const h8*)&Kl[swz<HP>(16 * j + fi, 4 * ks + fg)];
+          const h8 kl8 = *(const h8*)&Kl[swz<HP>(kq + 16 * j + fi, 4 * ks + fg)];
           s[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kl8, qh[ks], s[j], 0, 0, 0);
         }
       }
@@ -367,24 +396,24 @@ __global__ void __launch_bounds__(kThreads, 1) k_attn_prefill(AttnPrefillArgs a,
     // wave's diagonal or the chunk's end (a uniform branch).
     float bm = -INFINITY;
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-      const float4 kf = *(const float4*)&kfac_s[16 * j + 4 * fg];
+    for (int j = 0; j < NJ; j++) {
+      const float4 kf = *(const float4*)&kfac_s[kq + 16 * j + 4 * fg];
       s[j][0] *= kf.x;
       s[j][1] *= kf.y;
       s[j][2] *= kf.z;
       s[j][3] *= kf.w;
     }
-    const bool full = k0 + kKB <= kend && (!a.causal || k0 + kKB - 1 <= q0 + 16 * (uint32_t)wave);
+    const bool full = k0 + kKB <= kend && (!a.causal || k0 + kKB - 1 <= q0 + 16 * (uint32_t)qw);
     if (!full) {
-      // key k0 + 4 fg + 16 j + r is attended iff 16 j + r <= lim
-      const int lim = (int)(a.causal ? min(qt, kend - 1) : kend - 1) - (int)(k0 + 4 * (uint32_t)fg);
+      // key k0 + kq + 4 fg + 16 j + r is attended iff 16 j + r <= lim
+      const int lim = (int)(a.causal ? min(qt, kend - 1) : kend - 1) - (int)(k0 + kq + 4 * (uint32_t)fg);
 #pragma unroll
-      for (int j = 0; j < 4; j++)
+      for (int j = 0; j < NJ; j++)
 #pragma unroll
         for (int r = 0; r < 4; r++) s[j][r] = 16 * j + r <= lim ? s[j][r] : -INFINITY;
     }
 #pragma unroll
-    for (int j = 0; j < 4; j++)
+    for (int j = 0; j < NJ; j++)
 #pragma unroll
       for (int r = 0; r < 4; r++) bm = fmaxf(bm, s[j][r]);
     bm = fmaxf(bm, __shfl_xor(bm, 16, 64));
@@ -397,9 +426,9 @@ __global__ void __launch_bounds__(kThreads, 1) k_attn_prefill(AttnPrefillArgs a,
     const float pscale = ldexpf(1.f, ve - vnew);            // this block's weights, <= 1
     const float c = none ? 0.f : -(qinv * mn);              // exact: qinv is a power of 2
     float ps = 0.f;
-    h4 ph[4], pl[4];
+    h4 ph[NJ], pl[NJ];
 #pragma unroll
-    for (int j = 0; j < 4; j++)
+    for (int j = 0; j < NJ; j++)
 #pragma unroll
       for (int r = 0; r < 4; r++) {
         const float p = __builtin_amdgcn_exp2f(fmaf(qinv, s[j][r], c));
@@ -424,10 +453,10 @@ __global__ void __launch_bounds__(kThreads, 1) k_attn_prefill(AttnPrefillArgs a,
       for (int t = 0; t < NT; t++) o[t] *= oscale;
     }
 #pragma unroll
-    for (int c = 0; c < 2; c++) {
+    for (int c = 0; c < NC; c++) {
       const h8 p8h = __builtin_shufflevector(ph[2 * c], ph[2 * c + 1], 0, 1, 2, 3, 4, 5, 6, 7);
       const h8 p8l = __builtin_shufflevector(pl[2 * c], pl[2 * c + 1], 0, 1, 2, 3, 4, 5, 6, 7);
-      const int va = 32 * c + 4 * fg, vb = va + 16;
+      const int va = kq + 32 * c + 4 * fg, vb = va + 16;
 #pragma unroll
       for (int t = 0; t < NT; t++) {
         const int vr = 16 * t + fi;
@@ -446,6 +475,29 @@ __global__ void __launch_bounds__(kThreads, 1) k_attn_prefill(AttnPrefillArgs a,
       }
     }
   }
+  if constexpr (KS == 2) {
+    // the second half of the keys into the first half's sums, lane by lane
+    // (both waves saw the same blocks: one vref); half of them fill Kh, half Vh
+    __shared__ float half_m[QW][64], half_l[QW][64];
+    constexpr int NH = NT / 2;
+    auto half_o = [&](int t) __attribute__((always_inline)) -> f4& {
+      return ((f4*)(t < NH ? Kh : Vh))[(NH * qw + t % NH) * 64 + lane];
+    };
+    __syncthreads();  // every wave is past its reads of the last block
+    if (kw) {
+#pragma unroll
+      for (int t = 0; t < NT; t++) half_o(t) = o[t];
+      half_m[qw][lane] = m;
+      half_l[qw][lane] = l;
+    }
+    __syncthreads();
+    if (kw) return;
+    const float mo = half_m[qw][lane], mn = fmaxf(m, mo);
+    const float am = __builtin_amdgcn_exp2f(qinv * (m - mn)), ao = __builtin_amdgcn_exp2f(qinv * (mo - mn));
+    l = l * am + half_l[qw][lane] * ao;
+#pragma unroll
+    for (int t = 0; t < NT; t++) o[t] = o[t] * am + half_o(t) * ao;
+  }
   if (qt < a.n) {
     const float inv = ldexpf(1.f, vref - 14) / l;
 #pragma unroll
@@ -463,11 +515,13 @@ hipError_t go(const AttnPrefillArgs& a, hipStream_t st) {
   using D = Dims<HD>;
   const PrepWs w = prep_ws(a.ws, a.n, a.n_kv_heads, D::HP);
   const uint32_t nkb = (a.n + kKB - 1) / kKB;
-  if (a.kv_f16) hipLaunchKernelGGL((k_kv_prep<HD, _Float16>), dim3(nkb, a.n_kv_heads), dim3(kPrepThreads), 0, st, a, w);
-  else hipLaunchKernelGGL((k_kv_prep<HD, float>), dim3(nkb, a.n_kv_heads), dim3(kPrepThreads), 0, st, a, w);
-  const dim3 grid(((a.n + kQ - 1) / kQ) * a.n_heads);
-  if (a.kv_f16) hipLaunchKernelGGL((k_attn_prefill<HD, false>), grid, dim3(kThreads), 0, st, a, w);
-  else hipLaunchKernelGGL((k_attn_prefill<HD, true>), grid, dim3(kThreads), 0, st, a, w);
+  if (a.kv_f16) hipLaunchKernelGGL((k_kv_prep<HD, _Float16>), dim3(nkb, a.n_kv_heads, 2), dim3(kPrepThreads), 0, st, a, w);
+  else hipLaunchKernelGGL((k_kv_prep<HD, float>), dim3(nkb, a.n_kv_heads, 2), dim3(kPrepThreads), 0, st, a, w);
+  auto run = [&](auto kern, uint32_t q) {
+    hipLaunchKernelGGL(kern, dim3((a.n + q - 1) / q * a.n_heads), dim3(kThreads), 0, st, a, w);
+  };
+  if ((a.n + 127) / 128 * a.n_heads >= kFull) a.kv_f16 ? run(k_attn_prefill<HD, false, 1>, 128) : run(k_attn_prefill<HD, true, 1>, 128);
+  else a.kv_f16 ? run(k_attn_prefill<HD, false, 2>, 64) : run(k_attn_prefill<HD, true, 2>, 64);
   return hipGetLastError();
 }
 
