@@ -132,10 +132,12 @@ int ifx_session_len(const ifx_session* s, uint64_t* len);  /* KvCache::len (cach
 int ifx_session_set_rope_mode(ifx_session* s, int mode);
 
 /* Prefill path of a session.  Model::prefill (src/model/forward.rs:496-538)
- * runs chunks of at least min_rows ids (default 64; 0 = never) layer by layer
- * as dequant-to-LDS GEMMs on the fp16 matrix cores and a batched causal
+ * runs chunks of at least min_rows ids (0 = never) layer by layer as GEMMs over
+ * the quantized weights on the fp16 matrix cores and a batched causal
  * attention, when the model is eligible (ifx_model_batched_prefill); shorter
- * chunks replay the decode step per id.  Both give the reference's semantics
+ * chunks replay the decode step per id.  The default is 3 where the launches
+ * for a few tokens take the model (the same type for q and k, and for v or
+ * Q6_K beside Q4_K), and 64 elsewhere.  Both give the reference's semantics
  * (chunk-relative RoPE, chunk-only attention, logits of every row) within
  * f32-level rounding. */
 int ifx_session_set_prefill_batch(ifx_session* s, uint64_t min_rows);

@@ -49,7 +49,23 @@ struct ifx_model {
   uint64_t dev_bytes = 0, gguf_bytes = 0;
   bool dims_ok = false;
   bool gemm_ok = false;  // every layer matrix and the output fit the batched prefill GEMM
+  bool few_ok = false;   // and the few-row launches (gemm_skinny.h) take every layer's q/k/v types
 };
+
+// Chunks of at least this many ids run layer by layer unless the session says
+// otherwise: through the tile GEMMs, or with the few-row launches.  From three
+// ids on the 8B shape's chunk is the faster one (one layer and a step, replayed
+// and layer by layer: 252 and 274 us with two ids, 302 and 271 with three, 909
+// and 292 with 16).
+constexpr uint64_t kBatchMin = 64, kFewMin = 3;
+
+// Chunks through the few-row launches: up to 32 ids, and to 64 where the model
+// is narrow.  Past 32 a workgroup has 256 weight rows and the normed
+// projections, whose K is not cut, few workgroups: the 8B shape's layer (4096
+// columns) takes 440 us with 64 ids against the tile GEMMs' 363, the tiny
+// model's (288) 180 against 239.  The line lies where the two would meet, on
+// the safe side of the ~2000 columns that these give.
+constexpr uint64_t kFewIds = 32, kFewCols = 1024;
 
 struct ifx_session {
   ifx_model* m = nullptr;
@@ -89,9 +105,9 @@ struct ifx_session {
   std::vector<void*> allocs;
   // batched prefill: chunks of at least batch_min rows (0: never) run layer by
   // layer through the GEMMs; the workspace grows to the largest chunk seen
-  uint64_t batch_min = 64;
+  uint64_t batch_min = 0;
   struct {
-    uint64_t cap = 0, logit_rows = 0;
+    uint64_t cap = 0, logit_rows = 0, part_bytes = 0;
     void* alloc = nullptr;
     void* logits = nullptr;
     float *x = nullptr, *q = nullptr, *att = nullptr, *mid = nullptr;
@@ -492,27 +508,40 @@ int state_op(ifx_session* s, uint32_t kind, uint32_t value, uint32_t len) {
   return IFX_OK;
 }
 
+bool few_rows(const ifx_model* m, uint64_t n) {
+  return m->few_ok && n <= (m->cfg.hidden_size <= kFewCols ? kSkinnyRows : kFewIds);
+}
+
 // Prefill workspace for chunks of up to n rows (grows, never shrinks), plus a
-// fixed buffer for the split-K partial tiles of short chunks.
+// buffer for the split-K partial tiles: fixed for the tile GEMMs, what the
+// few-row launches may need for sessions that have seen no longer chunk.
 constexpr uint64_t kSplitPartBytes = 64ull << 20;
-int ensure_ws(ifx_session* s, uint64_t n) {
-  if (n <= s->ws.cap) return IFX_OK;
+int ensure_ws(ifx_session* s, uint64_t n, bool few) {
+  if (n <= s->ws.cap && (few || s->ws.part_bytes == kSplitPartBytes)) return IFX_OK;
+  n = std::max({n, s->ws.cap, few ? (uint64_t)kSkinnyRows : 0});  // one size for every short chunk
+  const uint64_t part_bytes = few && s->ws.part_bytes < kSplitPartBytes ? gemm_skinny_ws_most(kSkinnyRows) : kSplitPartBytes;
   const ifx_config& c = s->m->cfg;
   const uint64_t D = c.hidden_size, F = c.intermediate_size;
   auto al = [](uint64_t b) { return (b + 255) & ~255ull; };
   const uint64_t W = std::max(D, F);  // widest GEMM input
   const uint64_t bx = al(n * D * 4), bm = al(n * F * 4), bh = al(n * W * 2), bg = al(n * (W / 256 + 1) * 32),
-                 br = al(n * 4), bp = kSplitPartBytes;
+                 br = al(n * 4), bp = al(part_bytes);
   const uint64_t ba = al(attn_prefill_ws_bytes((uint32_t)n, (uint32_t)c.n_kv_heads, (uint32_t)c.head_dim));
-  if (s->ws.alloc) {
+  if (s->ws.alloc && s->ws.part_bytes < kSplitPartBytes) {
+    s->allocs.push_back(s->ws.alloc);  // the short chunks': small, and freeing it waits for the device
+    s->ws.alloc = nullptr;
+    s->ws.cap = s->ws.part_bytes = 0;
+  } else if (s->ws.alloc) {
     IFX_HIP(hipStreamSynchronize(s->stream));
     IFX_HIP(hipFree(s->ws.alloc));
     s->ws.alloc = nullptr;
-    s->ws.cap = 0;
+    s->ws.cap = s->ws.part_bytes = 0;
   }
   void* p = nullptr;
-  if (hipMalloc(&p, 3 * bx + bm + 2 * bh + bg + br + bp + ba) != hipSuccess)
+  if (hipMalloc(&p, 3 * bx + bm + 2 * bh + bg + br + bp + ba) != hipSuccess) {
+    (void)hipGetLastError();
     return set_error(IFX_E_OOM, "prefill workspace of %llu rows", (unsigned long long)n);
+  }
   uint8_t* b = (uint8_t*)p;
   s->ws.x = (float*)b;
   s->ws.q = (float*)(b + bx);
@@ -527,6 +556,7 @@ int ensure_ws(ifx_session* s, uint64_t n) {
   s->ws.kv_split = b + bm + 2 * bh + bg + br + bp;
   s->ws.alloc = p;
   s->ws.cap = n;
+  s->ws.part_bytes = part_bytes;
   return IFX_OK;
 }
 
@@ -542,7 +572,8 @@ int ensure_ws(ifx_session* s, uint64_t n) {
 int batched_prefill(ifx_session* s, uint64_t n, uint64_t start, bool causal, float* logits_out) {
   ifx_model* m = s->m;
   const ifx_config& c = m->cfg;
-  IFX_TRY(ensure_ws(s, n));
+  const bool few = few_rows(m, n);
+  IFX_TRY(ensure_ws(s, n, few));
   hipStream_t st = s->stream;
   const uint32_t N = (uint32_t)n, D = (uint32_t)c.hidden_size, F = (uint32_t)c.intermediate_size;
   const uint32_t hd = (uint32_t)c.head_dim, rd = (uint32_t)c.rope_dim;
@@ -550,13 +581,25 @@ int batched_prefill(ifx_session* s, uint64_t n, uint64_t start, bool causal, flo
   const uint32_t pos0 = s->rope_mode == IFX_ROPE_ABSOLUTE ? row0 : 0u;
   auto& w = s->ws;
   // the GEMM operand of rows of k columns (prep writes it, the GEMMs read it)
-  auto op = [&](uint32_t rows, uint32_t k) { return GemmIn{w.ahi, w.alo, w.gsum, w.rexp, rows, k, w.part, kSplitPartBytes}; };
+  auto op = [&](uint32_t rows, uint32_t k) { return GemmIn{w.ahi, w.alo, w.gsum, w.rexp, rows, k, w.part, w.part_bytes}; };
   IFX_HIP(launch_embed_rows(devw(m->embd), s->feed_ids, n, w.x, st));
   for (size_t l = 0; l < m->layers.size(); l++) {
     const LayerDev& L = m->layers[l];
     void* kc = s->kc + l * s->max_seq * kvd * s->kv_es;
     void* vc = s->vc + l * s->max_seq * kvd * s->kv_es;
     const bool kv16 = s->kv_es == 2;
+    if (few) {  // the same layer, each projection one launch from the f32 rows
+      const GemmW qkv[3] = {gw(L.q), gw(L.k), gw(L.v)};
+      const SkinnyQkv d{w.q, kc, vc, s->max_seq * hd, row0, pos0, hd, rd, s->rope_cs, kv16};
+      IFX_HIP(skinny_qkv(w.x, N, L.attn_norm, c.norm_eps, qkv, d, st));
+      const AttnPrefillArgs aa{w.q, kc, vc, w.att, N, row0, (uint32_t)c.n_heads, (uint32_t)c.n_kv_heads, hd,
+                               (uint32_t)s->max_seq, causal, w.kv_split, kv16};
+      IFX_HIP(launch_attn_prefill(aa, st));
+      IFX_HIP(gemm_skinny_residual(w.att, N, gw(L.o), w.x, w.part, st));
+      IFX_HIP(skinny_swiglu(w.x, N, L.ffn_norm, c.norm_eps, gw(L.gate), gw(L.up), w.mid, st));
+      IFX_HIP(gemm_skinny_residual(w.mid, N, gw(L.down), w.x, w.part, st));
+      continue;
+    }
     const GemmIn in = op(N, D);
     IFX_HIP(launch_prep_rows(w.x, N, D, D, L.attn_norm, c.norm_eps, in, st));
     const uint64_t kv_hs = s->max_seq * hd;  // head stride of the head-major cache
@@ -609,6 +652,16 @@ int batched_prefill(ifx_session* s, uint64_t n, uint64_t start, bool causal, flo
     }
   }
   return IFX_OK;
+}
+
+// Whether a chunk of n ids runs layer by layer.  A chunk of fewer than 64 needs
+// no memory but the session's own when it is replayed, as it is where the
+// workspace finds none.
+bool prefill_batched(ifx_session* s, uint64_t n) {
+  if (!s->batch_min || !s->m->gemm_ok || n < s->batch_min) return false;
+  if (n >= kBatchMin || ensure_ws(s, n, few_rows(s->m, n)) == IFX_OK) return true;
+  clear_error();
+  return false;
 }
 
 int check_vocab(const ifx_model* m) {
@@ -709,35 +762,14 @@ int model_open(const char* path, uint32_t flags, ifx_model** out) {
   }
   if (rc != IFX_OK) { model_free(m); return rc; }
   m->gemm_ok = gemm_eligible(m);
+  m->few_ok = m->gemm_ok;
+  for (const LayerDev& L : m->layers)
+    m->few_ok = m->few_ok && skinny_qkv_types(L.q->L.type, L.k->L.type, L.v->L.type);
   *out = m;
   return IFX_OK;
 }
 
-}  // namespace
-
-extern "C" {
-
-void ifx_model_close(ifx_model* m) { model_free(m); }
-
-int ifx_model_config(const ifx_model* m, ifx_config* out) {
-  if (!m || !out) return set_error(IFX_E_INVALID_ARG, "null argument");
-  *out = m->cfg;
-  return IFX_OK;
-}
-
-int ifx_model_weight_bytes(const ifx_model* m, uint64_t* dev, uint64_t* gguf) {
-  if (!m) return set_error(IFX_E_INVALID_ARG, "null model");
-  if (dev) *dev = m->dev_bytes;
-  if (gguf) *gguf = m->gguf_bytes;
-  return IFX_OK;
-}
-
-int ifx_session_create(ifx_model* m, uint64_t max_seq_len, ifx_session** out) {
-  return ifx_session_create_kv(m, max_seq_len, IFX_KV_F32, out);
-}
-
-int ifx_session_create_kv(ifx_model* m, uint64_t max_seq_len, int kv_type, ifx_session** out) {
-  clear_error();
+int session_create(ifx_model* m, uint64_t max_seq_len, int kv_type, ifx_session** out) {
   if (!m || !out || max_seq_len == 0 || max_seq_len > 0x7fffffffull || (kv_type != IFX_KV_F32 && kv_type != IFX_KV_F16))
     return set_error(IFX_E_INVALID_ARG, "bad session arguments");
   *out = nullptr;
@@ -750,6 +782,7 @@ int ifx_session_create_kv(ifx_model* m, uint64_t max_seq_len, int kv_type, ifx_s
   s->m = m;
   s->max_seq = max_seq_len;
   s->kv_es = kv_type == IFX_KV_F16 ? 2 : 4;
+  s->batch_min = m->few_ok ? kFewMin : kBatchMin;
   const uint64_t D = c.hidden_size, F = c.intermediate_size, kvd = c.n_kv_heads * c.head_dim;
   const uint64_t G = c.n_heads / c.n_kv_heads;
   s->max_chunks = (uint32_t)((max_seq_len + s->attn_chunk - 1) / s->attn_chunk);
@@ -801,6 +834,39 @@ int ifx_session_create_kv(ifx_model* m, uint64_t max_seq_len, int kv_type, ifx_s
     return set_error(IFX_E_HIP, "session initialisation failed");
   }
   *out = s;
+  return IFX_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
+void ifx_model_close(ifx_model* m) { model_free(m); }
+
+int ifx_model_config(const ifx_model* m, ifx_config* out) {
+  if (!m || !out) return set_error(IFX_E_INVALID_ARG, "null argument");
+  *out = m->cfg;
+  return IFX_OK;
+}
+
+int ifx_model_weight_bytes(const ifx_model* m, uint64_t* dev, uint64_t* gguf) {
+  if (!m) return set_error(IFX_E_INVALID_ARG, "null model");
+  if (dev) *dev = m->dev_bytes;
+  if (gguf) *gguf = m->gguf_bytes;
+  return IFX_OK;
+}
+
+int ifx_session_create(ifx_model* m, uint64_t max_seq_len, ifx_session** out) {
+  return ifx_session_create_kv(m, max_seq_len, IFX_KV_F32, out);
+}
+
+int ifx_session_create_kv(ifx_model* m, uint64_t max_seq_len, int kv_type, ifx_session** out) {
+  clear_error();
+  IFX_TRY(session_create(m, max_seq_len, kv_type, out));
+  // room for every short chunk: taken by a session's first prompt it would be
+  // that prompt's time (588 -> 749 us over three ids and one layer of the 8B
+  // shape); the ids are replayed where there is none
+  if ((*out)->batch_min == kFewMin && max_seq_len >= kFewMin && ensure_ws(*out, kSkinnyRows, true) != IFX_OK) clear_error();
   return IFX_OK;
 }
 
@@ -885,7 +951,7 @@ int ifx_prefill(ifx_session* s, const uint32_t* ids, uint64_t n, float* logits_o
   IFX_TRY(check_vocab(m));
   if (s->len + n > s->max_seq) return set_error(IFX_E_KV_FULL, "prefill of %llu rows overflows the KV cache", (unsigned long long)n);
   IFX_HIP(hipMemcpyAsync(s->feed_ids, ids, n * 4, hipMemcpyHostToDevice, s->stream));
-  if (s->batch_min && n >= s->batch_min && m->gemm_ok) {
+  if (prefill_batched(s, n)) {
     IFX_HIP(hipEventRecord(s->ev0, s->stream));
     IFX_TRY(batched_prefill(s, n, s->len, true, logits_out));
     IFX_HIP(hipEventRecord(s->ev1, s->stream));
@@ -1263,8 +1329,9 @@ static int forward_rows(ifx_model* m, const uint32_t* ids, uint64_t n, float* lo
   if (n == 0) return IFX_OK;
   IFX_TRY(check_vocab(m));
   ifx_session* s = nullptr;
-  IFX_TRY(ifx_session_create(m, n, &s));
-  if (m->gemm_ok && n >= s->batch_min) {
+  clear_error();
+  IFX_TRY(session_create(m, n, IFX_KV_F32, &s));
+  if (prefill_batched(s, n)) {
     int rc = IFX_OK;
     if (hipMemcpyAsync(s->feed_ids, ids, n * 4, hipMemcpyHostToDevice, s->stream) != hipSuccess)
       rc = set_error(IFX_E_HIP, "forward: id upload failed");

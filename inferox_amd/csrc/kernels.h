@@ -209,7 +209,28 @@ inline bool gemm_skinny_ok(const float* x, uint64_t m, const GemmW& w, const flo
   return m <= kSkinnyRows && (x0 + m * w.cols * 4 <= y0 || y0 + m * w.rows * 4 <= x0);
 }
 uint64_t gemm_skinny_ws_bytes(uint32_t m, const GemmW& w);
+uint64_t gemm_skinny_ws_most(uint32_t m);  // at most, over every matrix and up to m tokens
 hipError_t gemm_skinny(const float* x, uint32_t m, const GemmW& w, float* y, float* ws, hipStream_t st);
+// h[m][rows] += x W^T
+hipError_t gemm_skinny_residual(const float* x, uint32_t m, const GemmW& w, float* h, float* ws, hipStream_t st);
+// q, k, v of rms_norm(x): q [m][rows] with RoPE; k (RoPE) and v rows to cache
+// rows row0 + t of [n_kv][max_seq][head_dim] (kv_stride: max_seq * head_dim);
+// RoPE at positions pos0 + t.  q and k of one type, v of it or (Q4_K) of Q6_K.
+struct SkinnyQkv {
+  float* q;
+  void* k;
+  void* v;
+  uint64_t kv_stride;
+  uint32_t row0, pos0, head_dim, rope_dim;
+  const float2* cs;
+  bool kv_f16;
+};
+bool skinny_qkv_types(uint32_t tq, uint32_t tk, uint32_t tv);
+hipError_t skinny_qkv(const float* x, uint32_t m, const float* norm_w, float eps, const GemmW (&w)[3],
+                      const SkinnyQkv& d, hipStream_t st);
+// mid[m][rows] = swiglu(gate, up) of rms_norm(x)
+hipError_t skinny_swiglu(const float* x, uint32_t m, const float* norm_w, float eps, const GemmW& gate, const GemmW& up,
+                         float* mid, hipStream_t st);
 // rows x cols of x (row stride ld), rms_norm'ed with norm_w when non-null
 // (src/ops.rs:155-180), into the GEMM operand `out` (out.k == cols, rows <= out.m)
 hipError_t launch_prep_rows(const float* x, uint32_t rows, uint32_t ld, uint32_t cols, const float* norm_w,
