@@ -14,7 +14,13 @@
 // a_lo, products accumulated in f32, block scales applied in f32, the Q4_K
 // minimum as one K = 32 MFMA per 256 columns against the activations' group
 // sums.  The activation scale is 2^(14 - e) per row and 256-column block (there:
-// per row), so the split needs no pass over the whole row first.
+// per row), so the split needs no pass over the whole row first.  Products with
+// a lo part go to a sum of their own (kLoSums), small beside the other: 8 steps
+// of a block round at its size instead of 16 (Q4_K) or 24 (Q6_K), and the error
+// against 64 bits is 0.82 (Q4_K) and 0.4 to 0.7 (Q6_K) of kern_gemm.hip's, for
+// ~1% of the time up to 32 tokens (8 tokens x 14336 x 4096: 15.8 -> 15.95 us).
+// In one sum it was up to 1.06 of it over 512 columns whose largest activations
+// come early.
 //
 // Layout: a wave owns NB = 2 tiles of 16 weight rows and every token tile; it
 // loads its rows' blocks straight into registers in the layout they are
@@ -325,9 +331,15 @@ __device__ __forceinline__ void skinny_tiles(const SkinnyArgs& a, const GemmW& w
       }
     }
   };
+  // The products with a lo part summed apart; not in a layer's projections of
+  // more than 32 tokens, whose registers are full (in one sum a short prompt's
+  // logits are within 0.5 to 0.8 of the error that the same ids fed one at a
+  // time have).
+  constexpr bool kLoSums = !W::kPerStep && !(NORM && MT == 4);
   // two sets of weights (this iteration's, the next one's), or one, refilled
-  // once it is used (Q8_0 and Q4_0 with 64 tokens: the registers are full)
-  constexpr int kWSets = W::kPerStep && MT == 4 ? 1 : 2;
+  // once it is used (64 tokens with Q8_0 and Q4_0, or with the second sums: the
+  // registers are full; Q4_K 4096 x 14336 34.9 -> 34.1 us with the one set)
+  constexpr int kWSets = MT == 4 && (W::kPerStep || kLoSums) ? 1 : 2;
   W wb[kWSets][kNB];
   auto load_w = [&](W (&w)[kNB], uint32_t it) __attribute__((always_inline)) {
     const uint32_t b = min(b0 + it * WK + (uint32_t)wk, a.nblk - 1);
@@ -347,11 +359,12 @@ __device__ __forceinline__ void skinny_tiles(const SkinnyArgs& a, const GemmW& w
     // 32-blocks of the wave's block that the row has
     const uint32_t have = min(8u, (a.k >> 5) - min(a.k >> 5, 8 * (b0 + it * WK + (uint32_t)wk)));
     const int r0 = wk * 16 * MT;  // the wave's block of the set
-    f4 cs[kNB][MT];
+    // products of the hi parts, and (kLoSums) those with a lo part
+    f4 cs[kNB][MT], cl[kNB][MT];
 #pragma unroll
     for (int nb = 0; nb < kNB; nb++)
 #pragma unroll
-      for (int mt = 0; mt < MT; mt++) cs[nb][mt] = f4{0.f, 0.f, 0.f, 0.f};
+      for (int mt = 0; mt < MT; mt++) cs[nb][mt] = cl[nb][mt] = f4{0.f, 0.f, 0.f, 0.f};
     float sc[kNB];
     // the fragment address of step 0; step s differs by an exclusive or (kept
     // from being hoisted, as eight addresses per set, into spilled registers)
@@ -368,7 +381,7 @@ __device__ __forceinline__ void skinny_tiles(const SkinnyArgs& a, const GemmW& w
       }
       // every tile's product with a_hi, then with a_lo: independent chains
       h8 bh[kNB], bl[kNB];
-      f4 t[kNB][MT];
+      f4 t[kNB][MT], u[kNB][MT];
 #pragma unroll
       for (int nb = 0; nb < kNB; nb++) {
         if constexpr (W::kPair) {
@@ -388,12 +401,12 @@ __device__ __forceinline__ void skinny_tiles(const SkinnyArgs& a, const GemmW& w
 #pragma unroll
       for (int nb = 0; nb < kNB; nb++)
 #pragma unroll
-        for (int mt = 0; mt < MT; mt++) t[nb][mt] = mfma(al[mt], bh[nb], t[nb][mt]);
+        for (int mt = 0; mt < MT; mt++) u[nb][mt] = mfma(al[mt], bh[nb], kLoSums ? cl[nb][mt] : t[nb][mt]);
       if constexpr (W::kPair) {
 #pragma unroll
         for (int nb = 0; nb < kNB; nb++)
 #pragma unroll
-          for (int mt = 0; mt < MT; mt++) t[nb][mt] = mfma(ah[mt], bl[nb], t[nb][mt]);
+          for (int mt = 0; mt < MT; mt++) u[nb][mt] = mfma(ah[mt], bl[nb], u[nb][mt]);
       }
 #pragma unroll
       for (int nb = 0; nb < kNB; nb++) {
@@ -402,10 +415,11 @@ __device__ __forceinline__ void skinny_tiles(const SkinnyArgs& a, const GemmW& w
         for (int mt = 0; mt < MT; mt++) {
           if constexpr (W::kPerStep) {
 #pragma unroll
-            for (int r = 0; r < 4; r++) cs[nb][mt][r] = fmaf(d, t[nb][mt][r], cs[nb][mt][r]);
+            for (int r = 0; r < 4; r++) cs[nb][mt][r] = fmaf(d, u[nb][mt][r], cs[nb][mt][r]);
             asm volatile("" : "+v"(cs[nb][mt]));  // summed here: not put off with the products held in registers
           } else {
-            cs[nb][mt] = t[nb][mt];
+            cs[nb][mt] = kLoSums ? t[nb][mt] : u[nb][mt];
+            if (kLoSums) cl[nb][mt] = u[nb][mt];
           }
         }
       }
@@ -432,11 +446,21 @@ __device__ __forceinline__ void skinny_tiles(const SkinnyArgs& a, const GemmW& w
         const float d = w[nb].d();
 #pragma unroll
         for (int mt = 0; mt < MT; mt++) {
+          if (kLoSums) {  // d cs is rounded only with the minimum added
+            const f4 mn = mfma(as[mt], bm, cl[nb][mt] * d);
 #pragma unroll
-          for (int r = 0; r < 4; r++) cs[nb][mt][r] *= d;
-          cs[nb][mt] = mfma(as[mt], bm, cs[nb][mt]);
+            for (int r = 0; r < 4; r++) cs[nb][mt][r] = fmaf(d, cs[nb][mt][r], mn[r]);
+          } else {
+            cs[nb][mt] = mfma(as[mt], bm, cs[nb][mt] * d);
+          }
         }
       }
+    }
+    if constexpr (kLoSums && !W::kMins) {
+#pragma unroll
+      for (int nb = 0; nb < kNB; nb++)
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++) cs[nb][mt] += cl[nb][mt];
     }
 #pragma unroll
     for (int mt = 0; mt < MT; mt++) {

@@ -118,6 +118,29 @@ def test_output_over_the_input():
     assert np.all(np.abs(got - a.astype(np.float64) @ wf.T) <= _bound(a.astype(np.float64), wf))
 
 
+@pytest.mark.parametrize("t", [Q4_K, Q6_K])
+@pytest.mark.parametrize("rows,cols", [(1024, 512), (1024, 2048)])
+def test_error_is_no_larger_than_the_tile_gemm(t, rows, cols):
+    """Against float64, on activations with a few large channels. The same call
+    with its output over its input takes the tile GEMM."""
+    few = tile = 0.0
+    for seed in range(3):
+        raw = synth.random_centred_blocks(t, rows * cols, cols, "q", 50 + seed)
+        _, wf = orc.dequantize(t, raw, rows * cols)
+        w, wf = Tensor(t, raw, rows, cols), np.asarray(wf, np.float64).reshape(rows, cols)
+        for m in (3, 8, 16, 24, 40, 64):
+            a = np.random.default_rng(100 * seed + m).standard_normal((m, cols)).astype(np.float32)
+            a[:, ::97] *= 8.0
+            ref = a.astype(np.float64) @ wf.T
+            d = Dev.of(np.concatenate([a.reshape(-1), np.zeros(m * rows, np.float32)]))
+            assert _native.lib().ifx_matmul_qt(d.ptr, m, w.h, d.ptr, None) == 0
+            over = d.get(np.float32, m * rows).reshape(m, rows)
+            n2 = np.sum(ref * ref)
+            few += np.sum((_run(w, a, rows) - ref) ** 2) / n2
+            tile += np.sum((over - ref) ** 2) / n2
+    assert few <= tile, np.sqrt(few / tile)
+
+
 def test_both_entry_points():
     w, wf = _weights(Q4_K, 640, 2048, 77)
     for m in (3, 40):
