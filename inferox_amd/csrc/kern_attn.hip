@@ -170,11 +170,13 @@ __device__ __forceinline__ float4 lanes_sum4(float4 v) {
 
 constexpr int kRowsPerWave = kChunk / (kThreads / 64);  // 16
 
-// Cache rows [lo, hi) the current token attends to.  The three fields are read
-// unconditionally, so that they come in one memory round trip (a conditional
-// read of len would be a second one).
+// Cache rows [lo, hi) the current token attends to: a.rows (ROWS), or what the
+// session's state says.  The three fields are read unconditionally, so that
+// they come in one memory round trip (a conditional read of len would be a
+// second one).
+template <bool ROWS>
 __device__ __forceinline__ void attended_rows(const AttnArgs& a, uint32_t& lo, uint32_t& hi) {
-  if (a.rows) {  // uniform
+  if constexpr (ROWS) {
     lo = 0;
     hi = a.rows;
     return;
@@ -202,7 +204,10 @@ __device__ __forceinline__ void attended_rows(const AttnArgs& a, uint32_t& lo, u
 // At least 3 waves per SIMD: the 70B shape (group 8) otherwise takes 172
 // registers, 2 waves per SIMD, and its ~1040 workgroups at ctx 8192 run in 3
 // rounds instead of 2.
-template <int HDT, int GT, typename E>
+// ROWS, ONE: AttnArgs::rows and one_chunk, as instances of their own: as
+// uniform branches of one kernel they cost the session's attention 4% (8B at
+// 2048 rows 6.88 -> 7.19 us, decode 677.6 -> 672.5 tok/s).
+template <int HDT, int GT, typename E, bool ROWS, bool ONE>
 __global__ void __launch_bounds__(kThreads, GT == 8 ? 3 : 1) k_attn_decode(AttnArgs a) {
   constexpr int EPC = 16 / (int)sizeof(E);     // cache elements per 16-byte K chunk
   constexpr int GM = GT > 0 ? GT : kMaxGroup;  // loop bound over query heads
@@ -219,7 +224,7 @@ __global__ void __launch_bounds__(kThreads, GT == 8 ? 3 : 1) k_attn_decode(AttnA
   const uint32_t G = GT > 0 ? (uint32_t)GT : a.n_heads / a.n_kv_heads;
   const uint32_t HD = HDT > 0 ? (uint32_t)HDT : a.head_dim, nc4 = HD / 4, nck = HD / EPC;
   uint32_t lo, hi;
-  attended_rows(a, lo, hi);
+  attended_rows<ROWS>(a, lo, hi);
   const uint32_t nrows = hi > lo ? hi - lo : 0;
   const uint32_t nch = (nrows + kChunk - 1) / kChunk;
   if (c >= nch) return;
@@ -402,7 +407,7 @@ __global__ void __launch_bounds__(kThreads, GT == 8 ? 3 : 1) k_attn_decode(AttnA
       acc.x += wo[w][g][cp].x;
       acc.y += wo[w][g][cp].y;
     }
-    if (a.one_chunk) {  // the softmax is over this chunk alone: what its merge would write
+    if constexpr (ONE) {  // the softmax is over this chunk alone: what its merge would write
       float L = wst[0][1][g];
 #pragma unroll
       for (int w = 1; w < kThreads / 64; w++) L += wst[w][1][g];
@@ -411,7 +416,7 @@ __global__ void __launch_bounds__(kThreads, GT == 8 ? 3 : 1) k_attn_decode(AttnA
       *(float2*)(part + g * HD + 2 * cp) = acc;
     }
   }
-  if (a.one_chunk) return;
+  if constexpr (ONE) return;
   if (tid < (int)G) {
     float L = wst[0][1][tid];
 #pragma unroll
@@ -432,7 +437,7 @@ __global__ void __launch_bounds__(kThreads, GT == 8 ? 3 : 1) k_attn_decode(AttnA
 // while M is formed.
 // CS workgroups per query head, each producing HD / CS of its columns (every
 // one forms the same weights from all records' max and sum).
-template <int HDT, int GT, int CS>
+template <int HDT, int GT, int CS, bool ROWS>
 __global__ void __launch_bounds__(kThreads) k_attn_merge(AttnArgs a) {
   __shared__ float cw[kThreads];
   __shared__ float wred[2][kThreads / 64];
@@ -441,7 +446,7 @@ __global__ void __launch_bounds__(kThreads) k_attn_merge(AttnArgs a) {
   const uint32_t HD = HDT > 0 ? (uint32_t)HDT : a.head_dim, nc4 = HD / 4 / CS;  // float4 columns of the slice
   const uint32_t h = blockIdx.x / CS, hk = h / G, g = h % G, cb = (blockIdx.x % CS) * nc4;
   uint32_t lo, hi;
-  attended_rows(a, lo, hi);
+  attended_rows<ROWS>(a, lo, hi);
   const uint32_t nrows = hi > lo ? hi - lo : 0;
   const uint32_t nch = (nrows + kChunk - 1) / kChunk;
   if (nch == 0) return;
@@ -547,7 +552,7 @@ int attn_cu_count() {
   return n;
 }
 
-template <typename E>
+template <typename E, bool ROWS, bool ONE>
 void launch_typed(const AttnArgs& a0, hipStream_t st, bool merge) {
   // Chunk grid order: kv head fastest while the grid holds at most two
   // workgroups per CU, so that every chunk of kv head hk runs on XCD hk
@@ -561,7 +566,7 @@ void launch_typed(const AttnArgs& a0, hipStream_t st, bool merge) {
   const char* hf = getenv("IFX_ATTN_HKF");
   const bool forced = hf && (hf[0] == '0' || hf[0] == '1') && hf[1] == 0;
   a.hk_fast = forced ? hf[0] == '1' : (uint64_t)a.max_chunks * a.n_kv_heads <= 2ull * (uint64_t)attn_cu_count();
-  if (a.one_chunk) {
+  if (ONE) {
     // One launch instead of two, and no workgroups for the cache's other
     // chunks: a step of at most 64 rows pays one kernel latency less per layer
     // (tiny model, 24 steps of 6 layers: 4394 -> 3823 us; the operator over 16
@@ -574,10 +579,10 @@ void launch_typed(const AttnArgs& a0, hipStream_t st, bool merge) {
   const uint32_t G = a.n_heads / a.n_kv_heads;
 #define IFX_ATTN(HD_, G_)                                                                          \
   do {                                                                                             \
-    hipLaunchKernelGGL((k_attn_decode<HD_, G_, E>), grid, dim3(kThreads), 0, st, a);              \
+    hipLaunchKernelGGL((k_attn_decode<HD_, G_, E, ROWS, ONE>), grid, dim3(kThreads), 0, st, a);    \
     constexpr int CS_ = (HD_ > 0 && (HD_ / 4) % 4 == 0) ? 4 : 1;                                  \
     if (merge)                                                                                     \
-      hipLaunchKernelGGL((k_attn_merge<HD_, G_, CS_>), dim3(a.n_heads * CS_), dim3(kThreads), 0, st, a); \
+      hipLaunchKernelGGL((k_attn_merge<HD_, G_, CS_, ROWS>), dim3(a.n_heads * CS_), dim3(kThreads), 0, st, a); \
   } while (0)
   if (a.head_dim == 128 && G == 4) IFX_ATTN(128, 4);        // Llama-3 8B
   else if (a.head_dim == 128 && G == 8) IFX_ATTN(128, 8);   // Llama-3 70B
@@ -601,8 +606,13 @@ hipError_t launch_attn(const AttnArgs& a, hipStream_t st, bool merge) {
       !attn_decode_head_dim(a.head_dim, a.kv_f16) || a.chunk != kChunk ||
       a.max_chunks == 0)
     return hipErrorInvalidValue;
-  if (a.kv_f16) launch_typed<_Float16>(a, st, merge);
-  else launch_typed<float>(a, st, merge);
+  auto go = [&](auto e) {
+    using E = decltype(e);
+    if (a.rows) a.one_chunk ? launch_typed<E, true, true>(a, st, merge) : launch_typed<E, true, false>(a, st, merge);
+    else a.one_chunk ? launch_typed<E, false, true>(a, st, merge) : launch_typed<E, false, false>(a, st, merge);
+  };
+  if (a.kv_f16) go((_Float16)0);
+  else go(0.f);
   return hipGetLastError();
 }
 }  // namespace
