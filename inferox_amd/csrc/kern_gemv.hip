@@ -11,8 +11,8 @@
 //   * A row's 16-byte pieces lie one after another; lane l of the L lanes that
 //     share a row takes pieces l, l + L, ... (K of them), so every weight load
 //     of a wave covers contiguous memory.  The lane's x values (K pieces of
-//     them) stay in registers for all the rows the wave runs: no LDS, and no
-//     barrier between the kernel's start and its first dot product.  A launch
+//     them) stay in registers for all the rows the wave runs: no barrier
+//     between the kernel's start and its first dot product.  A launch
 //     on a small matrix is that start (the x loads, a few hundred cycles of
 //     arithmetic, the row reduction), not the stream: with x staged through
 //     LDS, 9 of 64 lanes at work on rows of 288 and 9 workgroups for 288 rows,
@@ -70,7 +70,7 @@ __device__ __forceinline__ uint32_t opaque(uint32_t v) {
 // byte b of v as a signed int8, to f32 (v_bfe_i32 + v_cvt_f32_i32)
 __device__ __forceinline__ float sbyte(int v, int b) { return (float)((v << (24 - 8 * b)) >> 24); }
 
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef float f4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ uint4 ldw(const uint8_t* p) {
   return *(const uint4*)p;
 }
@@ -213,6 +213,13 @@ struct Segs {
   }
 };
 
+// (by value: a conditional over the members selects an address to load from;
+// eight steps of two 288-wide Q8_0 layers 445 -> 362 us, 4096-wide 1310 -> 1137)
+template <class V>
+__device__ __forceinline__ V pick(int s, V a, V b, V c) {
+  return s == 2 ? c : s == 1 ? b : a;
+}
+
 // Unit u of the launch: the rows of its two sums.  Units past the end read
 // unit 0 (in bounds, unused); the row past an odd segment's end reads the last.
 struct Unit {
@@ -233,7 +240,7 @@ __device__ __forceinline__ Unit unit_of(const KArgs& a, const Segs<Epi>& g, uint
     if constexpr (Segs<Epi>::kN == 3) {
       const uint32_t n1 = a.nunits[0], n2 = n1 + a.nunits[1];
       n.s = u >= n2 ? 2 : u >= n1 ? 1 : 0;
-      rows = n.s == 2 ? g.rows[2] : n.s == 1 ? g.rows[1] : rows;
+      rows = pick(n.s, rows, g.rows[1], g.rows[2]);
       u -= n.s == 2 ? n2 : n.s == 1 ? n1 : 0u;
     }
     n.r0 = 2 * u;
@@ -255,8 +262,8 @@ struct Buf {
       b = g.body[t];
       sc = g.scal[t];
     } else if constexpr (Segs<Epi>::kN == 3) {
-      b = n.s == 2 ? g.body[2] : n.s == 1 ? g.body[1] : b;
-      sc = n.s == 2 ? g.scal[2] : n.s == 1 ? g.scal[1] : sc;
+      b = pick(n.s, b, g.body[1], g.body[2]);
+      sc = pick(n.s, sc, g.scal[1], g.scal[2]);
     }
 #pragma unroll
     for (int i = 0; i < K; i++) q[t][i].load(b, sc, t ? n.r1 : n.r0, a.pieces, pc[i]);
@@ -287,6 +294,31 @@ __device__ __forceinline__ float lanes_sum(float v, uint32_t lg) {
 
 constexpr int kMinWaves = 2;  // per SIMD
 
+// Q4_0, several pieces per lane: the 64 pieces of 32 x values that a wave's
+// lanes take come from memory whole lines at a time, through the wave's own
+// part of LDS (no barrier).  Read where they lie, a lane's values are 128 bytes
+// from the next lane's and every load touches 64 cache lines: 4096 x 4096 7.63
+// -> 5.89 us, 14336 x 4096 10.14 -> 8.26, 512 x 8192 8.01 -> 5.99.  The row
+// stride of 36 floats spreads 16 lanes' reads over all banks.
+constexpr int kStageRow = 36, kStageFloats = 64 * kStageRow;
+// floats first .. first + 2047 of v (past `n`: its last four, unused)
+__device__ __forceinline__ void stage_load(f4 (&g)[8], const float* v, uint32_t first, uint32_t n, int lane) {
+#pragma unroll
+  for (int r = 0; r < 8; r++) g[r] = *(const f4*)(v + min(first + 4u * (uint32_t)(lane + 64 * r), n - 4));
+}
+// orders this wave's LDS accesses, which run in the order they are issued
+__device__ __forceinline__ void stage_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+__device__ __forceinline__ void stage_put(const f4 (&g)[8], float* lds, int lane) {
+  stage_order();
+#pragma unroll
+  for (int r = 0; r < 8; r++) *(f4*)(lds + (lane / 8 + 8 * r) * kStageRow + 4 * (lane % 8)) = g[r];
+  stage_order();
+}
+
 // K pieces of a row per lane; WIDE: a.split waves of the workgroup per row.
 template <class Epi, class Q, int K, bool WIDE>
 __global__ void __launch_bounds__(64 * (WIDE ? kWavesWide : kWavesNarrow), kMinWaves) k_gemv(KArgs a, Epi epi) {
@@ -296,6 +328,7 @@ __global__ void __launch_bounds__(64 * (WIDE ? kWavesWide : kWavesNarrow), kMinW
   // registers a row; the other waves of the CU cover them)
   constexpr int kDepth = sizeof(Q) * K > 128 ? 0 : sizeof(Q) * K > 100 ? 1 : 2;
   constexpr int kSlots = kDepth ? kDepth : 1;
+  constexpr bool kStaged = kE == 32 && (K > 1 || WIDE);  // x by way of LDS
   __shared__ float part[2][kW][2];
   __shared__ float red[kW];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -319,35 +352,66 @@ __global__ void __launch_bounds__(64 * (WIDE ? kWavesWide : kWavesNarrow), kMinW
     valid[i] = p < a.pieces;
     pc[i] = min(p, a.pieces - 1);
   }
+  // x w (norm) of the lane's pieces, and its part of x . x; the first units'
+  // rows are in flight meanwhile
   float x[K][kE], sx[K];
-#pragma unroll
-  for (int i = 0; i < K; i++)
-#pragma unroll
-    for (int e = 0; e < kE; e += 4) {
-      const float4 v = *(const float4*)(a.x + (uint64_t)pc[i] * kE + e);
-      x[i][e] = v.x; x[i][e + 1] = v.y; x[i][e + 2] = v.z; x[i][e + 3] = v.w;
-    }
   float nscale = 1.f, ss = 0.f;
-  if (a.norm_w) {
+  Buf<Epi, Q, K> buf[kSlots];
+  // x[i][e ..] = t * w, as ss gathers t * t
+  auto normed = [&](int i, int e, float4 v) __attribute__((always_inline)) {
+    const float w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+      const float t = x[i][e + c];
+      ss = valid[i] ? fmaf(t, t, ss) : ss;
+      x[i][e + c] = t * w[c];
+    }
+  };
+  f4 gx[kStaged ? K : 1][8], gn[kStaged ? K : 1][8];
+  if constexpr (kStaged) {
+#pragma unroll
+    for (int i = 0; i < K; i++) {
+      const uint32_t first = kE * 64u * (j + S * i);
+      stage_load(gx[i], a.x, first, a.cols, lane);
+      if (a.norm_w) stage_load(gn[i], a.norm_w, first, a.cols, lane);
+    }
+  } else {
 #pragma unroll
     for (int i = 0; i < K; i++)
 #pragma unroll
       for (int e = 0; e < kE; e += 4) {
-        const float4 v = *(const float4*)(a.norm_w + (uint64_t)pc[i] * kE + e);
-        const float w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-        for (int c = 0; c < 4; c++) {
-          const float t = x[i][e + c];
-          ss = valid[i] ? fmaf(t, t, ss) : ss;
-          x[i][e + c] = t * w[c];
-        }
+        const float4 v = *(const float4*)(a.x + (uint64_t)pc[i] * kE + e);
+        x[i][e] = v.x; x[i][e + 1] = v.y; x[i][e + 2] = v.z; x[i][e + 3] = v.w;
       }
+    if (a.norm_w) {
+#pragma unroll
+      for (int i = 0; i < K; i++)
+#pragma unroll
+        for (int e = 0; e < kE; e += 4) normed(i, e, *(const float4*)(a.norm_w + (uint64_t)pc[i] * kE + e));
+    }
   }
-  Buf<Epi, Q, K> buf[kSlots];
 #pragma unroll
   for (int d = 0; d < kDepth; d++) {
     buf[d].template load<0>(a, sg, u0 + d * ustep, pc);
     buf[d].template load<1>(a, sg, u0 + d * ustep, pc);
+  }
+  if constexpr (kStaged) {
+    __shared__ __attribute__((aligned(16))) float stage[kW][kStageFloats];
+    float* mine = stage[wave];
+#pragma unroll
+    for (int i = 0; i < K; i++) {
+      stage_put(gx[i], mine, lane);
+#pragma unroll
+      for (int e = 0; e < kE; e += 4) {
+        const float4 v = *(const float4*)(mine + lane * kStageRow + e);
+        x[i][e] = v.x; x[i][e + 1] = v.y; x[i][e + 2] = v.z; x[i][e + 3] = v.w;
+      }
+      if (a.norm_w) {
+        stage_put(gn[i], mine, lane);
+#pragma unroll
+        for (int e = 0; e < kE; e += 4) normed(i, e, *(const float4*)(mine + lane * kStageRow + e));
+      }
+    }
   }
   if (a.norm_w) {  // rms_norm (src/ops.rs:162-167): scale = 1/sqrt(mean(x^2) + eps)
     ss = lanes_sum<K>(ss, lg);

@@ -51,7 +51,7 @@ def test_row_lengths(t, cols):
         assert np.all(err <= _bound(x, wf)), (rows, (err / _bound(x, wf)).max())
 
 
-@pytest.mark.parametrize("t", [Q8_0, F16])
+@pytest.mark.parametrize("t", [Q8_0, Q4_0, F16])
 @pytest.mark.parametrize("cols", [96, 288, 1056, 4096, 4128, 16416])
 def test_norm_and_rope(t, cols):
     """q/k/v of one token (ifx_ops_qkv, the tiled launch), float64 norm and RoPE."""
