@@ -51,6 +51,24 @@ def test_row_lengths(t, cols):
         assert np.all(err <= _bound(x, wf)), (rows, (err / _bound(x, wf)).max())
 
 
+@pytest.mark.parametrize("t", [Q8_0, Q4_0, F16, F32])
+@pytest.mark.parametrize("rows,cols", [(40001, 288), (9001, 2048), (9001, 4096), (5001, 8192), (2501, 16384),
+                                       (1301, 32320)])
+def test_rows_past_the_grid(t, rows, cols):
+    """More rows than the launch's waves take at once (2048 waves of one to four
+    units of two rows, or groups of 2, 4 and 8 waves per unit): each runs three
+    units and more, the last round a part of them and the last unit one row."""
+    w, wf = _weights(t, rows, cols, rows + t)
+    x = np.random.default_rng(rows).standard_normal(cols).astype(np.float32)
+    d_x, d_y = Dev.of(x), Dev.of(np.full(rows + 4, 7.0, np.float32))
+    for _ in range(2):
+        assert _native.lib().ifx_gemv(w.h, d_x.ptr, d_y.ptr, None) == 0
+        y = d_y.get(np.float32, rows + 4)
+        assert np.all(y[rows:] == 7.0)
+        err = np.abs(y[:rows] - wf @ x.astype(np.float64))
+        assert np.all(err <= _bound(x, wf)), (np.nonzero(err > _bound(x, wf))[0][:8], (err / _bound(x, wf)).max())
+
+
 @pytest.mark.parametrize("t", [Q8_0, Q4_0, F16])
 @pytest.mark.parametrize("cols", [96, 288, 1056, 4096, 4128, 16416])
 def test_norm_and_rope(t, cols):
