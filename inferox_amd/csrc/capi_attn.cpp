@@ -103,6 +103,21 @@ int alloc_records(CallScratch& cs, AttnArgs* a) {
                   (uint64_t)a->n_kv_heads * a->max_chunks * attn_partial_floats((uint32_t)G, a->head_dim) * 4);
 }
 
+bool apart(const void* a, uint64_t na, const void* b, uint64_t nb) {
+  return (uintptr_t)a + na <= (uintptr_t)b || (uintptr_t)b + nb <= (uintptr_t)a;
+}
+
+// Rows of one chunk are written by the kernel that reads q and the cache, kv
+// head by kv head: an output that overlaps them other than as q itself (whose
+// heads a workgroup has read before it writes them) takes the records and
+// their merge, which starts when everything has been read.
+bool one_chunk_ok(const AttnArgs& a) {
+  const uint64_t nq = (uint64_t)a.n_heads * a.head_dim * 4;
+  const uint64_t nkv = (uint64_t)a.n_kv_heads * a.max_seq * a.head_dim * (a.kv_f16 ? 2 : 4);
+  return a.rows <= a.chunk && (a.out == a.q || apart(a.out, nq, a.q, nq)) && apart(a.out, nq, a.k_cache, nkv) &&
+         apart(a.out, nq, a.v_cache, nkv);
+}
+
 GemvLaunch single(const ifx_tensor* w, const float* x) {
   GemvLaunch g;
   g.seg[0] = gemv_seg(w->L);
@@ -128,7 +143,7 @@ int ifx_ops_attention_decode(const float* q, const void* k_cache, const void* v_
   CallScratch cs(st);
   a.rows = (uint32_t)n_rows;
   a.out = out;
-  a.one_chunk = n_rows <= a.chunk;
+  a.one_chunk = one_chunk_ok(a);
   if (!a.one_chunk) IFX_TRY(alloc_records(cs, &a));
   IFX_HIP(launch_attn_decode(a, st));
   return cs.finish();
@@ -164,7 +179,7 @@ int ifx_ops_attention_decode_o(const float* q, const void* k_cache, const void* 
     IFX_HIP(launch_mfma_residual_merge(go, a, h, st, merge_bound));
   } else {
     a.rows = (uint32_t)n_rows;
-    a.one_chunk = n_rows <= a.chunk;
+    a.one_chunk = one_chunk_ok(a);
     IFX_HIP(launch_attn_decode(a, st));
     IFX_HIP(gemv_residual(go, h, st));
   }

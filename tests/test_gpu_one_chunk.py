@@ -4,6 +4,8 @@ against float64, and a session's steps across the 64-row line giving the bits
 of the separate-merge steps (fixed summation order, the merge forced)."""
 from __future__ import annotations
 
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -33,6 +35,29 @@ def test_rows_around_one_chunk(heads, kv_heads, hd, f16):
             ref = (e / e.sum()) @ vv
             # scores: hd f32 products and sums (|s| to ~10): 2e-5 of each weight at most
             assert np.abs(got[h] - ref).max() <= 4e-5 * np.abs(vv).max(), (rows, h)
+
+
+@pytest.mark.parametrize("rows", [40, 64, 65])
+@pytest.mark.parametrize("where", ["q", "q+1", "q-1", "k", "v"])
+def test_output_over_the_inputs(rows, where):
+    """The output may overwrite what the attention reads: q itself, q a head
+    further on or back, rows of a cache. Bit for bit what lies apart gives."""
+    heads, kv_heads, hd, seq = 32, 8, 128, 80
+    r = np.random.default_rng(rows)
+    q = r.standard_normal(heads * hd).astype(np.float32)
+    k, v = (r.standard_normal(kv_heads * seq * hd).astype(np.float32) for _ in range(2))
+    buf = np.concatenate([np.zeros(hd, np.float32), q, np.zeros(hd, np.float32)])
+
+    def run(over):
+        d_q, d_k, d_v, d_o = Dev.of(buf), Dev.of(k), Dev.of(v), Dev(4 * heads * hd)
+        at = {"": (d_o, 0), "q": (d_q, hd), "q+1": (d_q, 2 * hd), "q-1": (d_q, 0), "k": (d_k, 3 * seq * hd),
+              "v": (d_v, 2 * seq * hd)}[over]
+        ptr = C.c_void_p(at[0].ptr.value + 4 * at[1])
+        assert _native.lib().ifx_ops_attention_decode(C.c_void_p(d_q.ptr.value + 4 * hd), d_k.ptr, d_v.ptr, 0, seq, rows,
+                                                      heads, kv_heads, hd, ptr, None) == 0
+        return at[0].get(np.float32, at[0].nbytes // 4)[at[1]:at[1] + heads * hd]
+
+    assert np.array_equal(run(where), run(""))
 
 
 def test_steps_across_the_line(tiny_path, monkeypatch):
