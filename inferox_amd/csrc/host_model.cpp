@@ -18,6 +18,7 @@
 
 #include "host_config.h"
 #include "host_gguf.h"
+#include "host_workspace.h"
 #include "ifx_common.h"
 #include "kernels.h"
 
@@ -67,6 +68,17 @@ constexpr uint64_t kBatchMin = 64, kFewMin = 3;
 // the safe side of the ~2000 columns that these give.
 constexpr uint64_t kFewIds = 32, kFewCols = 1024;
 
+// Buffers of a chunk that runs layer by layer.
+struct PrefillWs {
+  float *x = nullptr, *q = nullptr, *att = nullptr, *mid = nullptr;
+  float* part = nullptr;  // split-K partial tiles of the GEMMs
+  uint64_t part_bytes = 0;
+  // the GEMM activation operand (launch_prep_rows), sized for the widest input
+  uint16_t *ahi = nullptr, *alo = nullptr, *gsum = nullptr;
+  int* rexp = nullptr;
+  void* kv_split = nullptr;  // the attention's fp16 K/V pairs (attn_prefill_ws_bytes)
+};
+
 struct ifx_session {
   ifx_model* m = nullptr;
   uint64_t max_seq = 0, len = 0, steps = 0;
@@ -104,19 +116,12 @@ struct ifx_session {
   float last_ms = 0.f;
   std::vector<void*> allocs;
   // batched prefill: chunks of at least batch_min rows (0: never) run layer by
-  // layer through the GEMMs; the workspace grows to the largest chunk seen
+  // layer through the GEMMs; the workspace of the tile GEMMs' chunks grows to
+  // the largest one seen (the short chunks': ChunkWs)
   uint64_t batch_min = 0;
-  struct {
-    uint64_t cap = 0, logit_rows = 0, part_bytes = 0;
-    void* alloc = nullptr;
-    void* logits = nullptr;
-    float *x = nullptr, *q = nullptr, *att = nullptr, *mid = nullptr;
-    float* part = nullptr;  // split-K partial tiles of the GEMMs
-    // the GEMM activation operand (launch_prep_rows), sized for the widest input
-    uint16_t *ahi = nullptr, *alo = nullptr, *gsum = nullptr;
-    int* rexp = nullptr;
-    void* kv_split = nullptr;  // the attention's fp16 K/V pairs (attn_prefill_ws_bytes)
-  } ws;
+  PrefillWs ws;
+  uint64_t ws_cap = 0, logit_rows = 0;
+  void *ws_alloc = nullptr, *ws_logits = nullptr;
 };
 
 namespace ifx {
@@ -508,55 +513,81 @@ int state_op(ifx_session* s, uint32_t kind, uint32_t value, uint32_t len) {
   return IFX_OK;
 }
 
-bool few_rows(const ifx_model* m, uint64_t n) {
-  return m->few_ok && n <= (m->cfg.hidden_size <= kFewCols ? kSkinnyRows : kFewIds);
+uint64_t few_most(const ifx_model* m) { return m->cfg.hidden_size <= kFewCols ? kSkinnyRows : kFewIds; }
+bool few_rows(const ifx_model* m, uint64_t n) { return m->few_ok && n <= few_most(m); }
+
+// Lays the buffers of a chunk of up to n rows out from `base`; returns their
+// bytes.  The few-row launches take the GEMM operand for the output head alone.
+constexpr uint64_t kSplitPartBytes = 64ull << 20;
+uint64_t lay_out_ws(const ifx_model* m, uint64_t n, bool few, uint8_t* base, PrefillWs* w) {
+  const ifx_config& c = m->cfg;
+  const uint64_t D = c.hidden_size, F = c.intermediate_size, W = few ? D : std::max(D, F);
+  uint64_t at = 0;
+  auto take = [&](uint64_t bytes) {
+    uint8_t* p = (uint8_t*)((uintptr_t)base + at);  // (base may be null: sizes only)
+    at += (bytes + 255) & ~255ull;
+    return (void*)p;
+  };
+  w->part_bytes = few ? gemm_skinny_ws_most((uint32_t)n) : kSplitPartBytes;
+  w->x = (float*)take(n * D * 4);
+  w->q = (float*)take(n * D * 4);
+  w->att = (float*)take(n * D * 4);
+  w->mid = (float*)take(n * F * 4);
+  w->ahi = (uint16_t*)take(n * W * 2);
+  w->alo = (uint16_t*)take(n * W * 2);
+  w->gsum = (uint16_t*)take(n * (W / 256 + 1) * 32);
+  w->rexp = (int*)take(n * 4);
+  w->part = (float*)take(w->part_bytes);
+  w->kv_split = take(attn_prefill_ws_bytes((uint32_t)n, (uint32_t)c.n_kv_heads, (uint32_t)c.head_dim));
+  return at;
 }
 
-// Prefill workspace for chunks of up to n rows (grows, never shrinks), plus a
-// buffer for the split-K partial tiles: fixed for the tile GEMMs, what the
-// few-row launches may need for sessions that have seen no longer chunk.
-constexpr uint64_t kSplitPartBytes = 64ull << 20;
-int ensure_ws(ifx_session* s, uint64_t n, bool few) {
-  if (n <= s->ws.cap && (few || s->ws.part_bytes == kSplitPartBytes)) return IFX_OK;
-  n = std::max({n, s->ws.cap, few ? (uint64_t)kSkinnyRows : 0});  // one size for every short chunk
-  const uint64_t part_bytes = few && s->ws.part_bytes < kSplitPartBytes ? gemm_skinny_ws_most(kSkinnyRows) : kSplitPartBytes;
-  const ifx_config& c = s->m->cfg;
-  const uint64_t D = c.hidden_size, F = c.intermediate_size;
-  auto al = [](uint64_t b) { return (b + 255) & ~255ull; };
-  const uint64_t W = std::max(D, F);  // widest GEMM input
-  const uint64_t bx = al(n * D * 4), bm = al(n * F * 4), bh = al(n * W * 2), bg = al(n * (W / 256 + 1) * 32),
-                 br = al(n * 4), bp = al(part_bytes);
-  const uint64_t ba = al(attn_prefill_ws_bytes((uint32_t)n, (uint32_t)c.n_kv_heads, (uint32_t)c.head_dim));
-  if (s->ws.alloc && s->ws.part_bytes < kSplitPartBytes) {
-    s->allocs.push_back(s->ws.alloc);  // the short chunks': small, and freeing it waits for the device
-    s->ws.alloc = nullptr;
-    s->ws.cap = s->ws.part_bytes = 0;
-  } else if (s->ws.alloc) {
+// The session's workspace for the tile GEMMs' chunks of up to n rows.
+int ensure_ws(ifx_session* s, uint64_t n) {
+  if (n <= s->ws_cap) return IFX_OK;
+  if (s->ws_alloc) {
     IFX_HIP(hipStreamSynchronize(s->stream));
-    IFX_HIP(hipFree(s->ws.alloc));
-    s->ws.alloc = nullptr;
-    s->ws.cap = s->ws.part_bytes = 0;
+    IFX_HIP(hipFree(s->ws_alloc));
+    s->ws_alloc = nullptr;
+    s->ws_cap = 0;
   }
   void* p = nullptr;
-  if (hipMalloc(&p, 3 * bx + bm + 2 * bh + bg + br + bp + ba) != hipSuccess) {
+  if (hipMalloc(&p, lay_out_ws(s->m, n, false, nullptr, &s->ws)) != hipSuccess) {
     (void)hipGetLastError();
     return set_error(IFX_E_OOM, "prefill workspace of %llu rows", (unsigned long long)n);
   }
-  uint8_t* b = (uint8_t*)p;
-  s->ws.x = (float*)b;
-  s->ws.q = (float*)(b + bx);
-  s->ws.att = (float*)(b + 2 * bx);
-  b += 3 * bx;
-  s->ws.mid = (float*)b;
-  s->ws.ahi = (uint16_t*)(b + bm);
-  s->ws.alo = (uint16_t*)(b + bm + bh);
-  s->ws.gsum = (uint16_t*)(b + bm + 2 * bh);
-  s->ws.rexp = (int*)(b + bm + 2 * bh + bg);
-  s->ws.part = (float*)(b + bm + 2 * bh + bg + br);
-  s->ws.kv_split = b + bm + 2 * bh + bg + br + bp;
-  s->ws.alloc = p;
-  s->ws.cap = n;
-  s->ws.part_bytes = part_bytes;
+  lay_out_ws(s->m, n, false, (uint8_t*)p, &s->ws);
+  s->ws_alloc = p;
+  s->ws_cap = n;
+  return IFX_OK;
+}
+
+// The buffers of one chunk: the session's own, or, for the few-row launches, a
+// workspace that is the call's alone until its launches have completed
+// (host_workspace.h; one size for every short chunk of a model, so that calls
+// and sessions one after the other share one).
+struct ChunkWs {
+  hipStream_t st;
+  PrefillWs w;
+  WorkspaceLease lease;
+  bool drained = false;  // the call has waited for its launches
+  explicit ChunkWs(hipStream_t s) : st(s) {}
+  ~ChunkWs() {
+    if (lease.ptr() && !drained) (void)hipStreamSynchronize(st);
+  }
+};
+int chunk_ws(ifx_session* s, uint64_t n, ChunkWs* c) {
+  if (!few_rows(s->m, n)) {
+    IFX_TRY(ensure_ws(s, n));
+    c->w = s->ws;
+    return IFX_OK;
+  }
+  const uint64_t most = few_most(s->m);
+  if (c->lease.take(lay_out_ws(s->m, most, true, nullptr, &c->w)) != hipSuccess) {
+    (void)hipGetLastError();
+    return set_error(IFX_E_OOM, "prefill workspace of %llu rows", (unsigned long long)most);
+  }
+  lay_out_ws(s->m, most, true, (uint8_t*)c->lease.ptr(), &c->w);
   return IFX_OK;
 }
 
@@ -569,17 +600,15 @@ int ensure_ws(ifx_session* s, uint64_t n, bool few) {
 // then takes the decode head (final RMSNorm, logits, argmax) and the state
 // records its greedy pick as a step does; logits_out (host, n x vocab) gets
 // every row's logits when non-null.
-int batched_prefill(ifx_session* s, uint64_t n, uint64_t start, bool causal, float* logits_out) {
+int batched_prefill(ifx_session* s, const PrefillWs& w, uint64_t n, uint64_t start, bool causal, float* logits_out) {
   ifx_model* m = s->m;
   const ifx_config& c = m->cfg;
   const bool few = few_rows(m, n);
-  IFX_TRY(ensure_ws(s, n, few));
   hipStream_t st = s->stream;
   const uint32_t N = (uint32_t)n, D = (uint32_t)c.hidden_size, F = (uint32_t)c.intermediate_size;
   const uint32_t hd = (uint32_t)c.head_dim, rd = (uint32_t)c.rope_dim;
   const uint32_t kvd = (uint32_t)(c.n_kv_heads * c.head_dim), row0 = (uint32_t)start;
   const uint32_t pos0 = s->rope_mode == IFX_ROPE_ABSOLUTE ? row0 : 0u;
-  auto& w = s->ws;
   // the GEMM operand of rows of k columns (prep writes it, the GEMMs read it)
   auto op = [&](uint32_t rows, uint32_t k) { return GemmIn{w.ahi, w.alo, w.gsum, w.rexp, rows, k, w.part, w.part_bytes}; };
   IFX_HIP(launch_embed_rows(devw(m->embd), s->feed_ids, n, w.x, st));
@@ -632,36 +661,39 @@ int batched_prefill(ifx_session* s, uint64_t n, uint64_t start, bool causal, flo
   IFX_HIP(launch_finalize(s->state, st));
   if (logits_out) {
     const uint64_t V = c.vocab_size, rows = std::min<uint64_t>(n, 512);
-    if (w.logit_rows < rows) {
-      if (w.logits) {
+    if (s->logit_rows < rows) {
+      if (s->ws_logits) {
         IFX_HIP(hipStreamSynchronize(st));
-        IFX_HIP(hipFree(w.logits));
-        w.logits = nullptr;
-        w.logit_rows = 0;
+        IFX_HIP(hipFree(s->ws_logits));
+        s->ws_logits = nullptr;
+        s->logit_rows = 0;
       }
-      if (hipMalloc(&w.logits, rows * V * 4) != hipSuccess)
+      if (hipMalloc(&s->ws_logits, rows * V * 4) != hipSuccess)
         return set_error(IFX_E_OOM, "prefill logits buffer of %llu rows", (unsigned long long)rows);
-      w.logit_rows = rows;
+      s->logit_rows = rows;
     }
     for (uint64_t r0 = 0; r0 < n; r0 += rows) {
       const uint32_t nr = (uint32_t)std::min<uint64_t>(rows, n - r0);
       const GemmIn in = op(nr, D);
       IFX_HIP(launch_prep_rows(w.x + r0 * D, nr, D, D, m->out_norm, c.norm_eps, in, st));
-      IFX_HIP(gemm_store(in, gw(m->output), (float*)w.logits, (uint32_t)V, st));
-      IFX_HIP(hipMemcpyAsync(logits_out + r0 * V, w.logits, (size_t)nr * V * 4, hipMemcpyDeviceToHost, st));
+      IFX_HIP(gemm_store(in, gw(m->output), (float*)s->ws_logits, (uint32_t)V, st));
+      IFX_HIP(hipMemcpyAsync(logits_out + r0 * V, s->ws_logits, (size_t)nr * V * 4, hipMemcpyDeviceToHost, st));
     }
   }
   return IFX_OK;
 }
 
-// Whether a chunk of n ids runs layer by layer.  A chunk of fewer than 64 needs
-// no memory but the session's own when it is replayed, as it is where the
-// workspace finds none.
-bool prefill_batched(ifx_session* s, uint64_t n) {
-  if (!s->batch_min || !s->m->gemm_ok || n < s->batch_min) return false;
-  if (n >= kBatchMin || ensure_ws(s, n, few_rows(s->m, n)) == IFX_OK) return true;
+// Whether a chunk of n ids runs layer by layer, in the buffers of *c.  A chunk
+// of fewer than 64 needs no memory but the session's own when it is replayed,
+// as it is where the workspace finds none.
+int prefill_batched(ifx_session* s, uint64_t n, ChunkWs* c, bool* batched) {
+  *batched = false;
+  if (!s->batch_min || !s->m->gemm_ok || n < s->batch_min) return IFX_OK;
+  const int rc = chunk_ws(s, n, c);
+  *batched = rc == IFX_OK;
+  if (rc == IFX_OK || n >= kBatchMin) return rc;
   clear_error();
-  return false;
+  return IFX_OK;
 }
 
 int check_vocab(const ifx_model* m) {
@@ -676,8 +708,8 @@ int check_vocab(const ifx_model* m) {
 void session_free(ifx_session* s) {
   if (!s) return;
   if (s->stream) (void)hipStreamSynchronize(s->stream);
-  if (s->ws.alloc) (void)hipFree(s->ws.alloc);
-  if (s->ws.logits) (void)hipFree(s->ws.logits);
+  if (s->ws_alloc) (void)hipFree(s->ws_alloc);
+  if (s->ws_logits) (void)hipFree(s->ws_logits);
   for (auto& row : s->exec)
     for (hipGraphExec_t e : row)
       if (e) (void)hipGraphExecDestroy(e);
@@ -863,10 +895,12 @@ int ifx_session_create(ifx_model* m, uint64_t max_seq_len, ifx_session** out) {
 int ifx_session_create_kv(ifx_model* m, uint64_t max_seq_len, int kv_type, ifx_session** out) {
   clear_error();
   IFX_TRY(session_create(m, max_seq_len, kv_type, out));
-  // room for every short chunk: taken by a session's first prompt it would be
-  // that prompt's time (588 -> 749 us over three ids and one layer of the 8B
-  // shape); the ids are replayed where there is none
-  if ((*out)->batch_min == kFewMin && max_seq_len >= kFewMin && ensure_ws(*out, kSkinnyRows, true) != IFX_OK) clear_error();
+  // the short chunks' workspace, kept for them: allocated by a session's first
+  // prompt it would be that prompt's time (588 -> 749 us over three ids and one
+  // layer of the 8B shape); the ids are replayed where there is no memory for it
+  ChunkWs c((*out)->stream);
+  if (m->few_ok && max_seq_len >= kFewMin && chunk_ws(*out, kFewMin, &c) != IFX_OK) clear_error();
+  c.drained = true;
   return IFX_OK;
 }
 
@@ -951,11 +985,15 @@ int ifx_prefill(ifx_session* s, const uint32_t* ids, uint64_t n, float* logits_o
   IFX_TRY(check_vocab(m));
   if (s->len + n > s->max_seq) return set_error(IFX_E_KV_FULL, "prefill of %llu rows overflows the KV cache", (unsigned long long)n);
   IFX_HIP(hipMemcpyAsync(s->feed_ids, ids, n * 4, hipMemcpyHostToDevice, s->stream));
-  if (prefill_batched(s, n)) {
+  ChunkWs ws(s->stream);
+  bool batched;
+  IFX_TRY(prefill_batched(s, n, &ws, &batched));
+  if (batched) {
     IFX_HIP(hipEventRecord(s->ev0, s->stream));
-    IFX_TRY(batched_prefill(s, n, s->len, true, logits_out));
+    IFX_TRY(batched_prefill(s, ws.w, n, s->len, true, logits_out));
     IFX_HIP(hipEventRecord(s->ev1, s->stream));
     IFX_HIP(hipStreamSynchronize(s->stream));
+    ws.drained = true;
     (void)hipEventElapsedTime(&s->last_ms, s->ev0, s->ev1);
     s->len += n;
     s->steps += n;
@@ -1331,17 +1369,25 @@ static int forward_rows(ifx_model* m, const uint32_t* ids, uint64_t n, float* lo
   ifx_session* s = nullptr;
   clear_error();
   IFX_TRY(session_create(m, n, IFX_KV_F32, &s));
-  if (prefill_batched(s, n)) {
-    int rc = IFX_OK;
-    if (hipMemcpyAsync(s->feed_ids, ids, n * 4, hipMemcpyHostToDevice, s->stream) != hipSuccess)
-      rc = set_error(IFX_E_HIP, "forward: id upload failed");
-    if (rc == IFX_OK) rc = batched_prefill(s, n, 0, false, last_only ? nullptr : logits_out);
-    // the last row's logits, from the head GEMV the batched prefill runs on it
-    if (rc == IFX_OK && last_only &&
-        hipMemcpyAsync(logits_out, s->logits, (size_t)m->cfg.vocab_size * 4, hipMemcpyDeviceToHost, s->stream) !=
-            hipSuccess)
-      rc = set_error(IFX_E_HIP, "forward: logits copy failed");
-    if (rc == IFX_OK && hipStreamSynchronize(s->stream) != hipSuccess) rc = set_error(IFX_E_HIP, "forward: sync failed");
+  bool batched;
+  int rc;
+  {  // (the workspace is given back before the session goes)
+    ChunkWs ws(s->stream);
+    rc = prefill_batched(s, n, &ws, &batched);
+    if (batched) {
+      if (hipMemcpyAsync(s->feed_ids, ids, n * 4, hipMemcpyHostToDevice, s->stream) != hipSuccess)
+        rc = set_error(IFX_E_HIP, "forward: id upload failed");
+      if (rc == IFX_OK) rc = batched_prefill(s, ws.w, n, 0, false, last_only ? nullptr : logits_out);
+      // the last row's logits, from the head GEMV the batched prefill runs on it
+      if (rc == IFX_OK && last_only &&
+          hipMemcpyAsync(logits_out, s->logits, (size_t)m->cfg.vocab_size * 4, hipMemcpyDeviceToHost, s->stream) !=
+              hipSuccess)
+        rc = set_error(IFX_E_HIP, "forward: logits copy failed");
+      if (rc == IFX_OK && hipStreamSynchronize(s->stream) != hipSuccess)
+        rc = set_error(IFX_E_HIP, "forward: sync failed");
+    }
+  }
+  if (batched || rc != IFX_OK) {
     session_free(s);
     return rc;
   }
@@ -1350,7 +1396,7 @@ static int forward_rows(ifx_model* m, const uint32_t* ids, uint64_t n, float* lo
   const size_t V = c.vocab_size;
   float *X = nullptr, *Q = nullptr, *A = nullptr;
   uint32_t* dids = nullptr;
-  int rc = dev_alloc(s->allocs, (void**)&X, n * D * 4);
+  rc = dev_alloc(s->allocs, (void**)&X, n * D * 4);
   if (rc == IFX_OK) rc = dev_alloc(s->allocs, (void**)&Q, n * D * 4);
   if (rc == IFX_OK) rc = dev_alloc(s->allocs, (void**)&A, n * D * 4);
   if (rc == IFX_OK) rc = dev_alloc(s->allocs, (void**)&dids, n * 4);
