@@ -109,7 +109,7 @@ int upload_matrix(uint32_t type, const uint8_t* src, uint64_t nbytes, uint64_t r
                      (unsigned long long)cols);
   ifx_tensor* t = new ifx_tensor();
   const uint64_t body_al = (body + 255) / 256 * 256;
-  if (hipMalloc(&t->alloc, body_al + scal + kTensorPad) != hipSuccess) {
+  if (device_malloc(&t->alloc, body_al + scal + kTensorPad) != hipSuccess) {
     delete t;
     return set_error(IFX_E_OOM, "hipMalloc of %llu bytes failed", (unsigned long long)(body_al + scal));
   }
@@ -224,7 +224,7 @@ int ifx_device_info(char* name, uint64_t cap, int* n_cu, uint64_t* hbm) {
 int ifx_malloc(void** p, uint64_t bytes) {
   IFX_TRY(device_init());
   if (!p) return set_error(IFX_E_INVALID_ARG, "null pointer");
-  if (hipMalloc(p, bytes ? bytes : 4) != hipSuccess) return set_error(IFX_E_OOM, "hipMalloc(%llu)", (unsigned long long)bytes);
+  if (device_malloc(p, bytes ? bytes : 4) != hipSuccess) return set_error(IFX_E_OOM, "hipMalloc(%llu)", (unsigned long long)bytes);
   return IFX_OK;
 }
 
@@ -292,7 +292,7 @@ void ifx_tensor_free(ifx_tensor* t) {
   if (!t) return;
   if (t->alloc) (void)hipFree(t->alloc);
   delete t;
-  if (--g_tensors == 0) workspace_trim(g_stream);
+  if (--g_tensors == 0) workspace_trim();
 }
 
 int ifx_tensor_bytes(const ifx_tensor* t, uint64_t* dev, uint64_t* gguf) {
@@ -335,7 +335,9 @@ static int with_workspace(hipStream_t st, uint64_t bytes, F enqueue) {
     return IFX_OK;
   }
   uint8_t* buf = nullptr;
-  IFX_HIP(hipMallocAsync((void**)&buf, bytes, st));
+  hipError_t ea = hipMallocAsync((void**)&buf, bytes, st);
+  if (ea == hipErrorOutOfMemory && workspace_give_up()) ea = hipMallocAsync((void**)&buf, bytes, st);
+  IFX_HIP(ea);
   const hipError_t e = enqueue(buf);
   const hipError_t ef = hipFreeAsync(buf, st);
   IFX_HIP(e);

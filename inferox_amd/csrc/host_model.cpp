@@ -146,7 +146,7 @@ namespace {
 
 int dev_alloc(std::vector<void*>& owner, void** p, size_t bytes) {
   if (bytes == 0) bytes = 4;
-  hipError_t e = hipMalloc(p, bytes);
+  const hipError_t e = device_malloc(p, bytes);
   if (e != hipSuccess) return set_error(IFX_E_OOM, "hipMalloc(%zu) failed: %s", bytes, hipGetErrorString(e));
   owner.push_back(*p);
   return IFX_OK;
@@ -165,7 +165,7 @@ int upload_norm(ifx_model* m, int64_t idx, uint64_t n, float** out) {
     return set_error(IFX_E_INVALID_ARG, "%s has %llu elements, expected %llu", t.name.c_str(),
                      (unsigned long long)t.n_elements(), (unsigned long long)n);
   void* raw = nullptr;
-  IFX_HIP(hipMalloc(&raw, sz));
+  IFX_HIP(device_malloc(&raw, sz));
   void* f = nullptr;
   IFX_TRY(dev_alloc(m->norm_allocs, &f, n * 4));
   IFX_HIP(hipMemcpy(raw, data, sz, hipMemcpyHostToDevice));
@@ -552,10 +552,8 @@ int ensure_ws(ifx_session* s, uint64_t n) {
     s->ws_cap = 0;
   }
   void* p = nullptr;
-  if (hipMalloc(&p, lay_out_ws(s->m, n, false, nullptr, &s->ws)) != hipSuccess) {
-    (void)hipGetLastError();
+  if (device_malloc(&p, lay_out_ws(s->m, n, false, nullptr, &s->ws)) != hipSuccess)
     return set_error(IFX_E_OOM, "prefill workspace of %llu rows", (unsigned long long)n);
-  }
   lay_out_ws(s->m, n, false, (uint8_t*)p, &s->ws);
   s->ws_alloc = p;
   s->ws_cap = n;
@@ -583,10 +581,8 @@ int chunk_ws(ifx_session* s, uint64_t n, ChunkWs* c) {
     return IFX_OK;
   }
   const uint64_t most = few_most(s->m);
-  if (c->lease.take(lay_out_ws(s->m, most, true, nullptr, &c->w)) != hipSuccess) {
-    (void)hipGetLastError();
+  if (c->lease.take(lay_out_ws(s->m, most, true, nullptr, &c->w)) != hipSuccess)
     return set_error(IFX_E_OOM, "prefill workspace of %llu rows", (unsigned long long)most);
-  }
   lay_out_ws(s->m, most, true, (uint8_t*)c->lease.ptr(), &c->w);
   return IFX_OK;
 }
@@ -668,7 +664,7 @@ int batched_prefill(ifx_session* s, const PrefillWs& w, uint64_t n, uint64_t sta
         s->ws_logits = nullptr;
         s->logit_rows = 0;
       }
-      if (hipMalloc(&s->ws_logits, rows * V * 4) != hipSuccess)
+      if (device_malloc(&s->ws_logits, rows * V * 4) != hipSuccess)
         return set_error(IFX_E_OOM, "prefill logits buffer of %llu rows", (unsigned long long)rows);
       s->logit_rows = rows;
     }
@@ -1110,11 +1106,11 @@ int ifx_sample_logits(const float* logits, uint32_t vocab, float temperature, ui
   void* dw = nullptr;
   DevState* ds = nullptr;
   uint32_t* dt = nullptr;
-  hipError_t e = hipMalloc(&dl, (size_t)vocab * 4);
-  if (e == hipSuccess) e = hipMalloc(&dp, (size_t)vocab * 4);
-  if (e == hipSuccess) e = hipMalloc(&dw, sample_ws_bytes());
-  if (e == hipSuccess) e = hipMalloc(&ds, sizeof(DevState));
-  if (e == hipSuccess) e = hipMalloc(&dt, (size_t)std::max<uint32_t>(n_draws, 1) * 4);
+  hipError_t e = device_malloc((void**)&dl, (size_t)vocab * 4);
+  if (e == hipSuccess) e = device_malloc((void**)&dp, (size_t)vocab * 4);
+  if (e == hipSuccess) e = device_malloc((void**)&dw, sample_ws_bytes());
+  if (e == hipSuccess) e = device_malloc((void**)&ds, sizeof(DevState));
+  if (e == hipSuccess) e = device_malloc((void**)&dt, (size_t)std::max<uint32_t>(n_draws, 1) * 4);
   if (e == hipSuccess) e = hipMemcpy(dl, logits, (size_t)vocab * 4, hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemset(dw, 0, sample_ws_bytes());
   DevState init{};

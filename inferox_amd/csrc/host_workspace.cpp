@@ -28,10 +28,11 @@ IdleList g_idle;  // oldest first
 std::mutex g_stream_mu;
 void* g_stream_ws = nullptr;
 size_t g_stream_bytes = 0;
+hipStream_t g_stream_of = nullptr;  // the stream it was allocated on
 
 size_t round_up(size_t b) { return (b + (1 << 20) - 1) >> 20 << 20; }
 
-void free_idle() {
+bool free_idle() {
   IdleList v;
   {
     std::lock_guard<std::mutex> lk(g_mu);
@@ -39,9 +40,49 @@ void free_idle() {
     g_idle.n = 0;
   }
   for (int i = 0; i < v.n; i++) (void)hipFree(v.v[i].p);
+  return v.n > 0;
+}
+
+// (g_stream_mu held) the stream's workspace back to its pool, in stream order
+bool free_stream() {
+  const bool had = g_stream_ws;
+  if (had) (void)hipFreeAsync(g_stream_ws, g_stream_of);
+  g_stream_ws = nullptr;
+  g_stream_bytes = 0;
+  return had;
+}
+
+// (g_stream_mu held) and from the pool to the device
+void drain_stream() {
+  (void)hipStreamSynchronize(g_stream_of);
+  hipMemPool_t pool;
+  int dev = 0;
+  if (hipGetDevice(&dev) == hipSuccess && hipDeviceGetDefaultMemPool(&pool, dev) == hipSuccess)
+    (void)hipMemPoolTrimTo(pool, 0);
 }
 
 }  // namespace
+
+bool workspace_give_up() {
+  (void)hipGetLastError();  // of the allocation that failed
+  bool any = free_idle();
+  std::lock_guard<std::mutex> lk(g_stream_mu);
+  if (free_stream()) {
+    drain_stream();
+    any = true;
+  }
+  return any;
+}
+
+hipError_t device_malloc(void** p, size_t bytes) {
+  hipError_t e = hipMalloc(p, bytes);
+  if (e == hipErrorOutOfMemory && workspace_give_up()) e = hipMalloc(p, bytes);
+  if (e != hipSuccess) {
+    (void)hipGetLastError();  // the caller has the status; the next launch's is its own
+    *p = nullptr;
+  }
+  return e;
+}
 
 hipError_t WorkspaceLease::take(size_t bytes) {
   give_back();
@@ -64,16 +105,8 @@ hipError_t WorkspaceLease::take(size_t bytes) {
     }
   }
   const size_t n = round_up(bytes);
-  e = hipMalloc(&p_, n);
-  if (e != hipSuccess) {  // what is kept may be what is missing
-    free_idle();
-    (void)hipGetLastError();
-    e = hipMalloc(&p_, n);
-  }
-  if (e != hipSuccess) {
-    p_ = nullptr;
-    return e;
-  }
+  e = device_malloc(&p_, n);
+  if (e != hipSuccess) return e;
   bytes_ = n;
   dev_ = dev;
   return hipSuccess;
@@ -100,23 +133,34 @@ void WorkspaceLease::give_back() {
 StreamWorkspace::StreamWorkspace(hipStream_t st) : lock_(g_stream_mu), st_(st) {}
 
 hipError_t StreamWorkspace::take(size_t bytes) {
-  if (bytes > kStreamWsKept) {
-    own_ = true;
-    return hipMallocAsync(&p_, bytes, st_);
+  const bool keep = bytes <= kStreamWsKept;
+  if (keep && bytes <= g_stream_bytes) {
+    p_ = g_stream_ws;
+    return hipSuccess;
   }
-  if (bytes > g_stream_bytes) {
-    if (g_stream_ws) (void)hipFreeAsync(g_stream_ws, st_);
-    g_stream_ws = nullptr;
-    g_stream_bytes = 0;
-    const size_t n = round_up(bytes);
-    const hipError_t e = hipMallocAsync(&g_stream_ws, n, st_);
-    if (e != hipSuccess) {
-      g_stream_ws = nullptr;
-      return e;
-    }
+  if (keep) free_stream();
+  const size_t n = keep ? round_up(bytes) : bytes;
+  hipError_t e = hipMallocAsync(&p_, n, st_);
+  if (e == hipErrorOutOfMemory) {  // what is kept may be what is missing
+    (void)hipGetLastError();
+    free_idle();
+    free_stream();
+    g_stream_of = st_;
+    drain_stream();
+    e = hipMallocAsync(&p_, n, st_);
+  }
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    p_ = nullptr;
+    return e;
+  }
+  if (keep) {
+    g_stream_ws = p_;
     g_stream_bytes = n;
+    g_stream_of = st_;
+  } else {
+    own_ = true;
   }
-  p_ = g_stream_ws;
   return hipSuccess;
 }
 
@@ -124,12 +168,10 @@ StreamWorkspace::~StreamWorkspace() {
   if (own_ && p_) (void)hipFreeAsync(p_, st_);
 }
 
-void workspace_trim(hipStream_t st) {
+void workspace_trim() {
   free_idle();
   std::lock_guard<std::mutex> lk(g_stream_mu);
-  if (g_stream_ws) (void)hipFreeAsync(g_stream_ws, st);
-  g_stream_ws = nullptr;
-  g_stream_bytes = 0;
+  free_stream();
 }
 
 }  // namespace ifx

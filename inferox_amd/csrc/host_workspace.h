@@ -11,8 +11,9 @@ namespace ifx {
 // returns (the attention operators, a session's short prompts).  With hipMalloc and hipFree (which waits for the whole device) in
 // each call a decode attention over 2048 rows took 43.6 us, 23.3 with buffers
 // kept for the next call (its kernels: 9.5); over 8192 rows 94.2 and 30.3.  At
-// most kLeaseSlots buffers and kLeaseKept bytes are kept over all devices, and
-// none once the last uploaded matrix is freed (workspace_trim).  A buffer
+// most kLeaseSlots buffers and kLeaseKept bytes are kept over all devices; they
+// go when the last uploaded matrix is freed (workspace_trim; what later calls
+// leave is kept again) and when an allocation finds no memory.  A buffer
 // belongs to one call at a time, so calls on several threads and streams never
 // share one.
 constexpr int kLeaseSlots = 8;
@@ -56,6 +57,12 @@ class StreamWorkspace {
 };
 
 // Frees what is kept and not in use (called when the last uploaded matrix goes).
-void workspace_trim(hipStream_t library_stream);
+void workspace_trim();
+// The same for an allocation that found no memory: what was kept is back with
+// the device on return.  Whether there was anything.
+bool workspace_give_up();
+// hipMalloc that gives up what is kept before it fails; leaves no last error.
+// Every device allocation of the library that outlives a call is one.
+hipError_t device_malloc(void** p, size_t bytes);
 
 }  // namespace ifx

@@ -90,6 +90,8 @@ hipError_t hipMalloc(void** p, size_t n) { return take(p, n); }
 hipError_t hipFree(void* p) { return give(p); }
 hipError_t hipMallocAsync(void** p, size_t n, hipStream_t) { return take(p, n); }
 hipError_t hipFreeAsync(void* p, hipStream_t) { return give(p); }
+hipError_t hipDeviceGetDefaultMemPool(hipMemPool_t* p, int) { *p = nullptr; return hipSuccess; }
+hipError_t hipMemPoolTrimTo(hipMemPool_t, size_t) { return hipSuccess; }
 hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind) { memcpy(d, s, n); return hipSuccess; }
 hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) { memcpy(d, s, n); return hipSuccess; }
 hipError_t hipMemcpy2DAsync(void* d, size_t dp, const void* s, size_t sp, size_t w, size_t h, hipMemcpyKind, hipStream_t) {

@@ -90,3 +90,15 @@ def test_a_request_past_what_is_kept():
     one = row.get(np.float32, 256)
     got = y.reshape(16384, 256)[16383]
     assert np.linalg.norm(got - one) <= 4e-6 * np.linalg.norm(one)  # 22-bit operands on both sides
+
+
+def test_after_an_allocation_that_failed():
+    """An allocation no device has room for gives up what is kept and fails; calls
+    after it start afresh and give what they gave."""
+    lin, att = _linear(SHAPES[1], 41), _attn(3000, 42)
+    want = _run_linear(SHAPES[1], *lin), _run_attn(3000, *att)
+    p = C.c_void_p()
+    assert L().ifx_malloc(C.byref(p), 1 << 42) != 0
+    for _ in range(2):
+        assert np.array_equal(_run_linear(SHAPES[1], *lin), want[0])
+        assert np.array_equal(_run_attn(3000, *att), want[1])

@@ -85,3 +85,50 @@ assert s.prefill(ids[:10], False)[0] == OK
 s.close(); g.close()
 assert used() == 0, used()
 """)
+
+
+def test_kept_workspaces_make_room(sim, tmp_path):
+    """What operators keep between calls goes to whoever finds no memory left: a
+    buffer, a matrix, a session, a prompt's workspace, another operator."""
+    _run(sim, tmp_path, """
+raw = synth.random_centred_blocks(Q4_K, 1024 * 512, 512, "q", 1)
+w = Tensor(Q4_K, raw, 1024, 512)
+x, q, cache = Dev(4 * 300 * 1024), Dev(4 * 32 * 128), Dev(4 * 8 * 3100 * 128)
+def keep():
+    plenty()
+    had = used()
+    assert L.ifx_matmul_qt(x.ptr, 300, w.h, x.ptr, None) == OK
+    assert L.ifx_ops_attention_decode(q.ptr, cache.ptr, cache.ptr, 0, 3100, 3000, 32, 8, 128, q.ptr, None) == OK
+    kept = used() - had
+    assert kept >= 2 * MB, kept
+    return kept
+
+kept = keep()
+room(0)
+d = Dev(kept)                      # all of it
+assert L.ifx_gemv(w.h, x.ptr, x.ptr, None) == OK   # the failed attempt left no error behind
+d.free()
+
+keep()
+room(0)
+w2 = Tensor(Q4_K, raw, 1024, 512)
+
+plenty()
+g = model()
+keep()
+room(256 << 10)
+s = g.session(16)                  # a megabyte or so
+
+plenty()
+s2 = g.session(128)
+s2.prefill(ids[:70], False)        # has its own workspace
+keep()
+room(0)
+s2.clear()
+assert s2.prefill(ids[:71], False)[0] == OK
+
+keep()
+room(0)
+assert L.ifx_matmul_qt(x.ptr, 290, w.h, x.ptr, C.c_void_p(8)) == OK  # a caller's stream: a workspace of its own
+assert L.ifx_ops_attention_decode(q.ptr, cache.ptr, cache.ptr, 0, 3100, 3000, 32, 8, 128, q.ptr, None) == OK
+""")
