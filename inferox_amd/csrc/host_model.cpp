@@ -587,6 +587,23 @@ int chunk_ws(ifx_session* s, uint64_t n, ChunkWs* c) {
   return IFX_OK;
 }
 
+// The buffer of the logits of every row of a chunk of n, up to 512 at a time.
+uint64_t logit_chunk(uint64_t n) { return std::min<uint64_t>(n, 512); }
+int ensure_logits(ifx_session* s, uint64_t n) {
+  const uint64_t rows = logit_chunk(n);
+  if (rows <= s->logit_rows) return IFX_OK;
+  if (s->ws_logits) {
+    IFX_HIP(hipStreamSynchronize(s->stream));
+    IFX_HIP(hipFree(s->ws_logits));
+    s->ws_logits = nullptr;
+    s->logit_rows = 0;
+  }
+  if (device_malloc(&s->ws_logits, rows * s->m->cfg.vocab_size * 4) != hipSuccess)
+    return set_error(IFX_E_OOM, "prefill logits buffer of %llu rows", (unsigned long long)rows);
+  s->logit_rows = rows;
+  return IFX_OK;
+}
+
 // Model::prefill (src/model/forward.rs:496-538) as whole-chunk GEMMs, layer by
 // layer (Layer::prefill, src/model/forward.rs:215-337): the n ids at
 // s->feed_ids (device) write K/V rows start .. start + n - 1; query t attends
@@ -656,18 +673,7 @@ int batched_prefill(ifx_session* s, const PrefillWs& w, uint64_t n, uint64_t sta
     IFX_HIP(launch_sample(s->logits, s->probs, sample_ws(s->sample_ws), (uint32_t)c.vocab_size, s->state, st));
   IFX_HIP(launch_finalize(s->state, st));
   if (logits_out) {
-    const uint64_t V = c.vocab_size, rows = std::min<uint64_t>(n, 512);
-    if (s->logit_rows < rows) {
-      if (s->ws_logits) {
-        IFX_HIP(hipStreamSynchronize(st));
-        IFX_HIP(hipFree(s->ws_logits));
-        s->ws_logits = nullptr;
-        s->logit_rows = 0;
-      }
-      if (device_malloc(&s->ws_logits, rows * V * 4) != hipSuccess)
-        return set_error(IFX_E_OOM, "prefill logits buffer of %llu rows", (unsigned long long)rows);
-      s->logit_rows = rows;
-    }
+    const uint64_t V = c.vocab_size, rows = logit_chunk(n);
     for (uint64_t r0 = 0; r0 < n; r0 += rows) {
       const uint32_t nr = (uint32_t)std::min<uint64_t>(rows, n - r0);
       const GemmIn in = op(nr, D);
@@ -679,13 +685,16 @@ int batched_prefill(ifx_session* s, const PrefillWs& w, uint64_t n, uint64_t sta
   return IFX_OK;
 }
 
-// Whether a chunk of n ids runs layer by layer, in the buffers of *c.  A chunk
-// of fewer than 64 needs no memory but the session's own when it is replayed,
-// as it is where the workspace finds none.
-int prefill_batched(ifx_session* s, uint64_t n, ChunkWs* c, bool* batched) {
+// Whether a chunk of n ids runs layer by layer, in the buffers of *c (logits:
+// with every row's).  All of its memory is taken here, before the first launch:
+// a chunk that fails leaves the state as it was.  One of fewer than 64 needs no
+// memory but the session's own when it is replayed, as it is where there is
+// none for this.
+int prefill_batched(ifx_session* s, uint64_t n, bool logits, ChunkWs* c, bool* batched) {
   *batched = false;
   if (!s->batch_min || !s->m->gemm_ok || n < s->batch_min) return IFX_OK;
-  const int rc = chunk_ws(s, n, c);
+  int rc = chunk_ws(s, n, c);
+  if (rc == IFX_OK && logits) rc = ensure_logits(s, n);
   *batched = rc == IFX_OK;
   if (rc == IFX_OK || n >= kBatchMin) return rc;
   clear_error();
@@ -983,7 +992,7 @@ int ifx_prefill(ifx_session* s, const uint32_t* ids, uint64_t n, float* logits_o
   IFX_HIP(hipMemcpyAsync(s->feed_ids, ids, n * 4, hipMemcpyHostToDevice, s->stream));
   ChunkWs ws(s->stream);
   bool batched;
-  IFX_TRY(prefill_batched(s, n, &ws, &batched));
+  IFX_TRY(prefill_batched(s, n, logits_out != nullptr, &ws, &batched));
   if (batched) {
     IFX_HIP(hipEventRecord(s->ev0, s->stream));
     IFX_TRY(batched_prefill(s, ws.w, n, s->len, true, logits_out));
@@ -1369,7 +1378,7 @@ static int forward_rows(ifx_model* m, const uint32_t* ids, uint64_t n, float* lo
   int rc;
   {  // (the workspace is given back before the session goes)
     ChunkWs ws(s->stream);
-    rc = prefill_batched(s, n, &ws, &batched);
+    rc = prefill_batched(s, n, !last_only, &ws, &batched);
     if (batched) {
       if (hipMemcpyAsync(s->feed_ids, ids, n * 4, hipMemcpyHostToDevice, s->stream) != hipSuccess)
         rc = set_error(IFX_E_HIP, "forward: id upload failed");

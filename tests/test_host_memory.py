@@ -132,3 +132,28 @@ room(0)
 assert L.ifx_matmul_qt(x.ptr, 290, w.h, x.ptr, C.c_void_p(8)) == OK  # a caller's stream: a workspace of its own
 assert L.ifx_ops_attention_decode(q.ptr, cache.ptr, cache.ptr, 0, 3100, 3000, 32, 8, 128, q.ptr, None) == OK
 """)
+
+
+def test_logits_without_room(sim, tmp_path):
+    """The logits of every row of a short prompt, where there is no memory for
+    them: the ids are fed one at a time. Of a long one: an error before anything
+    is queued, and the session goes on as it was."""
+    _run(sim, tmp_path, """
+g = model()
+s = g.session(400)
+assert s.prefill(ids[:10], False)[0] == OK
+few, steps = launches("k_skinny_qkv"), launches("k_finalize")
+sim.sim_limit(0)
+assert s.prefill(ids[:10], True)[0] == OK
+assert len(s) == 20 and launches("k_skinny_qkv") == few and launches("k_finalize") == steps + 10
+plenty()
+assert s.prefill(ids[:200], False)[0] == OK
+steps, states = launches("k_finalize"), launches("k_state")
+sim.sim_limit(0)
+assert s.prefill(ids[:100], True)[0] != OK
+assert len(s) == 220 and launches("k_finalize") == steps and launches("k_state") == states
+plenty()
+assert s.prefill(ids[:100], True)[0] == OK
+assert len(s) == 320
+assert g.forward(ids[:10])[0] == OK
+""")
