@@ -50,7 +50,6 @@ struct KArgs {
   GemvSeg seg[3];
   uint32_t nunits[3];  // per logical segment (paired: one logical segment)
   uint32_t total;      // their sum
-  int nseg;            // logical segments
   uint32_t cols, pieces;
   uint32_t lg_lanes;   // log2 of the lanes per row (6 unless K = 1)
   uint32_t split;      // waves per row
@@ -656,9 +655,9 @@ hipError_t launch(const GemvLaunch& L, const Epi& epi, hipStream_t st) {
   if (Epi::kPaired &&
       (L.nseg != 2 || L.seg[0].rows != L.seg[1].rows || L.seg[0].type != L.seg[1].type))
     return hipErrorInvalidValue;
-  // The longest rows taken: what 150 KiB hold of x, its 16-element sums and
-  // the norm weights (32336 columns, 17552 with a norm), so that both kernels
-  // accept the same matrices.
+  // The longest rows taken: 32336 columns, 17552 of whole 32-groups with a norm
+  // (what 150 KiB hold of x, its 16-element sums and the norm weights, as both
+  // kernels once staged them; the generic one's LDS is less).
   const size_t lds = (size_t)((L.cols + 31) / 32) * kGroupStride * 4 + (size_t)((L.cols / 16 + 3) & ~3u) * 4 +
                      (L.norm_w && !generic ? (size_t)L.cols * 4 : 0);
   if (lds > 150 * 1024) return hipErrorInvalidValue;
@@ -669,16 +668,16 @@ hipError_t launch(const GemvLaunch& L, const Epi& epi, hipStream_t st) {
   a.x = L.x;
   a.norm_w = L.norm_w;
   a.eps = L.eps;
-  a.nseg = Epi::kPaired ? 1 : L.nseg;
+  const int nseg = Epi::kPaired ? 1 : L.nseg;
   for (int s = 0; s < L.nseg; s++) a.seg[s] = L.seg[s];
-  for (int s = 0; s < a.nseg; s++) {
+  for (int s = 0; s < nseg; s++) {
     a.nunits[s] = Epi::kPaired ? L.seg[s].rows : (L.seg[s].rows + 1) / 2;
     a.total += a.nunits[s];
   }
   if (a.total == 0) return hipSuccess;
   // one type per launch on this path (the mixed Q4_K / Q6_K layers take the MFMA kernel)
   const uint32_t ta = L.seg[0].type;
-  for (int s = 1; s < a.nseg; s++)
+  for (int s = 1; s < nseg; s++)
     if (L.seg[s].type != ta) return hipErrorInvalidValue;
   switch (ta) {
     case T_Q8_0: return dispatch<Epi, PieceQ80, 2, 4, 4>(a, epi, st);
