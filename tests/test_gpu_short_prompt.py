@@ -8,6 +8,7 @@ import numpy as np
 import pytest
 
 from inferox_amd import synth
+from inferox_amd.gguf_writer import Q4_0, Q4_K, Q6_K
 from oracle import binding as orc
 from tests.conftest import rel_l2
 from tests.gpu_util import GpuModel
@@ -110,3 +111,38 @@ def test_forward(tiny, n):
     orc_rc, ref = o.forward(ids)
     assert rc == 0 and orc_rc == 0
     assert max(rel_l2(a, b) for a, b in zip(lg, ref)) < TOL
+
+
+NARROW = synth.reduced(synth.LLAMA3_8B, dim=512, ffn=1280, n_layers=2, n_heads=8, n_kv_heads=4, vocab=2048, ctx=256)
+ONE_TYPE = {Q4_0: synth.reduced(synth.TINY, n_layers=2, vocab=2048), Q4_K: NARROW, Q6_K: NARROW}
+
+
+@pytest.fixture(scope="module", params=sorted(ONE_TYPE), ids=["q4_0", "q4_k", "q6_k"])
+def one_type(request, tmpdir_session):
+    """A narrow model whose every matrix is of one type: q/k/v and gate/up in the
+    few-row launches that the models above do not reach."""
+    t = request.param
+    spec = synth.reduced(ONE_TYPE[t], types={r: t for r in list(synth.ROLES) + ["embd", "output"]}, centred=t != Q4_0)
+    p = str(tmpdir_session / f"one_type_{t}.gguf")
+    synth.write_llama(p, spec, seed=20 + t)
+    g, o = GpuModel(p), orc.Model(p)
+    yield g, o, spec
+    g.close()
+    o.close()
+
+
+@pytest.mark.parametrize("n", [3, 8, 9, 16, 17, 32, 33, 64])
+def test_one_type(one_type, n):
+    """Against the oracle, and with an f16 cache against the same ids fed one at a
+    time (tolerances: test_chunks_of_every_kind)."""
+    g, o, spec = one_type
+    ids = synth.token_ids(n, spec.vocab, seed=n)
+    s, kv = g.session(128), o.kv(128)
+    rc, ref = o.prefill(kv, ids)
+    assert rc == 0
+    _same_rows(_fed(s, [ids]), (ref, *kv.export(n)))
+    s.close()
+    a, b = g.session(128, kv_f16=True), g.session(128, kv_f16=True)
+    b.set_prefill_batch(0)
+    _same_rows(_fed(a, [ids]), _fed(b, [ids]), 2.0 ** -8, 2.0 ** -10)
+    a.close(), b.close()

@@ -1,7 +1,8 @@
 """Workspaces kept between operator calls: calls of growing and shrinking
-sizes, from several threads at once, on the library's stream and on others,
-give what a lone call gives (bit for bit: the summation order does not depend
-on the workspace), also after everything kept was given back."""
+sizes, from several threads at once, half of them on streams of their own, give
+what a lone call gives (bit for bit: the summation order does not depend on the
+workspace), also with matrices uploaded after the last one was freed. (That
+freeing it gives back what is kept: test_host_memory.py.)"""
 from __future__ import annotations
 
 import ctypes as C
@@ -13,11 +14,12 @@ import pytest
 from inferox_amd import _native, synth
 from inferox_amd.gguf_writer import Q4_K
 from tests.gpu_util import Dev, Tensor
+from tests.test_gpu_other_capture import NON_BLOCKING, _hip as hip
 
 pytestmark = pytest.mark.gpu
 
 L = _native.lib
-SHAPES = [(2, 512, 256), (70, 1024, 512), (300, 512, 1024), (3, 2048, 512), (513, 256, 256)]
+SHAPES = [(2, 512, 256), (70, 1024, 512), (300, 512, 1024), (3, 2048, 512), (513, 256, 256), (3, 512, 4096)]  # the last cuts K
 
 
 def _linear(case, seed):
@@ -41,9 +43,9 @@ def _attn(rows, seed):
     return Dev.of(r.standard_normal(8 * 64).astype(np.float32)), k, v
 
 
-def _run_attn(rows, q, k, v):
+def _run_attn(rows, q, k, v, stream=None):
     out = Dev(4 * 8 * 64)
-    assert L().ifx_ops_attention_decode(q.ptr, k.ptr, v.ptr, 0, rows + 8, rows, 8, 2, 64, out.ptr, None) == 0
+    assert L().ifx_ops_attention_decode(q.ptr, k.ptr, v.ptr, 0, rows + 8, rows, 8, 2, 64, out.ptr, stream) == 0
     return out.get(np.float32, 8 * 64)
 
 
@@ -53,14 +55,19 @@ def test_calls_of_all_sizes_and_threads_agree():
     want_l, want_a = [_run_linear(*x) for x in lin], [_run_attn(*x) for x in att]
     bad = []
 
+    streams = [None] * 6
+    for i in (1, 3, 5):
+        streams[i] = C.c_void_p()
+        assert hip().hipStreamCreateWithFlags(C.byref(streams[i]), NON_BLOCKING) == 0
+
     def work(i):
         try:
             for k in range(6):
                 x = (i + k) % len(lin)
-                if not np.array_equal(_run_linear(*lin[x]), want_l[x]):
+                if not np.array_equal(_run_linear(*lin[x], streams[i]), want_l[x]):
                     bad.append(("linear", SHAPES[x]))
                 y = (i + k) % len(att)
-                if not np.array_equal(_run_attn(*att[y]), want_a[y]):
+                if not np.array_equal(_run_attn(*att[y], streams[i]), want_a[y]):
                     bad.append(("attention", att[y][0]))
         except Exception as e:  # noqa: BLE001 - reported by the assertion below
             bad.append(repr(e))
@@ -70,9 +77,11 @@ def test_calls_of_all_sizes_and_threads_agree():
         t.start()
     for t in th:
         t.join()
+    for st in streams:
+        if st is not None:
+            hip().hipStreamDestroy(st)
     assert not bad, bad
-    # the last matrix freed: what was kept is given back, and later calls start afresh
-    del lin
+    del lin  # the last matrices
     again = _linear(SHAPES[1], 11)
     assert np.array_equal(_run_linear(SHAPES[1], *again), want_l[1])
 
