@@ -674,6 +674,12 @@ int batched_prefill(ifx_session* s, const PrefillWs& w, uint64_t n, uint64_t sta
   IFX_HIP(launch_finalize(s->state, st));
   if (logits_out) {
     const uint64_t V = c.vocab_size, rows = logit_chunk(n);
+    if (few) {  // as the layers: through the tile GEMMs' 128 rows, three ids took longer than their replay
+      IFX_HIP(launch_rms_norm_rows(w.x, m->out_norm, D, n, c.norm_eps, st));
+      IFX_HIP(gemm_skinny(w.x, N, gw(m->output), (float*)s->ws_logits, w.part, st));
+      IFX_HIP(hipMemcpyAsync(logits_out, s->ws_logits, n * V * 4, hipMemcpyDeviceToHost, st));
+      return IFX_OK;
+    }
     for (uint64_t r0 = 0; r0 < n; r0 += rows) {
       const uint32_t nr = (uint32_t)std::min<uint64_t>(rows, n - r0);
       const GemmIn in = op(nr, D);

@@ -157,3 +157,15 @@ assert s.prefill(ids[:100], True)[0] == OK
 assert len(s) == 320
 assert g.forward(ids[:10])[0] == OK
 """)
+
+
+def test_short_prompt_launches(sim, tmp_path):
+    """A short prompt with every row's logits: the few-row launches from the layers
+    to the output head, none of the tile GEMMs' (128 rows, whatever the ids)."""
+    _run(sim, tmp_path, """
+g = model()
+s = g.session(64)
+assert s.prefill(ids[:3], True)[0] == OK
+assert launches("k_skinny_qkv") == 2 and launches("k_gemm_skinny") == 5
+assert launches("k_prep_rows") == 0
+""")
