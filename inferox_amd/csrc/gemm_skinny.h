@@ -6,7 +6,7 @@
 // tile GEMM (kern_gemm.hip) computes 128 token rows whatever m is, reads the
 // operand a separate launch prepared, and cuts K over workgroups whose partial
 // tiles a third launch adds: 8 tokens x 14336 x 4096 Q4_K took 38 us, this
-// kernel takes 15.1 (2.2 TB/s of weights; splitting 16 instead of 8 rows, with
+// kernel takes 15.3 (2.2 TB/s of weights; splitting 16 instead of 8 rows, with
 // its reductions through LDS, it took 20.7).
 //
 // Arithmetic: that of kern_gemm.hip.  Weights are the integers p of w = s p - c
@@ -18,7 +18,7 @@
 // a lo part go to a sum of their own (kLoSums), small beside the other: 8 steps
 // of a block round at its size instead of 16 (Q4_K) or 24 (Q6_K), and the error
 // against 64 bits is 0.82 (Q4_K) and 0.4 to 0.7 (Q6_K) of kern_gemm.hip's, for
-// ~1% of the time up to 32 tokens (8 tokens x 14336 x 4096: 15.8 -> 15.95 us).
+// 0.4 to 0.7% of the time up to 32 tokens (8 tokens x 14336 x 4096: 15.2 -> 15.3).
 // In one sum it was up to 1.06 of it over 512 columns whose largest activations
 // come early.
 //
@@ -423,8 +423,8 @@ __device__ __forceinline__ void skinny_tiles(const SkinnyArgs& a, const GemmW& w
           }
         }
       }
-      // two steps' fragments live at once (all eight hoisted spill)
-      if (MT > 1 || W::kPerStep || (s & 1)) __builtin_amdgcn_sched_barrier(0);
+      // four steps' fragments live at once, or one (all eight hoisted spill)
+      if (MT > 1 || W::kPerStep || (s & 3) == 3) __builtin_amdgcn_sched_barrier(0);
     }
     if constexpr (W::kMins) {
       // lanes of group g: S_hi (g < 2) or S_lo of groups 4 (g & 1) .. + 3
