@@ -338,14 +338,17 @@ int ifx_ops_argmax(const float* x, uint64_t n, uint32_t* out, int* status_out, v
  * The decode step's attention, q/k/v and residual launches as operators, on
  * caller buffers (device pointers).  A device KV cache here is head-major,
  * [n_kv_heads][max_seq][head_dim] of kv_type (IFX_KV_F32 or IFX_KV_F16), the
- * layout a session keeps.  Each call allocates its small device state, runs
- * on `stream` (NULL = the library's) and returns when its work is complete.
+ * layout a session keeps.  Each call takes its small device state from a
+ * bounded list of buffers kept between calls, runs on `stream` (NULL = the
+ * library's) and returns when its work is complete.
  * ------------------------------------------------------------------------- */
 /* The decode attention of Layer::decode_step (src/model/forward.rs:383-414,
  * softmax_rows src/ops.rs:223-239): query head h (kv head h / (n_heads /
  * n_kv_heads)) of q [n_heads*head_dim] attends to cache rows 0 .. n_rows-1:
  * out[h] = sum_t softmax_t(q_h . k_t / sqrt(head_dim)) v_t, through the
- * step's launches (records of 64-row chunks, then their merge).  head_dim a
+ * step's launches (records of 64-row chunks, then their merge; up to 64 rows
+ * one launch that writes out, where out is apart from the caches and is q
+ * itself or apart from it).  out may overlap q and the caches.  head_dim a
  * multiple of 4 (f32 cache) or 8 (f16) up to 256; at most 8 query heads per
  * kv head. */
 int ifx_ops_attention_decode(const float* q, const void* k_cache, const void* v_cache, int kv_type, uint64_t max_seq,

@@ -55,17 +55,19 @@ struct ifx_model {
 
 // Chunks of at least this many ids run layer by layer unless the session says
 // otherwise: through the tile GEMMs, or with the few-row launches.  From three
-// ids on the 8B shape's chunk is the faster one (one layer and a step, replayed
-// and layer by layer: 252 and 274 us with two ids, 302 and 271 with three, 909
-// and 292 with 16).
+// ids on the chunk is the faster one at every width (two layers, us, replayed
+// and layer by layer: 4096 columns 278 and 242 with three ids, 1361 and 283
+// with 16; 8192 columns 650 and 565 with three; with two ids the 4096-column
+// layer took 252 and 274).
 constexpr uint64_t kBatchMin = 64, kFewMin = 3;
 
 // Chunks through the few-row launches: up to 32 ids, and to 64 where the model
 // is narrow.  Past 32 a workgroup has 256 weight rows and the normed
-// projections, whose K is not cut, few workgroups: the 8B shape's layer (4096
-// columns) takes 440 us with 64 ids against the tile GEMMs' 363, the tiny
-// model's (288) 180 against 239.  The line lies where the two would meet, on
-// the safe side of the ~2000 columns that these give.
+// projections, whose K is not cut, few workgroups.  Two layers of 40 to 48 ids,
+// few-row launches and tile GEMMs, us: 512 columns 200 and 279, 1024 264 and
+// 296 (Q8_0 289 and 305), 1536 321 and 333, 2048 382 and 352 (Q8_0 416 and
+// 362), 3072 486 and 389: the line lies at the last power of two on the near
+// side.
 constexpr uint64_t kFewIds = 32, kFewCols = 1024;
 
 // Buffers of a chunk that runs layer by layer.
