@@ -643,13 +643,17 @@ hipError_t dispatch(const GemmArgs& a, const Ep& ep, hipStream_t st) {
 // them.  The plan with the least estimated time is taken, in K steps (~0.95
 // us): rounds of steps and ~8 steps' worth of prologue and epilogue, then for
 // ranges the reduce launch (~4 us, and the partial tiles written and read at
-// ~4.5 TB/s).  Against ranges only for fewer than 256 tiles, and as many of
+// ~4.5 TB/s).  It has to be 5% below that of a range per CU (or whole tiles,
+// where there are 256): plans within 2% of it took up to 6% longer (Q8_0
+// 4096 x 4096 of 100 tokens as 13 ranges 30.2 us, as 16 28.6).  Against ranges only for fewer than 256 tiles, and as many of
 // them as pass 256 workgroups: Q4_K 14336 x 4096 of 129 tokens 93.1 -> 75.0 us
 // (112 tiles ran as 336 workgroups, two rounds), of 512 168.0 -> 147.8 and of
 // 2048 503 -> 485 (a last round of 192 tiles); Q8_0 of 100 tokens 78.4 -> 58.9;
-// Q6_K 4096 x 14336 of 300 tokens 191.5 -> 155.1.  One price for every type:
-// matrices of the four types, 512 x 512 to 14336 x 4096, are no slower under it
-// at any of 12 sizes from 65 to 2048 tokens than cut only below 256 tiles.
+// Q6_K 4096 x 14336 of 300 tokens 191.5 -> 155.1.  One price serves the four
+// types: over six shapes from 512 x 512 to 14336 x 4096 and 24 sizes from 65 to
+// 2048 tokens each, none is slower than a range per CU by more than two runs
+// differ (3 to 5%), and the others are up to 1.5 times as fast.
+constexpr double kClearly = 0.95;
 constexpr uint32_t kMinStepsPerSplit = 8, kMinHalfSteps = 32, kMaxReduceRows = 65535;  // rows of the reduce: its grid's y
 
 GemmArgs args_of(const GemmIn& in, const GemmW& w, bool paired) {
@@ -675,24 +679,35 @@ GemmArgs args_of(const GemmIn& in, const GemmW& w, bool paired) {
   a.half = a.kps >= kMinHalfSteps;
   if (!in.part || !a.ncols || !a.m) return a;
   auto rounds = [](uint64_t wgs) { return (double)((wgs + kTargetWgs - 1) / kTargetWgs); };
-  double best = rounds(tiles) * (nk + 8.0);
+  auto most = [&](uint64_t mbase) -> uint64_t {  // ranges at most
+    const uint64_t per = (a.m - mbase) * a.ncols * 4;
+    return a.m - mbase > kMaxReduceRows ? 0 : std::min<uint64_t>({nk / kMinStepsPerSplit, in.part_bytes / per, 64});
+  };
+  double best = 0.;
+  // tiles past `full` in s ranges (s = 1: whole tiles), if that is estimated below `best` (or there is none yet)
+  auto take = [&](uint64_t full, uint32_t s) {
+    const uint32_t kps = ((nk + s - 1) / s + sb - 1) / sb * sb, ranges = (nk + kps - 1) / kps;
+    const uint64_t rest = tiles - full;
+    const double bytes = 2.0 * ranges * (double)rest * (kBM * kBN * 4);
+    const double c = ranges == 1 ? rounds(tiles) * (nk + 8.0)
+                                 : rounds(full) * (nk + 8.0) + rounds(rest * ranges) * (kps + 8.0) + 4.0 + bytes / 4.5e6;
+    if (best > 0. && c >= best) return;
+    best = c;
+    a.full = (uint32_t)(ranges == 1 ? tiles : full);
+    a.kps = kps;
+    a.ksplit = ranges;
+    a.mbase = (uint32_t)(ranges == 1 ? 0 : full / a.nx * kBM);
+  };
+  // the plan to beat, clearly: a range per CU, or whole tiles if there are that many
+  const uint64_t each = tiles < kTargetWgs ? std::min((kTargetWgs + tiles - 1) / tiles, most(0)) : 1;
+  take(0, (uint32_t)std::max<uint64_t>(1, each));
+  best *= kClearly;
+  take(0, 1);
   // all tiles in ranges, or those past the last whole round
   const uint64_t whole = tiles / kTargetWgs * kTargetWgs;
   for (uint64_t full = 0; full < tiles; full += whole) {
-    const uint64_t mbase = full / a.nx * kBM, per = (a.m - mbase) * a.ncols * 4, rest = tiles - full;
-    const uint64_t most = a.m - mbase > kMaxReduceRows ? 0 : std::min<uint64_t>({nk / kMinStepsPerSplit, in.part_bytes / per, 64});
-    for (uint32_t s = 2; s <= most; s++) {
-      const uint32_t kps = ((nk + s - 1) / s + sb - 1) / sb * sb, ranges = (nk + kps - 1) / kps;
-      const double bytes = 2.0 * ranges * (double)rest * (kBM * kBN * 4);
-      const double c = rounds(full) * (nk + 8.0) + rounds(rest * ranges) * (kps + 8.0) + 4.0 + bytes / 4.5e6;
-      if (ranges > 1 && c < best) {
-        best = c;
-        a.full = (uint32_t)full;
-        a.kps = kps;
-        a.ksplit = ranges;
-        a.mbase = (uint32_t)mbase;
-      }
-    }
+    const uint64_t n = most(full / a.nx * kBM);
+    for (uint32_t s = 2; s <= n; s++) take(full, s);
     if (whole == 0) break;
   }
   a.rounds = a.full < a.tiles ? a.full / kTargetWgs : 0;
