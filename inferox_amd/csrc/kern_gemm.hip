@@ -645,11 +645,12 @@ hipError_t dispatch(const GemmArgs& a, const Ep& ep, hipStream_t st) {
 // ranges the reduce launch (~4 us, and the partial tiles written and read at
 // ~4.5 TB/s).  It has to be 5% below that of a range per CU (or whole tiles,
 // where there are 256): plans within 2% of it took up to 6% longer (Q8_0
-// 4096 x 4096 of 100 tokens as 13 ranges 30.2 us, as 16 28.6).  Against ranges only for fewer than 256 tiles, and as many of
-// them as pass 256 workgroups: Q4_K 14336 x 4096 of 129 tokens 93.1 -> 75.0 us
-// (112 tiles ran as 336 workgroups, two rounds), of 512 168.0 -> 147.8 and of
-// 2048 503 -> 485 (a last round of 192 tiles); Q8_0 of 100 tokens 78.4 -> 58.9;
-// Q6_K 4096 x 14336 of 300 tokens 191.5 -> 155.1.  One price serves the four
+// 4096 x 4096 of 100 tokens as 13 ranges 30.2 us, as 16 28.6).  Against ranges
+// only for fewer than 256 tiles, and as many of them as pass 256 workgroups:
+// Q4_K 14336 x 4096 of 129 tokens 93.1 -> 75.0 us (112 tiles ran as 336
+// workgroups, two rounds), of 512 168.0 -> 147.8 and of 2048 503 -> 485 (a last
+// round of 192 tiles); Q8_0 of 100 tokens 78.4 -> 58.9; Q6_K 4096 x 14336 of 300
+// tokens 191.5 -> 155.1.  One price serves the four
 // types: over six shapes from 512 x 512 to 14336 x 4096 and 24 sizes from 65 to
 // 2048 tokens each, none is slower than a range per CU by more than two runs
 // differ (3 to 5%), and the others are up to 1.5 times as fast.
